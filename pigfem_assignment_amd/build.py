@@ -17,7 +17,7 @@ DRIVER_SRC = os.path.join(CSRC, "driver", "pgf_driver.cpp")
 DRIVER = os.path.join(HERE, "pgf_driver")
 
 HOST_SRC = ["host/pgf_mesh.cpp", "host/pgf_dofs.cpp", "host/pgf_problem.cpp", "host/pgf_sens.cpp",
-            "host/pgf_writer.cpp", "host/pgf_batch_host.cpp"]
+            "host/pgf_writer.cpp", "host/pgf_batch_host.cpp", "host/pgf_team.cpp"]
 HIP_SRC = ["kernels/pgf_assemble.hip", "kernels/pgf_device.hip", "kernels/pgf_cnn.hip", "kernels/pgf_batch.hip",
            "kernels/pgf_sens.hip", "kernels/pgf_preprocess.hip"]
 # the device set-up shares its arithmetic with the host set-up (g++, no FMA on

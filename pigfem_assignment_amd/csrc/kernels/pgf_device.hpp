@@ -7,6 +7,7 @@
 #include <vector>
 
 #include "pgf_kernels.hpp"
+#include "pgf_team.hpp"
 
 struct pgf_ctx;  // the C-ABI handle (derives from pgfd::Ctx)
 
@@ -73,7 +74,6 @@ struct Ctx {
     int64_t* free_slot = nullptr;
     // matrix
     int32_t *rowptr = nullptr, *rowsplit = nullptr, *colidx = nullptr;
-    int32_t* grp_row = nullptr;  // [n_grp+1] first free row of each SpMV node group
     int64_t n_grp = 0;
     double* K = nullptr;
     float* K32 = nullptr;
@@ -81,12 +81,22 @@ struct Ctx {
     double* Fext_full = nullptr;   // [n_free]
     double* upres_full = nullptr;  // [n_pres]
     // solver work (FP64 and FP32)
-    double *r = nullptr, *x = nullptr, *z = nullptr, *p0 = nullptr, *p1 = nullptr, *q = nullptr, *dinv = nullptr,
-           *guess = nullptr, *res = nullptr;
+    double *r = nullptr, *x = nullptr, *q = nullptr, *dinv = nullptr, *guess = nullptr, *res = nullptr;
+    double2* zp = nullptr;         // [n_free] (z, p) pairs of the PCG
+    // PCG team of this system (pgf_team.hpp)
+    std::vector<pgft::GroupRec> h_grp;  // [n_grp + 1] host copy (shares of a batch)
+    pgft::GroupRec* grp = nullptr;
+    pgft::TeamPlan team;
+    int32_t *diag = nullptr, *team_row_ptr = nullptr, *team_list = nullptr, *team_halo = nullptr;
+    int64_t *team_halo_ptr = nullptr, *team_step_ptr = nullptr;
+    pgft::StepRec* team_steps = nullptr;
+    uint16_t* team_wcol = nullptr;
+    int* team_pos = nullptr;
+    unsigned long long* team_slots = nullptr;
+    int n_cu = 0;
     double* partial = nullptr;     // block partial sums
-    double* scal = nullptr;        // device scalars of the PCG recurrence
+    double* scal = nullptr;        // device scalars: PCG state (pgft::T_N), residual norm
     unsigned* counter = nullptr;   // last-block counters
-    int* done = nullptr;
     double* h_scal = nullptr;      // pinned mirror
     bool have_guess = false;
     hipEvent_t* timing_events = nullptr;  // when set: cut pass start, gather start, gather end

@@ -1,0 +1,672 @@
+// Jacobi-PCG in one cooperative launch: teams of blocks that stay resident
+// and iterate together.
+//
+// What bounds it: a PCG iteration is two sums over the whole system (p.q, then
+// r.z and r.r) around one pass over K.  As separate kernels that is five
+// launches of 2.4-6 us each, which is the whole iteration for systems whose K
+// fits the caches.  Here a team of blocks (all of the launch for one system)
+// iterates by itself:
+//
+//  * a sum over the team costs one exchange through memory: every block
+//    publishes its partial sums in its own slot, one wavefront of every block
+//    reads all slots until none is empty and adds them in slot order, so every
+//    block has the same total and takes the same decisions.  No
+//    read-modify-write: a single arrival counter costs ~60 ns per block on one
+//    line (15 us at 256 blocks); this exchange takes 2.0 to 2.6 us.
+//  * "empty" is a NaN pattern no sum is published as.  Slots rotate over three
+//    buffers: a block empties its slot of the buffer after next right after it
+//    has read a sum, when every block has left the sum that last used it.
+//  * the search direction is formed where it is used: each row publishes
+//    (z, p_old) as one 16-byte pair, and whoever needs that column computes
+//    p = z + beta p_old, so p needs no exchange of its own and an iteration
+//    has two.
+//  * a block keeps p of every column its rows touch in LDS (its window: its
+//    own rows, then the other blocks' columns, its halo) and finds it by a
+//    16-bit window index, so a product's gathers are LDS reads and the halo is
+//    read from memory once per iteration.
+//  * the pairs are the only data blocks read from each other.  They are
+//    written through to memory and read past the caches of the reading die
+//    (device-scope cache policy on the accesses themselves): a release and an
+//    acquire fence of the agent instead, which write back and drop the die's
+//    whole L2, take 4.5 us with 32 blocks per die, and K leaves the L2.
+//  * K entries and window indices of a block stay in registers where they all
+//    fit (KEEP steps a lane); otherwise they are streamed, the loads two steps
+//    ahead of the products.
+//  * the steps of a block's lane groups are laid out on the host: rows longer
+//    than a step take consecutive steps of one lane group, so no lane waits in
+//    a loop over a neighbour's long row, and every block has about as many.
+//
+// Every wait ends: a wait that has seen no change for WAIT_TICKS raises the
+// abort flag, all blocks leave and the host reports a device error.  The
+// launch is cooperative, so all blocks are resident.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cstdint>
+#include <vector>
+
+#include "../host/pgf_team.hpp"
+
+namespace pgft {
+
+constexpr int TT = TEAM_THREADS;                  // 512: 256 registers a lane for K entries
+constexpr int MAX_TEAM = 256;                     // blocks per team (four slots per lane of the reading wavefront)
+constexpr unsigned long long EMPTY = ~0ull;       // slot not yet published
+constexpr unsigned long long WAIT_TICKS = 2000000000ull;  // 20 s of the 100 MHz wall clock
+constexpr size_t LDS_MAX = 156 * 1024;            // dynamic LDS a block may take (of 160 KiB)
+constexpr int MAX_WINDOW = 65536;                 // 16-bit window indices
+
+// per (system, right-hand side) state between launches and result
+enum { T_RZ = 0, T_BETA, T_RR, T_RR0, T_TOL, T_IT, T_DONE, T_N = 8 };
+
+// Where a block's vectors live.  WIN_ALL: window p, and r, q, 1/diag of its
+// rows in LDS.  WIN_PQ: window p and q in LDS, r and 1/diag in memory.
+enum Tier { WIN_ALL = 0, WIN_PQ = 1 };
+
+template <typename TA>
+struct TeamArgs {
+    int n_teams, team_blocks;
+    const int32_t* team_sys;  // [n_teams + 1] range of each team in sys_list
+    const int32_t* sys_list;  // systems in the order their team solves them
+    int* team_pos;            // [n_teams][2] next entry of the list, 1 if that system is under way
+    const int32_t* row_ptr;   // [n_sys][team_blocks + 1] first row of each block
+    const int64_t* step_ptr;  // [n_sys * team_blocks + 1]
+    const StepRec* steps;
+    const uint16_t* wcol;     // window index of each entry (first row of every group)
+    const int64_t* halo_ptr;  // [n_sys * team_blocks + 1]
+    const int32_t* halo;      // columns of each block's halo
+    const int32_t* diag;      // entry of each row's diagonal, -1 without one
+    const TA* A;
+    const double* b;          // [n][NR]
+    const double* Ax;         // K x0 for a nonzero start (x then holds x0), or null
+    double *x, *r, *dinv;     // [n][NR] ([n] for dinv)
+    double2* zp;              // [n][NR] published (z, p)
+    int64_t zp_bytes;
+    double* state;            // [n_sys][NR][T_N]
+    unsigned long long* slots;  // [n_teams][COPIES][team_slots]
+    int* abort;
+    double tol2;              // squared relative tolerance
+    int maxit, launch_its;    // iterations per system, and per team in this launch
+    int single;               // stopping rules of the single solve (see below)
+};
+
+template <int NR>
+constexpr int slot_values() { return NR == 1 ? 3 : 2 * NR; }
+
+// Every slot is published in COPIES places, one for the readers of each die,
+// and has 64 bytes of its own: 256 wavefronts polling the same few lines wait
+// on each other, and so do blocks that write one line.  One sum with 160 to
+// 256 blocks: 2.8-3.3 us in one copy of packed slots (1.8 where the lines
+// happened to lie well), 2.0-2.6 so; 2 to 32 copies and 128-byte slots are
+// within 5 % of this.
+constexpr int COPIES = 8, SLOT = 8;
+static_assert(slot_values<4>() <= SLOT, "a slot holds every sum");
+__host__ __device__ constexpr int64_t team_slots(int nb) {  // one copy: three buffers, on pages of its own
+    return ((int64_t)3 * nb * SLOT + 511) / 512 * 512;
+}
+
+// ---- device-scope accesses of the pairs: SC1 on a buffer access (bit 4)
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+constexpr int SC1 = 16;
+__device__ inline double2 pair_load(__amdgpu_buffer_rsrc_t rs, uint32_t i) {
+    union { u32x4 u; double2 d; } v;
+    v.u = __builtin_amdgcn_raw_buffer_load_b128(rs, (int)(i * 16u), 0, SC1);
+    return v.d;
+}
+__device__ inline void pair_store(__amdgpu_buffer_rsrc_t rs, uint32_t i, double2 d) {
+    union { u32x4 u; double2 d; } v;
+    v.d = d;
+    __builtin_amdgcn_raw_buffer_store_b128(v.u, rs, (int)(i * 16u), 0, SC1);
+}
+
+__device__ inline unsigned long long slot_load(const unsigned long long* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline void slot_store(unsigned long long* p, unsigned long long v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// ---- sums over consecutive lanes by data-parallel primitives (every lane
+// gets the sum): lanes ^1, ^2, 7 - i, 15 - i of a row of 16
+template <int CTRL>
+__device__ inline double dpp(double v) {
+    const long long u = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)u, CTRL, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(u >> 32), CTRL, 0xf, 0xf, false);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+template <int G>
+__device__ inline double lane_sum(double v) {
+    v += dpp<0xB1>(v);
+    v += dpp<0x4E>(v);
+    v += dpp<0x141>(v);
+    if (G == 16) v += dpp<0x140>(v);
+    return v;
+}
+__device__ inline double wave_sum(double v) {
+    v = lane_sum<16>(v);
+    v += __shfl_xor(v, 16, 64);
+    v += __shfl_xor(v, 32, 64);
+    return v;
+}
+
+// a value all lanes agree on, in scalar registers
+__device__ inline double uniform(double v) {
+    const long long u = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_readfirstlane((int)u), hi = __builtin_amdgcn_readfirstlane((int)(u >> 32));
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
+// One block's end of the team's sums.
+template <int NR>
+struct TeamSum {
+    static constexpr int W = slot_values<NR>(), TW = TT / 64;
+    static_assert(TW <= 16, "one row of lanes adds the wavefronts");
+    unsigned long long* slots;  // this team's [COPIES][3][nb][SLOT]
+    int nb, me, copy;
+    unsigned phase;
+    double (*red)[W];           // [16][W] LDS, rows from TW on zero
+    double* tot;                // [W] LDS
+    int* bad;                   // LDS: the team gave up
+    int* abort;
+
+    // Sums v[0..NV) over the team; returns false if a wait ran out.  publish:
+    // other blocks read pairs this block stored before.  Wavefronts other than
+    // the first run `meanwhile`.
+    template <int NV, typename F>
+    __device__ bool operator()(double (&v)[NV], bool publish, F&& meanwhile) {
+        const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+        for (int k = 0; k < NV; ++k) v[k] = wave_sum(v[k]);
+        if (lane == 0)
+#pragma unroll
+            for (int k = 0; k < NV; ++k) red[w][k] = v[k];
+        // every wavefront's pairs have left it before the publication
+        if (publish) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (w == 0) {
+            double s[NV];
+#pragma unroll
+            for (int k = 0; k < NV; ++k) s[k] = lane_sum<16>(red[lane & 15][k]);
+            if (nb > 1) exchange<NV>(s, lane);
+            if (lane == 0)
+#pragma unroll
+                for (int k = 0; k < NV; ++k) tot[k] = s[k];
+        } else {
+            meanwhile();
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < NV; ++k) v[k] = uniform(tot[k]);
+        return __builtin_amdgcn_readfirstlane(*bad) == 0;
+    }
+
+    template <int NV>
+    __device__ void exchange(double (&s)[NV], int lane) {
+        const int64_t per = team_slots(nb), at = (int64_t)(phase % 3) * nb * SLOT;
+        const unsigned long long* buf = slots + copy * per + at;
+        // the emptied slot of the next buffer is in memory before this
+        // publication, after which another block may look for it
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if (lane < COPIES)
+#pragma unroll
+            for (int k = 0; k < NV; ++k) {
+                unsigned long long u = __double_as_longlong(s[k]);
+                if (u == EMPTY) u = 0x7ff8000000000000ull;
+                slot_store(&slots[lane * per + at + (int64_t)me * SLOT + k], u);
+            }
+        unsigned long long got[MAX_TEAM / 64][NV];
+        const unsigned long long t0 = wall_clock64();
+        for (unsigned round = 0;; ++round) {
+            bool all = true;
+#pragma unroll
+            for (int i = 0; i < MAX_TEAM / 64; ++i) {
+                const int m = lane + 64 * i;
+#pragma unroll
+                for (int k = 0; k < NV; ++k) got[i][k] = m < nb ? slot_load(&buf[(size_t)m * SLOT + k]) : 0ull;
+            }
+#pragma unroll
+            for (int i = 0; i < MAX_TEAM / 64; ++i)
+#pragma unroll
+                for (int k = 0; k < NV; ++k) all = all && got[i][k] != EMPTY;
+            if (__all(all)) break;
+            if ((round & 255u) == 255u && wall_clock64() - t0 > WAIT_TICKS) {
+                if (lane == 0) {
+                    *bad = 1;
+                    __hip_atomic_store(abort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+                break;
+            }
+        }
+        // nothing after this is read before the slots were
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int k = 0; k < NV; ++k) {
+            double a = 0.0;
+#pragma unroll
+            for (int i = 0; i < MAX_TEAM / 64; ++i) a += __longlong_as_double(got[i][k]);
+            s[k] = wave_sum(a);
+        }
+        if (lane < COPIES) {
+            unsigned long long* nxt = slots + lane * per + ((int64_t)((phase + 2) % 3) * nb + me) * SLOT;
+#pragma unroll
+            for (int k = 0; k < W; ++k) slot_store(&nxt[k], EMPTY);
+        }
+        ++phase;
+    }
+};
+
+// One step of a lane group: U columns per lane (window indices in pairs), their
+// entries in the group's rows.
+constexpr int U = TEAM_COLS;
+template <typename TA, int DIM>
+struct Step {
+    uint32_t c[(U + 1) / 2];
+    TA v[DIM][U];
+    __device__ int col(int u) const { return (int)(u & 1 ? c[u / 2] >> 16 : c[u / 2] & 0xffffu); }
+};
+
+template <typename TA, int NR, int DIM, int TIER, int KEEP>
+__global__ __launch_bounds__(TT) void k_team_pcg(TeamArgs<TA> a) {
+    constexpr int G = team_lanes(DIM), GP = TT / G;
+    constexpr bool ALL = TIER == WIN_ALL;
+    constexpr int RB = ALL ? 1 : 4;  // rows per trip: operands in memory want several on the way
+    constexpr int W = slot_values<NR>();
+    extern __shared__ __align__(16) unsigned char s_dyn[];
+    __shared__ double s_red[16][W], s_tot[W];
+    __shared__ int s_bad;
+    const int t = threadIdx.x, sub = t % G;
+    int team = blockIdx.x % a.n_teams, me = blockIdx.x / a.n_teams;
+    // blocks go round-robin to the dies (XCDs): neighbouring shares of one
+    // system on one die, so the entries they both read sit in one L2
+    if (a.n_teams == 1 && a.team_blocks % 8 == 0) me = (blockIdx.x % 8) * (a.team_blocks / 8) + blockIdx.x / 8;
+    TeamSum<NR> sum{a.slots + team * COPIES * team_slots(a.team_blocks), a.team_blocks, me,
+                    (int)(blockIdx.x % COPIES), 0u, s_red, s_tot, &s_bad, a.abort};
+    if (t < 16 * W) (&s_red[0][0])[t] = 0.0;
+    if (t == 0) s_bad = 0;
+    __syncthreads();
+    const __amdgpu_buffer_rsrc_t zrs =
+        __builtin_amdgcn_make_buffer_rsrc(a.zp, (short)0, (int)(uint32_t)a.zp_bytes, 0x00027000);
+    int pos = a.team_pos[2 * team], left = a.launch_its;
+    bool resume = a.team_pos[2 * team + 1] != 0;
+    const int end = a.team_sys[team + 1];
+    while (pos < end && left > 0) {
+        const int sys = a.sys_list[pos];
+        const size_t share = (size_t)sys * a.team_blocks + me;
+        const int32_t* rp = a.row_ptr + (size_t)sys * (a.team_blocks + 1) + me;
+        const int row0 = rp[0], nrow = rp[1] - row0;
+        const StepRec* steps = a.steps + a.step_ptr[share] * GP + t / G;  // this lane group's, GP apart
+        const int ns = (int)(a.step_ptr[share + 1] - a.step_ptr[share]);
+        const int64_t h0 = a.halo_ptr[share];
+        const int nh = (int)(a.halo_ptr[share + 1] - h0);
+        const int nw = nrow + nh;
+        // LDS: p of the window by right-hand side [NR][nw], then q (z from the
+        // update on) and r [NR][nrow], 1/diag [nrow]
+        double* Lp = (double*)s_dyn;
+        double* Lq = Lp + (size_t)nw * NR;
+        double* Lr = Lq + (size_t)nrow * NR;
+        double* Ld = Lr + (size_t)nrow * NR;
+        double* xg = a.x + (size_t)row0 * NR;
+        double* rg = a.r + (size_t)row0 * NR;
+        double2* zg = a.zp + (size_t)row0 * NR;
+        const double* dg = a.dinv + row0;
+        double* st = a.state + (size_t)sys * NR * T_N;
+        double rz[NR], beta[NR], rr[NR], rr0[NR], tol[NR];
+        bool act[NR];
+        int it[NR];
+        auto store_pair = [&](int i, int c, double z, double p) {
+            pair_store(zrs, (uint32_t)(row0 + i) * NR + c, double2{z, p});
+        };
+        // (unconditional loads at clamped places, zeroed afterwards: a load
+        // under a condition is a branch the next one waits behind)
+        auto load_step = [&](const StepRec& r, Step<TA, DIM>& s) {
+            const int k = (r.what >> 8) & 3, len = r.what & 255;
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int j = sub + u * G;
+                const int e = r.begin + min(j, max(len - 1, 0));
+                const uint32_t w = a.wcol[e];
+                if (u & 1) s.c[u / 2] |= (len > 0 ? w : 0u) << 16;
+                else s.c[u / 2] = len > 0 ? w : 0u;
+#pragma unroll
+                for (int h = 0; h < DIM; ++h) s.v[h][u] = a.A[e + (h < k ? h : 0) * r.stride];
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int h = 0; h < DIM; ++h) s.v[h][u] = sub + u * G < len && h < k ? s.v[h][u] : (TA)0;
+        };
+        // row in the share << 4, first and last step, rows of the group
+        auto info_of = [](const StepRec& r) {
+            return r.row << 4 | (r.what & STEP_CONT ? 8 : 0) | (r.what & STEP_LAST ? 4 : 0) | ((r.what >> 8) & 3);
+        };
+        if (resume) {
+            for (int i = t; i < nrow; i += TT) {
+                if (ALL) Ld[i] = dg[i];
+                for (int c = 0; c < NR; ++c) {
+                    if (ALL) Lr[c * nrow + i] = rg[i * NR + c];
+                    Lp[c * nw + i] = zg[i * NR + c].y;
+                    Lq[c * nrow + i] = zg[i * NR + c].x;
+                }
+            }
+            for (int c = 0; c < NR; ++c) {
+                rz[c] = uniform(st[c * T_N + T_RZ]);
+                beta[c] = uniform(st[c * T_N + T_BETA]);
+                rr[c] = uniform(st[c * T_N + T_RR]);
+                rr0[c] = uniform(st[c * T_N + T_RR0]);
+                tol[c] = uniform(st[c * T_N + T_TOL]);
+                it[c] = __builtin_amdgcn_readfirstlane((int)st[c * T_N + T_IT]);
+                act[c] = uniform(st[c * T_N + T_DONE]) == 0.0;
+            }
+        } else {
+            double v[W];
+            for (int k = 0; k < W; ++k) v[k] = 0.0;
+            for (int i = t; i < nrow; i += TT) {
+                const int32_t dgi = a.diag[row0 + i];
+                const double d = dgi >= 0 ? (double)a.A[dgi] : 0.0;
+                const double di = d != 0.0 ? 1.0 / d : (a.single ? 1.0 : 0.0);
+                a.dinv[row0 + i] = di;
+                if (ALL) Ld[i] = di;
+                for (int c = 0; c < NR; ++c) {
+                    const int64_t e = (int64_t)(row0 + i) * NR + c;
+                    const double bi = a.b[e], ri = a.Ax ? bi - a.Ax[e] : bi;
+                    const double zi = di * ri;
+                    if (!a.Ax) a.x[e] = 0.0;
+                    if (ALL) Lr[c * nrow + i] = ri;
+                    else a.r[e] = ri;
+                    Lp[c * nw + i] = 0.0;
+                    Lq[c * nrow + i] = zi;
+                    store_pair(i, c, zi, 0.0);
+                    v[c] += ri * zi;
+                    v[NR + c] += ri * ri;
+                    if (NR == 1) v[W - 1] += bi * bi;
+                }
+            }
+            if (!sum(v, true, [] {})) return;
+            for (int c = 0; c < NR; ++c) {
+                rz[c] = v[c];
+                rr[c] = v[NR + c];
+                // the single solve is relative to ||b||, also from a nonzero start
+                rr0[c] = NR == 1 && a.single ? v[W - 1] : rr[c];
+                tol[c] = uniform(a.tol2 * rr0[c]);
+                beta[c] = 0.0;
+                it[c] = 0;
+                act[c] = a.single ? (rr[c] > tol[c] && a.maxit > 0) : rr[c] != 0.0;
+            }
+        }
+        bool any = false;
+        for (int c = 0; c < NR; ++c) any = any || act[c];
+        // K entries that stay in registers: every step (KEEP), or the first two
+        constexpr int NK = KEEP > 0 ? KEEP : 2;
+        Step<TA, DIM> keep[NK];
+        int info[NK];
+#pragma unroll
+        for (int s = 0; s < NK; ++s) {
+            StepRec r = {0, 0, 0, 0};
+            if (s < ns) r = steps[s * GP];
+            info[s] = info_of(r);
+            load_step(r, keep[s]);
+        }
+        StepRec rec2 = {0, 0, 0, 0};
+        if (KEEP == 0 && ns > 2) rec2 = steps[2 * GP];
+        while (any && left > 0) {
+            // ---- p of the window
+            // (every loop over rows or columns issues the loads of several
+            // trips before it uses the first)
+            constexpr int HB = NR == 1 ? 8 : 8 / NR;
+            for (int i0 = t; i0 < nh; i0 += HB * TT) {
+                uint32_t col[HB];
+                double2 e[HB][NR];
+#pragma unroll
+                for (int k = 0; k < HB; ++k) col[k] = (uint32_t)a.halo[h0 + min(i0 + k * TT, nh - 1)];
+#pragma unroll
+                for (int k = 0; k < HB; ++k)
+#pragma unroll
+                    for (int c = 0; c < NR; ++c) e[k][c] = pair_load(zrs, col[k] * NR + c);
+#pragma unroll
+                for (int k = 0; k < HB; ++k)
+                    if (i0 + k * TT < nh)
+#pragma unroll
+                        for (int c = 0; c < NR; ++c)
+                            Lp[c * nw + nrow + i0 + k * TT] = e[k][c].x + beta[c] * e[k][c].y;
+            }
+            for (int i = t; i < nrow; i += TT)
+#pragma unroll
+                for (int c = 0; c < NR; ++c) Lp[c * nw + i] = Lq[c * nrow + i] + beta[c] * Lp[c * nw + i];
+            __syncthreads();
+            // ---- q = K p, p.q: G lanes per group of rows with one column list
+            double pq[NR];
+            for (int c = 0; c < NR; ++c) pq[c] = 0.0;
+            auto add = [&](const Step<TA, DIM>& s, double (&acc)[DIM][NR]) {
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+#pragma unroll
+                    for (int c = 0; c < NR; ++c) {
+                        const double p = Lp[c * nw + s.col(u)];
+#pragma unroll
+                        for (int h = 0; h < DIM; ++h) acc[h][c] += (double)s.v[h][u] * p;
+                    }
+            };
+            double acc[DIM][NR];
+            auto step = [&](const Step<TA, DIM>& s, int what) {
+                if (!(what & 8))
+#pragma unroll
+                    for (int h = 0; h < DIM; ++h)
+#pragma unroll
+                        for (int c = 0; c < NR; ++c) acc[h][c] = 0.0;
+                add(s, acc);
+                if (!(what & 4)) return;  // uniform over the lane group
+                const int k = what & 3, i = (what >> 4) + sub;
+#pragma unroll
+                for (int c = 0; c < NR; ++c) {
+#pragma unroll
+                    for (int h = 0; h < DIM; ++h) acc[h][c] = lane_sum<G>(acc[h][c]);
+                    if (sub < k) {
+                        double qi = acc[0][c];
+                        if (sub == 1) qi = acc[1][c];
+                        if (DIM == 3 && sub == 2) qi = acc[DIM - 1][c];
+                        Lq[c * nrow + i] = qi;
+                        pq[c] += Lp[c * nw + i] * qi;
+                    }
+                }
+            };
+            if (KEEP > 0) {
+#pragma unroll
+                for (int s = 0; s < NK; ++s)
+                    if (s < ns) {
+                        // FP32 entries stay FP32 in their registers: without
+                        // this the compiler widens them once before the loop
+                        if (sizeof(TA) == 4)
+#pragma unroll
+                            for (int h = 0; h < DIM; ++h)
+#pragma unroll
+                                for (int u = 0; u < U; ++u) asm volatile("" : "+v"(keep[s].v[h][u]));
+                        step(keep[s], info[s]);
+                    }
+            } else {
+                // three steps' entries in registers: one in use, two on the way
+                Step<TA, DIM> cur = keep[0], nxt = keep[1], far;
+                int ci = info[0], ni = info[1], fi = 0;
+                StepRec rf = rec2;
+                for (int s = 0; s < ns; ++s) {
+                    if (s + 2 < ns) {
+                        fi = info_of(rf);
+                        load_step(rf, far);
+                        if (s + 3 < ns) rf = steps[(size_t)(s + 3) * GP];
+                    }
+                    step(cur, ci);
+                    cur = nxt;
+                    nxt = far;
+                    ci = ni;
+                    ni = fi;
+                }
+            }
+            if (!sum(pq, false, [] {})) return;
+            double alpha[NR];
+            for (int c = 0; c < NR; ++c) {
+                alpha[c] = uniform(pq[c] != 0.0 && !(a.single && !isfinite(pq[c])) ? rz[c] / pq[c] : 0.0);
+                if (!act[c]) alpha[c] = 0.0;
+            }
+            // ---- r -= alpha q, z = r / diag, the pair (z, p); r.z and r.r
+            double v[2 * NR];
+            for (int k = 0; k < 2 * NR; ++k) v[k] = 0.0;
+            for (int i0 = t; i0 < nrow; i0 += RB * TT) {
+                double di[RB], ri[RB][NR], qi[RB][NR], pi[RB][NR];
+#pragma unroll
+                for (int k = 0; k < RB; ++k) {
+                    const int i = min(i0 + k * TT, nrow - 1);
+                    di[k] = ALL ? Ld[i] : dg[i];
+#pragma unroll
+                    for (int c = 0; c < NR; ++c) {
+                        ri[k][c] = ALL ? Lr[c * nrow + i] : rg[(size_t)i * NR + c];
+                        qi[k][c] = Lq[c * nrow + i];
+                        pi[k][c] = Lp[c * nw + i];
+                    }
+                }
+#pragma unroll
+                for (int k = 0; k < RB; ++k) {
+                    const int i = i0 + k * TT;
+                    if (i >= nrow) continue;
+#pragma unroll
+                    for (int c = 0; c < NR; ++c) {
+                        if (!act[c]) continue;
+                        const double rn = ri[k][c] - alpha[c] * qi[k][c];
+                        const double zi = di[k] * rn;
+                        if (ALL) Lr[c * nrow + i] = rn;
+                        else rg[(size_t)i * NR + c] = rn;
+                        store_pair(i, c, zi, pi[k][c]);
+                        Lq[c * nrow + i] = zi;
+                        v[c] += rn * zi;
+                        v[NR + c] += rn * rn;
+                    }
+                }
+            }
+            // x += alpha p by the wavefronts that do not wait
+            auto upx = [&] {
+                constexpr int XT = TT - 64, XB = 4;
+                for (int i0 = t - 64; i0 < nrow; i0 += XB * XT) {
+                    double xo[XB][NR];
+#pragma unroll
+                    for (int k = 0; k < XB; ++k)
+#pragma unroll
+                        for (int c = 0; c < NR; ++c) xo[k][c] = xg[(size_t)min(i0 + k * XT, nrow - 1) * NR + c];
+#pragma unroll
+                    for (int k = 0; k < XB; ++k) {
+                        const int i = i0 + k * XT;
+                        if (i >= nrow) continue;
+#pragma unroll
+                        for (int c = 0; c < NR; ++c)
+                            if (act[c])
+                                xg[(size_t)i * NR + c] =
+                                    xo[k][c] + alpha[c] * Lp[c * nw + i];
+                    }
+                }
+            };
+            if (!sum(v, true, upx)) return;
+            any = false;
+            for (int c = 0; c < NR; ++c) {
+                if (!act[c]) continue;
+                beta[c] = uniform(rz[c] != 0.0 ? v[c] / rz[c] : 0.0);
+                rz[c] = v[c];
+                rr[c] = v[NR + c];
+                ++it[c];
+                if (!(rr[c] > tol[c]) || it[c] >= a.maxit || (a.single && !isfinite(rr[c]))) {
+                    act[c] = false;
+                    beta[c] = 0.0;  // its direction stays put while other right-hand sides run
+                }
+                any = any || act[c];
+            }
+            --left;
+        }
+        if (any && ALL)  // to be resumed
+            for (int i = t; i < nrow; i += TT)
+                for (int c = 0; c < NR; ++c) rg[i * NR + c] = Lr[c * nrow + i];
+        if (me == 0 && t == 0)
+            for (int c = 0; c < NR; ++c) {
+                st[c * T_N + T_RZ] = rz[c];
+                st[c * T_N + T_BETA] = beta[c];
+                st[c * T_N + T_RR] = rr[c];
+                st[c * T_N + T_RR0] = rr0[c];
+                st[c * T_N + T_TOL] = tol[c];
+                st[c * T_N + T_IT] = it[c];
+                st[c * T_N + T_DONE] = act[c] ? 0.0 : 1.0;
+            }
+        resume = any;
+        if (any) break;
+        ++pos;
+        __syncthreads();  // the LDS arrays change hands
+    }
+    if (me == 0 && t == 0) {
+        a.team_pos[2 * team] = pos;
+        a.team_pos[2 * team + 1] = resume ? 1 : 0;
+    }
+}
+
+// Window indices of every group's columns (entries of its first row): own
+// rows first, then the place in the block's sorted halo.
+static __global__ __launch_bounds__(256) void k_team_cols(int n_shares, int team_blocks, const int32_t* __restrict__ part,
+                                                   const GroupRec* __restrict__ grp, const int32_t* __restrict__ col,
+                                                   const int64_t* __restrict__ halo_ptr,
+                                                   const int32_t* __restrict__ halo, uint16_t* __restrict__ wcol) {
+    const int share = blockIdx.x;
+    if (share >= n_shares) return;
+    const int32_t* pt = part + (size_t)(share / team_blocks) * (team_blocks + 1) + share % team_blocks;
+    const int g0 = pt[0], g1 = pt[1];
+    const int row0 = grp[g0].row, nrow = grp[g1].row - row0;
+    const int32_t* h = halo + halo_ptr[share];
+    const int nh = (int)(halo_ptr[share + 1] - halo_ptr[share]);
+    for (int g = g0 + (int)threadIdx.x / 8; g < g1; g += 32) {
+        const GroupRec gr = grp[g];
+        for (int j = threadIdx.x % 8; j < gr.len_k >> 2; j += 8) {
+            const int c = col[gr.begin + j];
+            int w = c - row0;
+            if (w < 0 || w >= nrow) {
+                int lo = 0, hi = nh;  // first halo entry >= c
+                while (lo < hi) {
+                    const int m = (lo + hi) >> 1;
+                    if (h[m] < c) lo = m + 1;
+                    else hi = m;
+                }
+                w = nrow + lo;
+            }
+            wcol[gr.begin + j] = (uint16_t)w;
+        }
+    }
+}
+
+// Passes a lane can keep in its registers.
+template <typename TA, int NR, int DIM>
+constexpr int max_keep() {
+    return sizeof(TA) == 8 ? (DIM == 3 ? 7 : (NR == 1 ? 10 : 8)) : (DIM == 3 ? 12 : 16);
+}
+
+struct TeamShape {
+    const void* kernel = nullptr;  // null: no kernel holds the plan's largest share
+    unsigned lds = 0;
+};
+
+// The kernel for the plan's largest share: everything in LDS and K in registers
+// where it fits, then K streamed, then r and 1/diag in memory.  us per
+// iteration of a single solve, against five launches:
+//   K in registers: 100 x 100 quads 5.9 (21.3), 333 x 333 10.2 (34.3),
+//     40^3 x 6 tets with FP32 values 12.3 (40.7);
+//   streamed: 460 x 460 quads 22.6 (49.4), 50^3 x 6 tets 36.9 (70.0);
+//   r and 1/diag in memory: 64^3 x 6 tets 100 (159), 700 x 700 quads 47.9 (93.6).
+// A window beyond the LDS was tried with gathers through the L2 and fences:
+// 1000 x 1000 quads 212 (196), 80^3 x 6 tets 297 (279): those keep the launches.
+template <typename TA, int NR, int DIM>
+TeamShape team_shape(const TeamPlan& p) {
+    const size_t win = sizeof(double) * NR * (size_t)p.max_window, row = sizeof(double) * (size_t)p.max_rows;
+    const size_t all = win + row * (2 * NR + 1), pq = win + row * NR;
+    constexpr int K = max_keep<TA, NR, DIM>();
+    TeamShape s;
+    if (p.max_window > MAX_WINDOW || pq > LDS_MAX) return s;
+    if (all > LDS_MAX) s = {reinterpret_cast<const void*>(&k_team_pcg<TA, NR, DIM, WIN_PQ, 0>), (unsigned)pq};
+    else if (p.max_passes > K) s = {reinterpret_cast<const void*>(&k_team_pcg<TA, NR, DIM, WIN_ALL, 0>), (unsigned)all};
+    else s = {reinterpret_cast<const void*>(&k_team_pcg<TA, NR, DIM, WIN_ALL, K>), (unsigned)all};
+    return s;
+}
+
+}  // namespace pgft
