@@ -1134,18 +1134,35 @@ __global__ void k_round32(int64_t n, const double* __restrict__ src, float* __re
 // Homogenised response of an RVE (SubscaleModel::homogenize_stress_strain,
 // src/SubscaleModel.cpp:42-196): over every volumetric point of the elements
 // of a segment, sum w * sigma with sigma = D (eps(u) + eps_bar), w * eps(u)
-// and w.  Segment k (elements [seg[k], seg[k+1])) is split evenly over
-// VOL_BLOCKS blocks; each block writes one partial per quantity, and
-// k_vol_finish adds a segment's partials in block order (deterministic).
-constexpr int VOL_BLOCKS = 64;
+// and w.  Segment k (elements [seg[k], seg[k+1])) is split evenly over vb
+// blocks; each block writes one partial per quantity, and k_vol_finish adds a
+// segment's partials in a fixed order (deterministic).
+//
+// Bound by memory latency: per element one connectivity record and four nodes.
+// vb gives every thread about one element as long as the launch stays within
+// VOL_LAUNCH blocks (701 x 701 quads in one segment: 1.66 ms with 64 blocks a
+// segment, 41 us with 1920).  The block's cut elements are listed and taken by
+// 32 (2D) or 16 (3D) lanes each, one point per lane: one thread walking its
+// points holds up the other 63, and one wavefront taking them one after the
+// other still needs 64 us.
+constexpr int VOL_LAUNCH = 4096;
+
+int vol_blocks(int n_seg, int64_t n_elem) {
+    const int64_t want = (n_elem / std::max(n_seg, 1) + 255) / 256;
+    return (int)std::max<int64_t>(1, std::min<int64_t>({want, VOL_LAUNCH / n_seg, 2048}));
+}
 
 template <int DIM>
-__global__ __launch_bounds__(256) void k_vol_partials(AsmArgs a, const double* __restrict__ eps_bar,
+__global__ __launch_bounds__(256) void k_vol_partials(AsmArgs a, int vb, const double* __restrict__ eps_bar,
                                                       const int64_t* __restrict__ seg, double* __restrict__ part) {
     constexpr int S = DIM == 2 ? 3 : 6, NQ = DIM == 2 ? 4 : 1, W = 2 * S + 1;
-    const int k = blockIdx.x / VOL_BLOCKS, b = blockIdx.x % VOL_BLOCKS;
+    const int k = blockIdx.x / vb, b = blockIdx.x % vb;
     const int64_t e0 = seg[k], len = seg[k + 1] - e0;
-    const int64_t c0 = e0 + len * b / VOL_BLOCKS, c1 = e0 + len * (b + 1) / VOL_BLOCKS;
+    const int64_t c0 = e0 + len * b / vb, c1 = e0 + len * (b + 1) / vb;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    constexpr int PL = max_vpt(DIM);  // lanes per cut element: its points
+    static_assert(64 % PL == 0, "a cut element's lanes stay in one wavefront");
+    __shared__ int s_n[4], s_cut[256];
     double acc[W];
     for (int i = 0; i < W; ++i) acc[i] = 0.0;
     double eb[S];
@@ -1160,16 +1177,25 @@ __global__ __launch_bounds__(256) void k_vol_partials(AsmArgs a, const double* _
         }
         acc[2 * S] += w;
     };
-    for (int64_t e = c0 + threadIdx.x; e < c1; e += blockDim.x) {
-        const int c = a.cut_index[e];
-        if (c < 0) {
+    for (int64_t base = c0; base < c1; base += 256) {
+        const int64_t e = base + threadIdx.x;
+        const int c = e < c1 ? a.cut_index[e] : -1;
+        if (e < c1 && c < 0) {
+            const int4 cn = a.el_conn4[e];
+            const int nd[4] = {cn.x, cn.y, cn.z, cn.w};
             double X[4][DIM], u[4 * DIM];
             for (int q = 0; q < 4; ++q) {
-                const int nd = a.el_conn[(int64_t)q * a.n_elem + e];
-                for (int i = 0; i < DIM; ++i) {
-                    X[q][i] = a.X[i * a.n_all + nd];
-                    u[q * DIM + i] = a.U[i * a.n_all + nd];
+                if (DIM == 2) {
+                    const double2 xv = ((const double2*)a.Xq)[nd[q]];
+                    X[q][0] = xv.x;
+                    X[q][1] = xv.y;
+                } else {
+                    const double4 xv = ((const double4*)a.Xq)[nd[q]];
+                    X[q][0] = xv.x;
+                    X[q][1] = xv.y;
+                    X[q][DIM - 1] = xv.z;
                 }
+                for (int i = 0; i < DIM; ++i) u[q * DIM + i] = a.U[i * a.n_all + nd[q]];
             }
             const Iso D = iso_of<DIM>(a.Dmat + a.el_mat[e] * 36);
             for (int q = 0; q < NQ; ++q) {
@@ -1178,45 +1204,71 @@ __global__ __launch_bounds__(256) void k_vol_partials(AsmArgs a, const double* _
                 strain_of<DIM>(4, g, u, eps);
                 add_point(D, eps, w);
             }
-        } else {
-            const int nt = a.ce_nt[c];
-            double u[MAX_NT * DIM];
-            for (int s = 0; s < nt; ++s) {
-                const int nd = a.ce_nodes[c * 16 + s];
-                for (int i = 0; i < DIM; ++i) u[s * DIM + i] = a.U[i * a.n_all + nd];
-            }
-            for (int64_t pt = a.vpt_ptr[c]; pt < a.vpt_ptr[c + 1]; ++pt) {
+        }
+        // the cut elements of these 256, in element order, PL lanes each
+        const unsigned long long cut = __ballot(c >= 0);
+        if (lane == 0) s_n[wv] = __popcll(cut);
+        __syncthreads();
+        int at = 0, n_cut = 0;
+        for (int w = 0; w < 4; ++w) {
+            at += w < wv ? s_n[w] : 0;
+            n_cut += s_n[w];
+        }
+        if (c >= 0) s_cut[at + __popcll(cut & ((1ull << lane) - 1))] = c;
+        __syncthreads();
+        for (int i = threadIdx.x / PL; i < n_cut; i += 256 / PL) {
+            const int cc = s_cut[i];
+            const int64_t pt = a.vpt_ptr[cc] + threadIdx.x % PL;
+            const int nt = a.ce_nt[cc];
+            if (pt < a.vpt_ptr[cc + 1]) {
+                const double* g = a.vpt_grad + a.vpt_grad_off[pt];
                 double eps[S];
-                strain_of<DIM>(nt, a.vpt_grad + a.vpt_grad_off[pt], u, eps);
+                for (int i = 0; i < S; ++i) eps[i] = 0.0;
+                for (int s = 0; s < nt; ++s) {
+                    const int nd = a.ce_nodes[cc * 16 + s];
+                    double u[DIM], e1[S];
+                    for (int i = 0; i < DIM; ++i) u[i] = a.U[i * a.n_all + nd];
+                    strain_of<DIM>(1, g + s * DIM, u, e1);
+                    for (int i = 0; i < S; ++i) eps[i] += e1[i];
+                }
                 add_point(iso_of<DIM>(a.Dmat + a.vpt_mat[pt] * 36), eps, a.vpt_w[pt]);
             }
         }
     }
-    // block tree sum in a fixed order
-    __shared__ double red[256];
+    // lanes, then wavefronts, in a fixed order
+    __shared__ double red[4][W];
     for (int i = 0; i < W; ++i) {
-        red[threadIdx.x] = acc[i];
-        __syncthreads();
-        for (int h = 128; h > 0; h >>= 1) {
-            if ((int)threadIdx.x < h) red[threadIdx.x] += red[threadIdx.x + h];
-            __syncthreads();
-        }
-        if (threadIdx.x == 0) part[(int64_t)blockIdx.x * W + i] = red[0];
-        __syncthreads();
+        for (int m = 32; m >= 1; m >>= 1) acc[i] += __shfl_xor(acc[i], m, 64);
+        if (lane == 0) red[wv][i] = acc[i];
     }
+    __syncthreads();
+    if (threadIdx.x < W)
+        part[(int64_t)blockIdx.x * W + threadIdx.x] =
+            (red[0][threadIdx.x] + red[1][threadIdx.x]) + (red[2][threadIdx.x] + red[3][threadIdx.x]);
 }
 
-// out[k] = (averaged stress [S], averaged fluctuation strain [S], volume)
-__global__ void k_vol_finish(int n_seg, int S, const double* __restrict__ part, double* __restrict__ out) {
-    const int W = 2 * S + 1;
-    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n_seg; k += gridDim.x * blockDim.x) {
-        double sum[13];
-        for (int i = 0; i < W; ++i) sum[i] = 0.0;
-        for (int b = 0; b < VOL_BLOCKS; ++b)
-            for (int i = 0; i < W; ++i) sum[i] += part[((int64_t)k * VOL_BLOCKS + b) * W + i];
-        const double v = sum[2 * S];
-        for (int i = 0; i < 2 * S; ++i) out[(int64_t)k * W + i] = v != 0.0 ? sum[i] / v : 0.0;
-        out[(int64_t)k * W + 2 * S] = v;
+// out[k] = (averaged stress [S], averaged fluctuation strain [S], volume): one
+// block per segment
+template <int DIM>
+__global__ __launch_bounds__(256) void k_vol_finish(int vb, const double* __restrict__ part, double* __restrict__ out) {
+    constexpr int S = DIM == 2 ? 3 : 6, W = 2 * S + 1;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const double* p = part + (int64_t)blockIdx.x * vb * W;
+    double acc[W];
+    for (int i = 0; i < W; ++i) acc[i] = 0.0;
+    for (int b = threadIdx.x; b < vb; b += 256)
+        for (int i = 0; i < W; ++i) acc[i] += p[(int64_t)b * W + i];
+    __shared__ double red[4][W];
+    for (int i = 0; i < W; ++i) {
+        for (int m = 32; m >= 1; m >>= 1) acc[i] += __shfl_xor(acc[i], m, 64);
+        if (lane == 0) red[wv][i] = acc[i];
+    }
+    __syncthreads();
+    if (threadIdx.x < W) {
+        const int i = threadIdx.x;
+        const double v = (red[0][2 * S] + red[1][2 * S]) + (red[2][2 * S] + red[3][2 * S]);
+        const double s = (red[0][i] + red[1][i]) + (red[2][i] + red[3][i]);
+        out[(int64_t)blockIdx.x * W + i] = i == 2 * S ? v : (v != 0.0 ? s / v : 0.0);
     }
 }
 
@@ -1315,14 +1367,19 @@ static void launch_dim(Ctx& c, const pgfk::AsmArgs& a, bool jac, bool func, bool
     if (func && (fp32 || !jac)) launch_gather<DIM, false, true, double>(c, a);
 }
 
-void enqueue_volume_average(Ctx& c, const double* d_eps_bar, int n_seg, const int64_t* d_seg, double* d_part,
+int volume_average_blocks(int n_seg, int64_t n_elem) { return pgfk::vol_blocks(n_seg, n_elem); }
+
+void enqueue_volume_average(Ctx& c, const double* d_eps_bar, int n_seg, int vb, const int64_t* d_seg, double* d_part,
                             double* d_out) {
     const pgfk::AsmArgs a = c.asm_args();
-    const dim3 grid((unsigned)(n_seg * pgfk::VOL_BLOCKS)), blk(256);
-    if (c.dim == 2) hipLaunchKernelGGL((pgfk::k_vol_partials<2>), grid, blk, 0, c.stream, a, d_eps_bar, d_seg, d_part);
-    else hipLaunchKernelGGL((pgfk::k_vol_partials<3>), grid, blk, 0, c.stream, a, d_eps_bar, d_seg, d_part);
-    hipLaunchKernelGGL(pgfk::k_vol_finish, dim3((unsigned)((n_seg + 63) / 64)), dim3(64), 0, c.stream, n_seg,
-                       c.dim == 2 ? 3 : 6, d_part, d_out);
+    const dim3 grid((unsigned)(n_seg * vb)), blk(256);
+    if (c.dim == 2) {
+        hipLaunchKernelGGL((pgfk::k_vol_partials<2>), grid, blk, 0, c.stream, a, vb, d_eps_bar, d_seg, d_part);
+        hipLaunchKernelGGL((pgfk::k_vol_finish<2>), dim3((unsigned)n_seg), blk, 0, c.stream, vb, d_part, d_out);
+    } else {
+        hipLaunchKernelGGL((pgfk::k_vol_partials<3>), grid, blk, 0, c.stream, a, vb, d_eps_bar, d_seg, d_part);
+        hipLaunchKernelGGL((pgfk::k_vol_finish<3>), dim3((unsigned)n_seg), blk, 0, c.stream, vb, d_part, d_out);
+    }
 }
 
 void enqueue_set_from_dofs(Ctx& c, const double* d_x, const double* d_up) {

@@ -76,6 +76,17 @@ void fill_async(Ctx& c, T* p, int64_t n, T v) {
 template void fill_async<double>(Ctx&, double*, int64_t, double);
 template void fill_async<float>(Ctx&, float*, int64_t, float);
 
+double* Ctx::workspace(int64_t doubles) {
+    if (doubles > work_n) {
+        if (work) HIPCHK(hipFree(work));
+        work = nullptr;
+        work_n = 0;
+        work = dalloc<double>(doubles);
+        work_n = doubles;
+    }
+    return work;
+}
+
 pgfk::AsmArgs Ctx::asm_args() const {
     pgfk::AsmArgs a{};
     a.n_all = n_all; a.n_free = n_free; a.n_rows = n_rows; a.n_uncut = n_uncut;
@@ -97,7 +108,7 @@ pgfk::AsmArgs Ctx::asm_args() const {
 }
 
 Ctx::~Ctx() {
-    void* ptrs[] = {X, dof, U, ue_conn, ue_mat, ue_off, Dmat, ce_list, ce_nodes, ce_nt, vpt_ptr, vpt_grad_off, cpt_ptr,
+    void* ptrs[] = {work, X, dof, U, ue_conn, ue_mat, ue_off, Dmat, ce_list, ce_nodes, ce_nt, vpt_ptr, vpt_grad_off, cpt_ptr,
                     ce_off_ptr, vpt_w, vpt_grad, cpt_w, cpt_N, cpt_R, vpt_mat, cpt_law, cpt_nodes, cpt_nh, ce_off, laws,
                     dmax_conv, dmax_trial, flags, free_slot, rowptr, rowsplit, colidx, K, K32, P, Fext_full,
                     upres_full, r, x, zp, q, dinv, guess, res, partial,
@@ -1166,13 +1177,13 @@ PGF_API int pgf_set_solution(pgf_ctx* c, const double* u) {
 PGF_API int pgf_set_solution_dofs(pgf_ctx* c, const double* x_free, const double* u_pres) {
     if (!c || !x_free) return PGF_EARG;
     return guard(c, [&]() -> int {
-        double* dx = pgfd::dupload(x_free, std::max<int64_t>(c->n_free, 1));
-        double* dp = u_pres ? pgfd::dupload(u_pres, std::max<int64_t>(c->n_pres, 1)) : nullptr;
-        pgfd::enqueue_set_from_dofs(*c, dx, dp);
+        // (c->res holds a solve's right-hand side, no longer than the solve)
+        double* dp = u_pres && c->n_pres ? c->workspace(c->n_pres) : nullptr;
+        HIPCHK(hipMemcpyAsync(c->res, x_free, sizeof(double) * c->n_free, hipMemcpyHostToDevice, c->stream));
+        if (dp) HIPCHK(hipMemcpyAsync(dp, u_pres, sizeof(double) * c->n_pres, hipMemcpyHostToDevice, c->stream));
+        pgfd::enqueue_set_from_dofs(*c, c->res, dp);
         HIPCHK(hipGetLastError());
         HIPCHK(hipStreamSynchronize(c->stream));
-        HIPCHK(hipFree(dx));
-        if (dp) HIPCHK(hipFree(dp));
         return 0;
     });
 }
@@ -1184,15 +1195,18 @@ PGF_API int pgf_volume_average(pgf_ctx* c, const double* eps_bar, int32_t n_seg,
             if (seg_elem[k] < 0 || seg_elem[k] > seg_elem[k + 1] || seg_elem[k + 1] > c->n_elem)
                 throw pgf::Error(PGF_EARG, "element segments must be ordered ranges inside [0, n_elem]");
         const int S = c->dim == 2 ? 3 : 6, W = 2 * S + 1;
-        double* de = pgfd::dupload(eps_bar, S);
-        int64_t* ds = pgfd::dupload(seg_elem, (int64_t)n_seg + 1);
-        double* dpart = pgfd::dalloc<double>((int64_t)n_seg * 64 * W);
-        double* dout = pgfd::dalloc<double>((int64_t)n_seg * W);
-        pgfd::enqueue_volume_average(*c, de, n_seg, ds, dpart, dout);
+        const int vb = pgfd::volume_average_blocks(n_seg, seg_elem[n_seg] - seg_elem[0]);
+        // eps_bar [8] | segments [n_seg + 1] | out [n_seg][W] | partials
+        double* de = c->workspace(8 + n_seg + 1 + (int64_t)n_seg * (vb + 1) * W);
+        int64_t* ds = (int64_t*)(de + 8);
+        double* dout = de + 8 + n_seg + 1;
+        double* dpart = dout + (int64_t)n_seg * W;
+        HIPCHK(hipMemcpyAsync(de, eps_bar, sizeof(double) * S, hipMemcpyHostToDevice, c->stream));
+        HIPCHK(hipMemcpyAsync(ds, seg_elem, sizeof(int64_t) * (n_seg + 1), hipMemcpyHostToDevice, c->stream));
+        pgfd::enqueue_volume_average(*c, de, n_seg, vb, ds, dpart, dout);
         HIPCHK(hipGetLastError());
         HIPCHK(hipMemcpyAsync(out, dout, sizeof(double) * n_seg * W, hipMemcpyDeviceToHost, c->stream));
         HIPCHK(hipStreamSynchronize(c->stream));
-        for (void* p : {(void*)de, (void*)ds, (void*)dpart, (void*)dout}) HIPCHK(hipFree(p));
         return 0;
     });
 }
@@ -1217,7 +1231,8 @@ PGF_API int pgf_volume_average_noalloc(pgf_ctx* c, const double* eps_bar, int32_
         double* dpart = dout + (size_t)PGF_NOALLOC_MAX_SEG * 13;
         HIPCHK(hipMemcpyAsync(de, eps_bar, sizeof(double) * S, hipMemcpyHostToDevice, c->stream));
         HIPCHK(hipMemcpyAsync(ds, seg_elem, sizeof(int64_t) * (n_seg + 1), hipMemcpyHostToDevice, c->stream));
-        pgfd::enqueue_volume_average(*c, de, n_seg, ds, dpart, dout);
+        pgfd::enqueue_volume_average(*c, de, n_seg, pgfd::volume_average_blocks(n_seg, seg_elem[n_seg] - seg_elem[0]), ds,
+                                     dpart, dout);
         HIPCHK(hipGetLastError());
         HIPCHK(hipMemcpyAsync(out, dout, sizeof(double) * n_seg * W, hipMemcpyDeviceToHost, c->stream));
         HIPCHK(hipStreamSynchronize(c->stream));

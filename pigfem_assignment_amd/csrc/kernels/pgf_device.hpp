@@ -98,6 +98,11 @@ struct Ctx {
     double* scal = nullptr;        // device scalars: PCG state (pgft::T_N), residual norm
     unsigned* counter = nullptr;   // last-block counters
     double* h_scal = nullptr;      // pinned mirror
+    // small inputs and results of one call (volume averages), grown as needed
+    // and freed with the context
+    double* work = nullptr;
+    int64_t work_n = 0;
+    double* workspace(int64_t doubles);
     bool have_guess = false;
     hipEvent_t* timing_events = nullptr;  // when set: cut pass start, gather start, gather end
     LearnState* learn = nullptr;
@@ -109,8 +114,11 @@ struct Ctx {
 template <typename T>
 void fill_async(Ctx& c, T* p, int64_t n, T v);
 void enqueue_assembly(Ctx& c, double dt, uint32_t flags);
-// homogenised response per element segment (partials [n_seg * 64][2S+1], out [n_seg][2S+1])
-void enqueue_volume_average(Ctx& c, const double* d_eps_bar, int n_seg, const int64_t* d_seg, double* d_part,
+// homogenised response per element segment: blocks per segment for n_seg
+// segments of n_elem elements in all, at most max(VOL_LAUNCH, n_seg) in the launch;
+// partials [n_seg * vb][2S+1], out [n_seg][2S+1]
+int volume_average_blocks(int n_seg, int64_t n_elem);
+void enqueue_volume_average(Ctx& c, const double* d_eps_bar, int n_seg, int vb, const int64_t* d_seg, double* d_part,
                             double* d_out);
 // the current device's scratch of the allocation-free entry point
 double* noalloc_scratch();
