@@ -6,17 +6,17 @@
 
 namespace pgft {
 
-void make_team_plan(int dim, const std::vector<GroupRec>& grp, const std::vector<int64_t>& sys_grp, const int32_t* colidx,
-                    int blocks, TeamPlan& plan) {
-    const int n_sys = (int)sys_grp.size() - 1;
+bool make_team_plan(int dim, const std::vector<GroupRec>& grp, const std::vector<SysGroups>& sys, const int32_t* colidx,
+                    int blocks, int64_t fit_window, TeamPlan& plan) {
+    const int n_sys = (int)sys.size();
     plan = TeamPlan();
     plan.blocks = blocks;
     plan.part.reserve((size_t)n_sys * (blocks + 1));
-    const int lg = TEAM_THREADS / team_lanes(dim), cols = TEAM_COLS * team_lanes(dim);
+    const int lg = TEAM_THREADS / team_lanes(dim), cols = team_cols(dim) * team_lanes(dim);
     auto cost = [&](int64_t g) { return (int64_t)std::max(1, ((grp[g].len_k >> 2) + cols - 1) / cols); };
     for (int s = 0; s < n_sys; ++s) {
-        const int64_t hi = sys_grp[s + 1];
-        int64_t g = sys_grp[s], total = 0, run = 0;
+        const int64_t hi = sys[s].hi;
+        int64_t g = sys[s].lo, total = 0, run = 0;
         for (int64_t i = g; i < hi; ++i) total += cost(i);
         for (int k = 0; k <= blocks; ++k) {
             const int64_t upto = 2 * (total / blocks * k + total % blocks * k / blocks);
@@ -27,17 +27,30 @@ void make_team_plan(int dim, const std::vector<GroupRec>& grp, const std::vector
     const int n_shares = n_sys * blocks;
     plan.row_ptr.resize(plan.part.size());
     for (size_t i = 0; i < plan.part.size(); ++i) plan.row_ptr[i] = grp[plan.part[i]].row;
+    int64_t sys_rows = 0;
+    for (const SysGroups& s : sys) sys_rows = std::max<int64_t>(sys_rows, grp[s.hi].row - grp[s.lo].row);
+    // a share's window is no smaller than its rows
+    plan.sys_window.assign(n_sys, 0);
+    bool fits = true;
+    for (size_t i = 1; i < plan.row_ptr.size(); ++i)
+        if (i % (blocks + 1) != 0) {
+            int32_t& w = plan.sys_window[i / (blocks + 1)];
+            w = std::max(w, plan.row_ptr[i] - plan.row_ptr[i - 1]);
+            fits = fits && w <= fit_window;
+        }
+    if (!fits) return false;
+    std::vector<int32_t> share_window(n_shares);
     std::vector<std::vector<int32_t>> found(n_shares);
     std::vector<std::vector<StepRec>> steps(n_shares);
     int rows = 0, passes = 0, window = 0;
-#pragma omp parallel reduction(max : rows, passes, window)
+#pragma omp parallel num_threads(std::min(omp_get_max_threads(), 16)) reduction(max : rows, passes, window)
     {
-        // the share that last met each column, per thread
-        std::vector<int32_t> seen((size_t)grp.back().row, -1);
+        // the share that last met each column of its system, per thread
+        std::vector<int32_t> seen((size_t)sys_rows, -1);
 #pragma omp for schedule(dynamic, 4)
         for (int k = 0; k < n_shares; ++k) {
             const int32_t* pt = &plan.part[(size_t)(k / blocks) * (blocks + 1) + k % blocks];
-            const int32_t r0 = grp[pt[0]].row, r1 = grp[pt[1]].row;
+            const int32_t r0 = grp[pt[0]].row, r1 = grp[pt[1]].row, first = grp[sys[k / blocks].lo].row;
             rows = std::max(rows, r1 - r0);
             // longest groups first, each to the lane group with the fewest
             // steps, the next one in order among equals: few passes, and
@@ -68,17 +81,21 @@ void make_team_plan(int dim, const std::vector<GroupRec>& grp, const std::vector
             std::vector<int32_t>& h = found[k];
             for (int32_t g = pt[0]; g < pt[1]; ++g)
                 for (const int32_t *c = colidx + grp[g].begin, *e = c + (grp[g].len_k >> 2); c < e; ++c)
-                    if ((*c < r0 || *c >= r1) && seen[*c] != k) {
-                        seen[*c] = k;
+                    if ((*c < r0 || *c >= r1) && seen[*c - first] != k) {
+                        seen[*c - first] = k;
                         h.push_back(*c);
                     }
             std::sort(h.begin(), h.end());
-            window = std::max(window, (int)(r1 - r0 + h.size()));
+            share_window[k] = r1 - r0 + (int32_t)h.size();
+            window = std::max(window, share_window[k]);
         }
     }
     plan.max_rows = rows;
     plan.max_passes = passes;
     plan.max_window = window;
+    for (int k = 0; k < n_shares; ++k)
+        plan.sys_window[k / blocks] = std::max(plan.sys_window[k / blocks], share_window[k]);
+    if (window > fit_window) return false;
     plan.halo_ptr.assign(n_shares + 1, 0);
     for (int k = 0; k < n_shares; ++k) plan.halo_ptr[k + 1] = plan.halo_ptr[k] + (int64_t)found[k].size();
     plan.step_ptr.assign(n_shares + 1, 0);
@@ -90,6 +107,7 @@ void make_team_plan(int dim, const std::vector<GroupRec>& grp, const std::vector
         std::copy(found[k].begin(), found[k].end(), plan.halo.begin() + plan.halo_ptr[k]);
         std::copy(steps[k].begin(), steps[k].end(), plan.steps.begin() + plan.step_ptr[k] * lg);
     }
+    return true;
 }
 
 }  // namespace pgft

@@ -441,6 +441,232 @@ void enqueue_iteration_g(int G, BArgs& a, hipStream_t st, int maxit) {
     else enqueue_iteration<NR, 16>(a, st, maxit);
 }
 
+// ---------------------------------------------------------------------------
+// The solve on resident teams (pgf_team.hpp): several teams of blocks, each
+// solving one system after the other for all its right-hand sides.
+__global__ void k_bfill_slots(int64_t n, unsigned long long* slots) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) slots[i] = pgft::EMPTY;
+}
+// every team at the start of its list
+__global__ void k_bteam_start(int n_teams, const int32_t* list, int* pos) {
+    for (int t = threadIdx.x; t < n_teams; t += blockDim.x) {
+        pos[2 * t] = list[t];
+        pos[2 * t + 1] = 0;
+    }
+}
+__global__ void k_bfill_zero(int64_t n, int* p) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) p[i] = 0;
+}
+
+template <int NR>
+pgft::TeamShape batch_shape(int dim, const pgft::TeamPlan& p) {
+    return dim == 3 ? pgft::team_shape<double, NR, 3>(p) : pgft::team_shape<double, NR, 2>(p);
+}
+
+// Teams for the batch, kept with the context for calls with the same systems.
+// A team's blocks hold their windows in LDS: as many teams as that allows, 8
+// down to 5, for all systems; if some do not fit even then, those that fit an
+// eighth of the CUs get a launch of their own and the rest at least a quarter,
+// and so on.  (32 RVEs of 64 to 160 divisions, three right-hand sides: 217 ms
+// with three of them in a second launch, BATCHT with all in one; launches with
+// tuned tiles 382 ms.)  Systems are dealt to the teams longest first.  False if
+// some system fits no team.
+template <int NR>
+bool make_batch_teams(pgfd::Ctx& c, const std::vector<int64_t>& sp) {
+    if (!c.batch_teams.empty() && c.batch_nrhs == NR && c.batch_sys == sp) return true;
+    c.batch_teams.clear();
+    const int n_sys = (int)sp.size() - 1, lg = pgft::TEAM_THREADS / pgft::team_lanes(c.dim);
+    std::vector<pgft::SysGroups> grp(n_sys);
+    std::vector<int32_t> left;
+    for (int s = 0; s < n_sys; ++s) {
+        auto at = [&](int64_t row) {
+            return std::lower_bound(c.h_grp.begin(), c.h_grp.end(), row,
+                                    [](const pgft::GroupRec& g, int64_t r) { return g.row < r; });
+        };
+        const auto lo = at(sp[s]), hi = at(sp[s + 1]);
+        if (lo->row != sp[s] || hi->row != sp[s + 1]) return false;  // a row group across two systems
+        grp[s] = {lo - c.h_grp.begin(), hi - c.h_grp.begin()};
+        if (sp[s + 1] > sp[s]) left.push_back(s);
+    }
+    const int64_t fit = pgft::LDS_MAX / (sizeof(double) * NR);
+    std::vector<pgft::Team> teams;
+    uint16_t* wcol = nullptr;
+    // plans teams for the systems `now`, at least the CUs / parts each
+    auto plan = [&](const std::vector<int32_t>& now, int parts, pgft::Team& t) {
+        int64_t most = 1;
+        std::vector<pgft::SysGroups> g;
+        for (int s : now) {
+            g.push_back(grp[s]);
+            most = std::max(most, grp[s].hi - grp[s].lo);
+        }
+        // fewer systems than teams of this size: larger teams, as far as the
+        // rows can use them
+        const int64_t useful = (most + lg - 1) / lg;
+        const int blocks = (int)std::max<int64_t>(
+            1, std::min<int64_t>({std::max(c.n_cu / parts, c.n_cu / (int)now.size()), useful, pgft::MAX_TEAM}));
+        t.sys = now;
+        t.n_teams = std::min(std::max(c.n_cu / blocks, 1), (int)now.size());
+        t.fits = pgft::make_team_plan(c.dim, c.h_grp, g, c.h_colidx.data(), blocks, fit, t.plan) &&
+                 batch_shape<NR>(c.dim, t.plan).kernel != nullptr;
+        return t.fits;
+    };
+    auto take = [&](pgft::Team& t) {
+        std::vector<std::vector<int32_t>> lists(t.n_teams);
+        std::vector<double> load(t.n_teams, 0.0);
+        std::vector<int32_t> order(t.sys.size());
+        for (size_t i = 0; i < order.size(); ++i) order[i] = (int32_t)i;
+        // iterations grow with the mesh's divisions; one takes about as long
+        // as 750 rows a block, plus its rows
+        auto cost = [&](int32_t i) {
+            const double rows = (double)(sp[t.sys[i] + 1] - sp[t.sys[i]]);
+            return std::pow(rows, c.dim == 3 ? 1.0 / 3.0 : 0.5) * (rows + 750.0 * t.plan.blocks);
+        };
+        std::stable_sort(order.begin(), order.end(), [&](int32_t a, int32_t b) { return cost(a) > cost(b); });
+        for (int32_t i : order) {
+            const int k = (int)(std::min_element(load.begin(), load.end()) - load.begin());
+            lists[k].push_back(i);
+            load[k] += cost(i);
+        }
+        BCHK(t.upload(lists, c.grp, c.colidx, c.nnz, wcol, c.stream));
+        wcol = t.wcol;
+        std::vector<int32_t> rest;
+        for (int s : left)
+            if (!std::binary_search(t.sys.begin(), t.sys.end(), s)) rest.push_back(s);
+        left.swap(rest);
+        teams.push_back(std::move(t));
+    };
+    static const std::vector<int> stages[] = {{8, 7, 6, 5}, {4, 3}, {2}, {1}};
+    for (const std::vector<int>& stage : stages) {
+        if (left.empty()) break;
+        std::vector<int32_t> small;  // systems that fit the stage's smallest team
+        for (size_t i = 0; i < stage.size() && !left.empty(); ++i) {
+            pgft::Team t;
+            if (plan(left, stage[i], t)) take(t);
+            else if (i == 0)
+                for (size_t k = 0; k < left.size(); ++k)
+                    if (t.plan.sys_window[k] * 4ll / 3 <= fit) small.push_back(left[k]);
+        }
+        if (left.empty() || small.empty()) continue;
+        pgft::Team t;
+        if (plan(small, stage[0], t)) take(t);
+    }
+    if (!left.empty()) return false;
+    c.batch_teams = std::move(teams);
+    c.batch_sys = sp;
+    c.batch_nrhs = NR;
+    return true;
+}
+
+// Device memory of one solve: kept with the context up to KEEP_BYTES, else of
+// the call.
+struct BatchWork {
+    static constexpr int64_t KEEP_BYTES = 256ll << 20;
+    double *p = nullptr, *own = nullptr;
+    BatchWork(pgfd::Ctx& c, int64_t doubles) {
+        if (doubles * (int64_t)sizeof(double) <= KEEP_BYTES) p = c.workspace(doubles);
+        else p = own = balloc<double>((size_t)doubles);
+    }
+    ~BatchWork() {
+        if (own) (void)hipFree(own);
+    }
+};
+
+// Iterations of a team per launch: the host waits that often.
+constexpr int BATCH_ITS = 4096;
+
+// The whole batch; false (nothing done) if it fits no teams or the device
+// gives no cooperative launch.
+template <int NR>
+bool run_teams(pgfd::Ctx& c, const std::vector<int64_t>& sp, const double* b, double* x, double rtol, int maxit,
+               int32_t* iters, double* relres, double* ms_out, int* rc) {
+    const int n_sys = (int)sp.size() - 1;
+    const int64_t nf = c.n_free, nv = nf * NR;
+    if (nf == 0 || nv * (int64_t)sizeof(double2) > 0xffffffffll || !make_batch_teams<NR>(c, sp)) return false;
+    // x, r [NR][n] (r first holds b) | (z, p) pairs | 1/diag | states
+    BatchWork work(c, 4 * nv + nf + (int64_t)n_sys * NR * pgft::T_N);
+    double *dx = work.p, *dr = dx + nv, *dz = dr + nv, *dd = dz + 2 * nv, *state = dd + nf;
+    BCHK(hipMemcpyAsync(dr, b, sizeof(double) * nv, hipMemcpyHostToDevice, c.stream));
+    struct Events {
+        hipEvent_t e[2] = {nullptr, nullptr};
+        ~Events() {
+            for (hipEvent_t v : e)
+                if (v) (void)hipEventDestroy(v);
+        }
+    } ev;
+    for (hipEvent_t& e : ev.e) BCHK(hipEventCreate(&e));
+    BCHK(hipEventRecord(ev.e[0], c.stream));
+    std::vector<double> st((size_t)n_sys * NR * pgft::T_N, 0.0);
+    int64_t base = 0;  // states of the teams before
+    for (size_t k = 0; k < c.batch_teams.size(); ++k) {
+        const pgft::Team& t = c.batch_teams[k];
+        const pgft::TeamShape shape = batch_shape<NR>(c.dim, t.plan);
+        if (shape.lds > 65536u)
+            BCHK(hipFuncSetAttribute(shape.kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shape.lds));
+        pgft::TeamArgs<double> a{};
+        t.args(a);
+        a.diag = c.diag;
+        a.A = c.K;
+        a.ld = nf;
+        a.b = dr;
+        a.x = dx; a.r = dr; a.dinv = dd;
+        a.zp = (double2*)dz;
+        a.zp_bytes = nv * (int64_t)sizeof(double2);
+        a.state = state + base;
+        a.tol2 = rtol * rtol;
+        a.maxit = maxit;
+        a.launch_its = BATCH_ITS;
+        a.single = 0;
+        void* args[] = {(void*)&a};
+        std::vector<int> pos(2 * (size_t)t.n_teams + 1);
+        std::vector<int32_t> ends(t.n_teams + 1);
+        hipLaunchKernelGGL(k_bfill_zero, dim3((unsigned)(pos.size() + 255) / 256), dim3(256), 0, c.stream, (int64_t)pos.size(),
+                           t.pos);
+        hipLaunchKernelGGL(k_bteam_start, dim3(1), dim3(256), 0, c.stream, t.n_teams, (const int32_t*)t.list, t.pos);
+        BCHK(hipMemcpyAsync(ends.data(), t.list, sizeof(int32_t) * ends.size(), hipMemcpyDeviceToHost, c.stream));
+        for (bool running = true, first = true; running; first = false) {
+            hipLaunchKernelGGL(k_bfill_slots, dim3((unsigned)((t.n_slots() + 255) / 256)), dim3(256), 0, c.stream, t.n_slots(),
+                               t.slots);
+            const hipError_t e = hipLaunchCooperativeKernel(shape.kernel, dim3((unsigned)(t.n_teams * t.plan.blocks)),
+                                                            dim3(pgft::TT), args, shape.lds, c.stream);
+            if (k == 0 && first && (e == hipErrorIllegalState || e == hipErrorCooperativeLaunchTooLarge)) {
+                (void)hipGetLastError();
+                return false;
+            }
+            BCHK(e);
+            BCHK(hipMemcpyAsync(pos.data(), t.pos, sizeof(int) * pos.size(), hipMemcpyDeviceToHost, c.stream));
+            BCHK(hipStreamSynchronize(c.stream));
+            if (pos.back()) throw std::string("HIP error: the resident blocks lost each other");
+            running = false;
+            for (int i = 0; i < t.n_teams; ++i) running = running || pos[2 * i] < ends[i + 1];
+        }
+        base += (int64_t)t.sys.size() * NR * pgft::T_N;
+    }
+    BCHK(hipEventRecord(ev.e[1], c.stream));
+    BCHK(hipMemcpyAsync(x, dx, sizeof(double) * nv, hipMemcpyDeviceToHost, c.stream));
+    BCHK(hipMemcpyAsync(st.data(), state, sizeof(double) * base, hipMemcpyDeviceToHost, c.stream));
+    BCHK(hipStreamSynchronize(c.stream));
+    float ms;
+    BCHK(hipEventElapsedTime(&ms, ev.e[0], ev.e[1]));
+    if (ms_out) *ms_out = ms;
+    bool all = true;
+    for (int i = 0; i < n_sys * NR; ++i) {
+        if (iters) iters[i] = 0;
+        if (relres) relres[i] = 0.0;
+    }
+    const double* s = st.data();
+    for (const pgft::Team& t : c.batch_teams)
+        for (int32_t sys : t.sys)
+            for (int r = 0; r < NR; ++r, s += pgft::T_N) {
+                if (iters) iters[sys * NR + r] = (int32_t)s[pgft::T_IT];
+                if (relres) relres[sys * NR + r] = s[pgft::T_RR0] > 0 ? std::sqrt(s[pgft::T_RR] / s[pgft::T_RR0]) : 0.0;
+                all = all && s[pgft::T_RR] <= s[pgft::T_TOL];
+            }
+    *rc = all ? 0 : PGF_ENOTCONVERGED;
+    return true;
+}
+
 constexpr int64_t PERSIST_MAX_TILES = 256;
 
 template <int NR>
@@ -456,6 +682,13 @@ int run_batch(pgfd::Ctx& c, const std::vector<int64_t>& sys_ptr, const double* b
               bool persistent) {
     const int n_sys = (int)sys_ptr.size() - 1;
     const int64_t nf = c.n_free;
+    if (!persistent && !(G_req > 0 && rows_req > 0)) {
+        int rc = 0;
+        if (run_teams<NR>(c, sys_ptr, b, x, rtol, maxit, iters, relres, ms_out, &rc)) {
+            if (tuned) tuned[0] = tuned[1] = 0;
+            return rc;
+        }
+    }
     // autotuner candidates: (threads per row, rows per tile)
     std::vector<std::pair<int, int>> cand;
     if (G_req > 0 && rows_req > 0) cand.push_back({G_req, rows_req});
@@ -736,12 +969,21 @@ static int batch_pcg(pgf_ctx* h, int32_t n_sys, const int64_t* sys_ptr, int32_t 
         for (int s = 0; s < n_sys; ++s)
             if (sp[s + 1] < sp[s]) throw std::string("system ranges must be ascending");
         // the free-free block must be block diagonal over these ranges
-        int s = 0;
-        for (int64_t r = 0; r < c->n_free; ++r) {
-            while (r >= sp[s + 1]) ++s;
-            for (int64_t j = c->h_rowptr[r]; j < c->h_rowptr[r] + c->h_rowsplit[r]; ++j)
-                if (c->h_colidx[j] < sp[s] || c->h_colidx[j] >= sp[s + 1])
-                    throw std::string("K_ff couples two systems: not block diagonal over the given ranges");
+        // (the rows of a group have one column list; ranges that the context
+        // laid its teams out for were found block diagonal then)
+        if (c->batch_sys != sp) {
+            int s = 0;
+            for (int64_t g = 0; g < c->n_grp; ++g) {
+                const pgft::GroupRec& gr = c->h_grp[g];
+                for (int k = 0; k < (gr.len_k & 3); ++k) {
+                    while (gr.row + k >= sp[s + 1]) ++s;
+                    for (int32_t j = gr.begin; j < gr.begin + (gr.len_k >> 2); ++j)
+                        if (c->h_colidx[j] < sp[s] || c->h_colidx[j] >= sp[s + 1])
+                            throw std::string("K_ff couples two systems: not block diagonal over the given ranges");
+                    // (further rows of the group need it only in another system)
+                    while (k + 1 < (gr.len_k & 3) && gr.row + k + 1 < sp[s + 1]) ++k;
+                }
+            }
         }
         const int Greq = tune ? tune[0] : 0, Rreq = tune ? tune[1] : 0;
         if (Greq && Greq != 4 && Greq != 8 && Greq != 16) throw std::string("threads per row must be 4, 8 or 16");

@@ -112,8 +112,7 @@ Ctx::~Ctx() {
                     ce_off_ptr, vpt_w, vpt_grad, cpt_w, cpt_N, cpt_R, vpt_mat, cpt_law, cpt_nodes, cpt_nh, ce_off, laws,
                     dmax_conv, dmax_trial, flags, free_slot, rowptr, rowsplit, colidx, K, K32, P, Fext_full,
                     upres_full, r, x, zp, q, dinv, guess, res, partial,
-                    scal, counter, grp, diag, team_row_ptr, team_step_ptr, team_steps, team_list, team_halo,
-                    team_halo_ptr, team_wcol, team_pos, team_slots, el_conn, cut_index, inc_elem, el_mat, inc_slot, inc_ptr, ke_ptr, pe_ptr,
+                    scal, counter, grp, diag, el_conn, cut_index, inc_elem, el_mat, inc_slot, inc_ptr, ke_ptr, pe_ptr,
                     inc_rel, ke, pe, blk_node, blk_seg, blk_rounds,  ce_rel, ce_rel_ptr, image,
                     sens_dgrad, sens_divv, sens_pe, sens_ds, sens_param, inc_rec, el_conn4, Xq};
     for (void* p : ptrs)
@@ -539,7 +538,7 @@ template <typename TA>
 static void pcg_launches(Ctx& c, const TA* A, const double* b, bool x0, double rtol, int maxit) {
     const int64_t n = c.n_free;
     double *z = (double*)c.zp, *p = z + n;
-    int* done = c.team_pos;
+    int* done = (int*)(c.scal + S_NSCAL + 4);
     hipLaunchKernelGGL(k_diag_inv<TA>, dim3(grid_for(n)), dim3(256), 0, c.stream, n, (const int32_t*)c.diag, A, c.dinv);
     if (!x0) fill_async<double>(c, c.x, n, 0.0);
     hipLaunchKernelGGL(k_cg_init, dim3(grid_for(n)), dim3(256), 0, c.stream, n, b, c.r, z, p,
@@ -589,43 +588,33 @@ constexpr int TEAM_ITS = 2048;
 
 template <typename TA>
 static bool pcg_team(Ctx& c, const TA* A, const double* b, bool x0, double rtol, int maxit) {
-    const pgft::TeamShape shape = c.dim == 3 ? pgft::team_shape<TA, 1, 3>(c.team) : pgft::team_shape<TA, 1, 2>(c.team);
-    if (!shape.kernel) return false;
+    if (!c.team.fits) return false;
+    const pgft::TeamShape shape =
+        c.dim == 3 ? pgft::team_shape<TA, 1, 3>(c.team.plan) : pgft::team_shape<TA, 1, 2>(c.team.plan);
     if (shape.lds > 65536u)
         HIPCHK(hipFuncSetAttribute(shape.kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shape.lds));
     pgft::TeamArgs<TA> a{};
-    a.n_teams = 1;
-    a.team_blocks = c.team.blocks;
-    a.team_sys = c.team_list;
-    a.sys_list = c.team_list;
-    a.team_pos = c.team_pos;
-    a.row_ptr = c.team_row_ptr;
-    a.step_ptr = c.team_step_ptr;
-    a.steps = c.team_steps;
-    a.wcol = c.team_wcol;
-    a.halo_ptr = c.team_halo_ptr;
-    a.halo = c.team_halo;
+    c.team.args(a);
     a.diag = c.diag;
     a.A = A;
+    a.ld = c.n_free;
     a.b = b;
     a.Ax = x0 ? c.q : nullptr;
     a.x = c.x; a.r = c.r; a.dinv = c.dinv; a.zp = c.zp;
     a.zp_bytes = c.n_free * (int64_t)sizeof(double2);
     a.state = c.scal;
-    a.slots = c.team_slots;
-    a.abort = c.team_pos + 2;
     a.tol2 = rtol * rtol;
     a.maxit = maxit;
     a.launch_its = TEAM_ITS;
     a.single = 1;
     void* args[] = {(void*)&a};
-    const int64_t n_slots = pgft::COPIES * pgft::team_slots(c.team.blocks);
+    const int64_t n_slots = c.team.n_slots();
     Progress progress;
-    hipLaunchKernelGGL(k_fill<int>, dim3(1), dim3(64), 0, c.stream, c.team_pos, (int64_t)3, 0);
+    hipLaunchKernelGGL(k_fill<int>, dim3(1), dim3(64), 0, c.stream, c.team.pos, (int64_t)3, 0);
     for (bool first = true;; first = false) {
         hipLaunchKernelGGL(k_fill<unsigned long long>, dim3((unsigned)((n_slots + 255) / 256)), dim3(256), 0, c.stream,
-                           c.team_slots, n_slots, pgft::EMPTY);
-        const hipError_t e = hipLaunchCooperativeKernel(shape.kernel, dim3((unsigned)c.team.blocks), dim3(pgft::TT), args,
+                           c.team.slots, n_slots, pgft::EMPTY);
+        const hipError_t e = hipLaunchCooperativeKernel(shape.kernel, dim3((unsigned)c.team.plan.blocks), dim3(pgft::TT), args,
                                                         shape.lds, c.stream);
         if (first && (e == hipErrorIllegalState || e == hipErrorCooperativeLaunchTooLarge)) {
             (void)hipGetLastError();
@@ -633,7 +622,7 @@ static bool pcg_team(Ctx& c, const TA* A, const double* b, bool x0, double rtol,
         }
         HIPCHK(e);
         HIPCHK(hipMemcpyAsync(c.h_scal, c.scal, sizeof(double) * pgft::T_N, hipMemcpyDeviceToHost, c.stream));
-        HIPCHK(hipMemcpyAsync(c.h_scal + pgft::T_N, c.team_pos, sizeof(int) * 3, hipMemcpyDeviceToHost, c.stream));
+        HIPCHK(hipMemcpyAsync(c.h_scal + pgft::T_N, c.team.pos, sizeof(int) * 3, hipMemcpyDeviceToHost, c.stream));
         HIPCHK(hipStreamSynchronize(c.stream));
         int pos[3];
         std::memcpy(pos, c.h_scal + pgft::T_N, sizeof(pos));
@@ -1066,8 +1055,9 @@ PGF_API int pgf_create(const pgf_mesh_desc* d, pgf_ctx** out) {
             grp.reserve(c->n_free / c->dim + 2);
             for (int64_t r = 0; r < c->n_free; ++r) {
                 const auto lo = pat.colidx.begin() + pat.rowptr[r], hi = lo + pat.rowsplit[r];
-                const auto d = std::lower_bound(lo, hi, (int32_t)r);
-                diag[r] = d != hi && *d == r ? (int32_t)(d - pat.colidx.begin()) : -1;
+                auto d = std::lower_bound(lo, hi, (int32_t)r);
+                if (d == hi || *d != r) d = std::find(lo, hi, (int32_t)r);  // columns follow the nodes, not the dof ids
+                diag[r] = d != hi ? (int32_t)(d - pat.colidx.begin()) : -1;
                 if (!grp.empty() && pat.rowsplit[r] > 0) {
                     pgft::GroupRec& g = grp.back();
                     if ((g.len_k & 3) < c->dim && g.len_k >> 2 == pat.rowsplit[r] &&
@@ -1088,29 +1078,15 @@ PGF_API int pgf_create(const pgf_mesh_desc* d, pgf_ctx** out) {
             int dev = 0;
             HIPCHK(hipGetDevice(&dev));
             HIPCHK(hipDeviceGetAttribute(&c->n_cu, hipDeviceAttributeMultiprocessorCount, dev));
-            const int64_t lanes = c->n_grp * (c->dim == 3 ? 16 : 8);
+            const int64_t lanes = c->n_grp * pgft::team_lanes(c->dim);
             const int blocks = (int)std::max<int64_t>(1, std::min<int64_t>({(lanes + pgft::TT - 1) / pgft::TT, c->n_cu, pgft::MAX_TEAM}));
-            pgft::make_team_plan(c->dim, grp, {0, c->n_grp}, pat.colidx.data(), blocks, c->team);
-            c->team_row_ptr = pgfd::dupload(c->team.row_ptr.data(), (int64_t)c->team.row_ptr.size());
-            c->team_step_ptr = pgfd::dupload(c->team.step_ptr.data(), (int64_t)c->team.step_ptr.size());
-            c->team_steps = pgfd::dupload(c->team.steps.data(), (int64_t)c->team.steps.size());
-            c->team_halo_ptr = pgfd::dupload(c->team.halo_ptr.data(), (int64_t)c->team.halo_ptr.size());
-            c->team_halo = pgfd::dupload(c->team.halo.data(), (int64_t)c->team.halo.size());
-            const int32_t list[2] = {0, 1};  // the one team's range of systems, and its one system
-            c->team_list = pgfd::dupload(list, 2);
-            c->team_pos = pgfd::dalloc<int>(3);
-            c->team_slots = pgfd::dalloc<unsigned long long>(pgft::COPIES * pgft::team_slots(blocks));
+            c->team.sys = {0};
+            c->team.fits = pgft::make_team_plan(c->dim, grp, {{0, c->n_grp}}, pat.colidx.data(), blocks,
+                                                pgft::LDS_MAX / sizeof(double), c->team.plan) &&
+                           pgft::team_shape<double, 1, 2>(c->team.plan).kernel != nullptr;
         }
         c->colidx = pgfd::dupload(pat.colidx.data(), c->nnz);
-        if (c->team.max_window <= pgft::MAX_WINDOW && sizeof(double) * (size_t)c->team.max_window <= pgft::LDS_MAX) {
-            c->team_wcol = pgfd::dalloc<uint16_t>(c->nnz);
-            int32_t* part = pgfd::dupload(c->team.part.data(), (int64_t)c->team.part.size());
-            hipLaunchKernelGGL(pgft::k_team_cols, dim3((unsigned)c->team.blocks), dim3(256), 0, c->stream, c->team.blocks,
-                               c->team.blocks, part, c->grp, c->colidx, c->team_halo_ptr, c->team_halo, c->team_wcol);
-            HIPCHK(hipGetLastError());
-            HIPCHK(hipStreamSynchronize(c->stream));
-            HIPCHK(hipFree(part));
-        }
+        if (c->team.fits) HIPCHK(c->team.upload({{0}}, c->grp, c->colidx, c->nnz, nullptr, c->stream));
         c->K = pgfd::dalloc<double>(c->nnz);
         c->K32 = pgfd::dalloc<float>(c->nnz);
         c->P = pgfd::dalloc<double>(c->n_rows);

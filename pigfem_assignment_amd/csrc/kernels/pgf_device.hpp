@@ -86,13 +86,13 @@ struct Ctx {
     // PCG team of this system (pgf_team.hpp)
     std::vector<pgft::GroupRec> h_grp;  // [n_grp + 1] host copy (shares of a batch)
     pgft::GroupRec* grp = nullptr;
-    pgft::TeamPlan team;
-    int32_t *diag = nullptr, *team_row_ptr = nullptr, *team_list = nullptr, *team_halo = nullptr;
-    int64_t *team_halo_ptr = nullptr, *team_step_ptr = nullptr;
-    pgft::StepRec* team_steps = nullptr;
-    uint16_t* team_wcol = nullptr;
-    int* team_pos = nullptr;
-    unsigned long long* team_slots = nullptr;
+    int32_t* diag = nullptr;       // entry of each free row's diagonal, -1 without one
+    pgft::Team team;               // of K_ff as one system
+    // teams of the last batched solve with automatic choice, by its systems
+    // and right-hand sides
+    std::vector<pgft::Team> batch_teams;
+    std::vector<int64_t> batch_sys;
+    int batch_nrhs = 0;
     int n_cu = 0;
     double* partial = nullptr;     // block partial sums
     double* scal = nullptr;        // device scalars: PCG state (pgft::T_N), residual norm

@@ -30,8 +30,8 @@
 //    acquire fence of the agent instead, which write back and drop the die's
 //    whole L2, take 4.5 us with 32 blocks per die, and K leaves the L2.
 //  * K entries and window indices of a block stay in registers where they all
-//    fit (KEEP steps a lane); otherwise they are streamed, the loads two steps
-//    ahead of the products.
+//    fit (KEEP steps a lane); otherwise they are streamed, the loads one
+//    or two steps ahead of the products.
 //  * the steps of a block's lane groups are laid out on the host: rows longer
 //    than a step take consecutive steps of one lane group, so no lane waits in
 //    a loop over a neighbour's long row, and every block has about as many.
@@ -45,6 +45,7 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <utility>
 #include <vector>
 
 #include "../host/pgf_team.hpp"
@@ -55,7 +56,7 @@ constexpr int TT = TEAM_THREADS;                  // 512: 256 registers a lane f
 constexpr int MAX_TEAM = 256;                     // blocks per team (four slots per lane of the reading wavefront)
 constexpr unsigned long long EMPTY = ~0ull;       // slot not yet published
 constexpr unsigned long long WAIT_TICKS = 2000000000ull;  // 20 s of the 100 MHz wall clock
-constexpr size_t LDS_MAX = 156 * 1024;            // dynamic LDS a block may take (of 160 KiB)
+constexpr size_t LDS_MAX = 158 * 1024;            // dynamic LDS a block may take (160 KiB less the static part)
 constexpr int MAX_WINDOW = 65536;                 // 16-bit window indices
 
 // per (system, right-hand side) state between launches and result
@@ -79,12 +80,13 @@ struct TeamArgs {
     const int32_t* halo;      // columns of each block's halo
     const int32_t* diag;      // entry of each row's diagonal, -1 without one
     const TA* A;
-    const double* b;          // [n][NR]
+    int64_t ld;               // stride of the right-hand sides in b, x, r and zp
+    const double* b;          // [NR][ld]
     const double* Ax;         // K x0 for a nonzero start (x then holds x0), or null
-    double *x, *r, *dinv;     // [n][NR] ([n] for dinv)
-    double2* zp;              // [n][NR] published (z, p)
+    double *x, *r, *dinv;     // [NR][ld] ([n] for dinv)
+    double2* zp;              // [NR][ld] published (z, p): a wavefront stores whole lines
     int64_t zp_bytes;
-    double* state;            // [n_sys][NR][T_N]
+    double* state;            // [n_sys][NR][T_N], systems in the order of their shares
     unsigned long long* slots;  // [n_teams][COPIES][team_slots]
     int* abort;
     double tol2;              // squared relative tolerance
@@ -141,8 +143,8 @@ template <int G>
 __device__ inline double lane_sum(double v) {
     v += dpp<0xB1>(v);
     v += dpp<0x4E>(v);
-    v += dpp<0x141>(v);
-    if (G == 16) v += dpp<0x140>(v);
+    if (G >= 8) v += dpp<0x141>(v);
+    if (G >= 16) v += dpp<0x140>(v);
     return v;
 }
 __device__ inline double wave_sum(double v) {
@@ -259,10 +261,14 @@ struct TeamSum {
 };
 
 // One step of a lane group: U columns per lane (window indices in pairs), their
-// entries in the group's rows.
-constexpr int U = TEAM_COLS;
+// entries in the group's rows.  The sums over the lanes are most of a product's
+// instructions and cost lanes times steps, so a 2D group has 4 lanes with 5
+// columns each, not 8 with 3 (333 x 333 quads: products 2.1 -> 1.2 us, 10.4 ->
+// 9.2 us per iteration).  In 3D 16 lanes with 3 columns stay: 8 with 6 take 111
+// us on 64^3 x 6 tets against 97 (coarser steps to stream and to balance).
 template <typename TA, int DIM>
 struct Step {
+    static constexpr int U = team_cols(DIM);
     uint32_t c[(U + 1) / 2];
     TA v[DIM][U];
     __device__ int col(int u) const { return (int)(u & 1 ? c[u / 2] >> 16 : c[u / 2] & 0xffffu); }
@@ -270,7 +276,7 @@ struct Step {
 
 template <typename TA, int NR, int DIM, int TIER, int KEEP>
 __global__ __launch_bounds__(TT) void k_team_pcg(TeamArgs<TA> a) {
-    constexpr int G = team_lanes(DIM), GP = TT / G;
+    constexpr int G = team_lanes(DIM), GP = TT / G, U = team_cols(DIM);
     constexpr bool ALL = TIER == WIN_ALL;
     constexpr int RB = ALL ? 1 : 4;  // rows per trip: operands in memory want several on the way
     constexpr int W = slot_values<NR>();
@@ -308,16 +314,16 @@ __global__ __launch_bounds__(TT) void k_team_pcg(TeamArgs<TA> a) {
         double* Lq = Lp + (size_t)nw * NR;
         double* Lr = Lq + (size_t)nrow * NR;
         double* Ld = Lr + (size_t)nrow * NR;
-        double* xg = a.x + (size_t)row0 * NR;
-        double* rg = a.r + (size_t)row0 * NR;
-        double2* zg = a.zp + (size_t)row0 * NR;
+        double* xg = a.x + row0;
+        double* rg = a.r + row0;
+        const double2* zg = a.zp + row0;
         const double* dg = a.dinv + row0;
         double* st = a.state + (size_t)sys * NR * T_N;
         double rz[NR], beta[NR], rr[NR], rr0[NR], tol[NR];
         bool act[NR];
         int it[NR];
         auto store_pair = [&](int i, int c, double z, double p) {
-            pair_store(zrs, (uint32_t)(row0 + i) * NR + c, double2{z, p});
+            pair_store(zrs, (uint32_t)(c * a.ld + row0 + i), double2{z, p});
         };
         // (unconditional loads at clamped places, zeroed afterwards: a load
         // under a condition is a branch the next one waits behind)
@@ -346,9 +352,9 @@ __global__ __launch_bounds__(TT) void k_team_pcg(TeamArgs<TA> a) {
             for (int i = t; i < nrow; i += TT) {
                 if (ALL) Ld[i] = dg[i];
                 for (int c = 0; c < NR; ++c) {
-                    if (ALL) Lr[c * nrow + i] = rg[i * NR + c];
-                    Lp[c * nw + i] = zg[i * NR + c].y;
-                    Lq[c * nrow + i] = zg[i * NR + c].x;
+                    if (ALL) Lr[c * nrow + i] = rg[c * a.ld + i];
+                    Lp[c * nw + i] = zg[c * a.ld + i].y;
+                    Lq[c * nrow + i] = zg[c * a.ld + i].x;
                 }
             }
             for (int c = 0; c < NR; ++c) {
@@ -370,7 +376,7 @@ __global__ __launch_bounds__(TT) void k_team_pcg(TeamArgs<TA> a) {
                 a.dinv[row0 + i] = di;
                 if (ALL) Ld[i] = di;
                 for (int c = 0; c < NR; ++c) {
-                    const int64_t e = (int64_t)(row0 + i) * NR + c;
+                    const int64_t e = c * a.ld + row0 + i;
                     const double bi = a.b[e], ri = a.Ax ? bi - a.Ax[e] : bi;
                     const double zi = di * ri;
                     if (!a.Ax) a.x[e] = 0.0;
@@ -398,8 +404,10 @@ __global__ __launch_bounds__(TT) void k_team_pcg(TeamArgs<TA> a) {
         }
         bool any = false;
         for (int c = 0; c < NR; ++c) any = any || act[c];
-        // K entries that stay in registers: every step (KEEP), or the first two
-        constexpr int NK = KEEP > 0 ? KEEP : 2;
+        // K entries that stay in registers: every step (KEEP), or the first
+        // AHEAD
+        constexpr int AHEAD = DIM == 3 ? 2 : 1;  // steps on the way while streaming
+        constexpr int NK = KEEP > 0 ? KEEP : AHEAD;
         Step<TA, DIM> keep[NK];
         int info[NK];
 #pragma unroll
@@ -409,8 +417,8 @@ __global__ __launch_bounds__(TT) void k_team_pcg(TeamArgs<TA> a) {
             info[s] = info_of(r);
             load_step(r, keep[s]);
         }
-        StepRec rec2 = {0, 0, 0, 0};
-        if (KEEP == 0 && ns > 2) rec2 = steps[2 * GP];
+        StepRec rec1 = {0, 0, 0, 0};
+        if (KEEP == 0 && ns > AHEAD) rec1 = steps[AHEAD * GP];
         while (any && left > 0) {
             // ---- p of the window
             // (every loop over rows or columns issues the loads of several
@@ -424,7 +432,7 @@ __global__ __launch_bounds__(TT) void k_team_pcg(TeamArgs<TA> a) {
 #pragma unroll
                 for (int k = 0; k < HB; ++k)
 #pragma unroll
-                    for (int c = 0; c < NR; ++c) e[k][c] = pair_load(zrs, col[k] * NR + c);
+                    for (int c = 0; c < NR; ++c) e[k][c] = pair_load(zrs, (uint32_t)(c * a.ld) + col[k]);
 #pragma unroll
                 for (int k = 0; k < HB; ++k)
                     if (i0 + k * TT < nh)
@@ -486,21 +494,27 @@ __global__ __launch_bounds__(TT) void k_team_pcg(TeamArgs<TA> a) {
                         step(keep[s], info[s]);
                     }
             } else {
-                // three steps' entries in registers: one in use, two on the way
-                Step<TA, DIM> cur = keep[0], nxt = keep[1], far;
-                int ci = info[0], ni = info[1], fi = 0;
-                StepRec rf = rec2;
+                // one step's entries in use, AHEAD steps' on the way
+                Step<TA, DIM> cur[AHEAD + 1];
+                int ci[AHEAD + 1];
+#pragma unroll
+                for (int k = 0; k < AHEAD; ++k) {
+                    cur[k] = keep[k];
+                    ci[k] = info[k];
+                }
+                StepRec rn = rec1;
                 for (int s = 0; s < ns; ++s) {
-                    if (s + 2 < ns) {
-                        fi = info_of(rf);
-                        load_step(rf, far);
-                        if (s + 3 < ns) rf = steps[(size_t)(s + 3) * GP];
+                    if (s + AHEAD < ns) {
+                        ci[AHEAD] = info_of(rn);
+                        load_step(rn, cur[AHEAD]);
+                        if (s + AHEAD + 1 < ns) rn = steps[(size_t)(s + AHEAD + 1) * GP];
                     }
-                    step(cur, ci);
-                    cur = nxt;
-                    nxt = far;
-                    ci = ni;
-                    ni = fi;
+                    step(cur[0], ci[0]);
+#pragma unroll
+                    for (int k = 0; k < AHEAD; ++k) {
+                        cur[k] = cur[k + 1];
+                        ci[k] = ci[k + 1];
+                    }
                 }
             }
             if (!sum(pq, false, [] {})) return;
@@ -520,7 +534,7 @@ __global__ __launch_bounds__(TT) void k_team_pcg(TeamArgs<TA> a) {
                     di[k] = ALL ? Ld[i] : dg[i];
 #pragma unroll
                     for (int c = 0; c < NR; ++c) {
-                        ri[k][c] = ALL ? Lr[c * nrow + i] : rg[(size_t)i * NR + c];
+                        ri[k][c] = ALL ? Lr[c * nrow + i] : rg[c * a.ld + i];
                         qi[k][c] = Lq[c * nrow + i];
                         pi[k][c] = Lp[c * nw + i];
                     }
@@ -535,7 +549,7 @@ __global__ __launch_bounds__(TT) void k_team_pcg(TeamArgs<TA> a) {
                         const double rn = ri[k][c] - alpha[c] * qi[k][c];
                         const double zi = di[k] * rn;
                         if (ALL) Lr[c * nrow + i] = rn;
-                        else rg[(size_t)i * NR + c] = rn;
+                        else rg[c * a.ld + i] = rn;
                         store_pair(i, c, zi, pi[k][c]);
                         Lq[c * nrow + i] = zi;
                         v[c] += rn * zi;
@@ -551,7 +565,7 @@ __global__ __launch_bounds__(TT) void k_team_pcg(TeamArgs<TA> a) {
 #pragma unroll
                     for (int k = 0; k < XB; ++k)
 #pragma unroll
-                        for (int c = 0; c < NR; ++c) xo[k][c] = xg[(size_t)min(i0 + k * XT, nrow - 1) * NR + c];
+                        for (int c = 0; c < NR; ++c) xo[k][c] = xg[c * a.ld + min(i0 + k * XT, nrow - 1)];
 #pragma unroll
                     for (int k = 0; k < XB; ++k) {
                         const int i = i0 + k * XT;
@@ -559,7 +573,7 @@ __global__ __launch_bounds__(TT) void k_team_pcg(TeamArgs<TA> a) {
 #pragma unroll
                         for (int c = 0; c < NR; ++c)
                             if (act[c])
-                                xg[(size_t)i * NR + c] =
+                                xg[c * a.ld + i] =
                                     xo[k][c] + alpha[c] * Lp[c * nw + i];
                     }
                 }
@@ -582,7 +596,7 @@ __global__ __launch_bounds__(TT) void k_team_pcg(TeamArgs<TA> a) {
         }
         if (any && ALL)  // to be resumed
             for (int i = t; i < nrow; i += TT)
-                for (int c = 0; c < NR; ++c) rg[i * NR + c] = Lr[c * nrow + i];
+                for (int c = 0; c < NR; ++c) rg[c * a.ld + i] = Lr[c * nrow + i];
         if (me == 0 && t == 0)
             for (int c = 0; c < NR; ++c) {
                 st[c * T_N + T_RZ] = rz[c];
@@ -639,8 +653,106 @@ static __global__ __launch_bounds__(256) void k_team_cols(int n_shares, int team
 // Passes a lane can keep in its registers.
 template <typename TA, int NR, int DIM>
 constexpr int max_keep() {
-    return sizeof(TA) == 8 ? (DIM == 3 ? 7 : (NR == 1 ? 10 : 8)) : (DIM == 3 ? 12 : 16);
+    return sizeof(TA) == 8 ? (DIM == 3 ? (NR < 3 ? 7 : 5) : (NR == 1 ? 6 : NR == 2 ? 5 : 4)) : (DIM == 3 ? 12 : 10);
 }
+
+// Teams laid out for some systems of a context: the host plan and its device
+// arrays (freed with it).
+struct Team {
+    TeamPlan plan;
+    int n_teams = 0;
+    bool fits = false;               // there is a kernel for the plan
+    std::vector<int32_t> sys;        // the systems, in the order of the plan's shares
+    int32_t *row_ptr = nullptr, *list = nullptr, *halo = nullptr;
+    int64_t *halo_ptr = nullptr, *step_ptr = nullptr;
+    StepRec* steps = nullptr;
+    uint16_t* wcol = nullptr;        // by matrix entry; a batch's teams share one array
+    bool own_wcol = false;
+    int* pos = nullptr;              // [n_teams][2], then the abort flag
+    unsigned long long* slots = nullptr;
+    Team() = default;
+    Team(Team&& o) noexcept { *this = std::move(o); }
+    Team& operator=(Team&& o) noexcept {
+        std::swap(plan, o.plan);
+        std::swap(n_teams, o.n_teams);
+        std::swap(fits, o.fits);
+        std::swap(sys, o.sys);
+        std::swap(row_ptr, o.row_ptr);
+        std::swap(list, o.list);
+        std::swap(halo, o.halo);
+        std::swap(halo_ptr, o.halo_ptr);
+        std::swap(step_ptr, o.step_ptr);
+        std::swap(steps, o.steps);
+        std::swap(wcol, o.wcol);
+        std::swap(own_wcol, o.own_wcol);
+        std::swap(pos, o.pos);
+        std::swap(slots, o.slots);
+        return *this;
+    }
+    ~Team() {
+        void* p[] = {row_ptr, list, halo, halo_ptr, step_ptr, steps, own_wcol ? wcol : nullptr, pos, slots};
+        for (void* q : p)
+            if (q) (void)hipFree(q);
+    }
+    int64_t n_slots() const { return (int64_t)n_teams * COPIES * team_slots(plan.blocks); }
+
+    // Device arrays of a made plan; lists[t]: places in `sys` that team t
+    // solves, in its order.  wcol_in: the array to fill, or null for one of
+    // nnz entries of its own.
+    hipError_t upload(const std::vector<std::vector<int32_t>>& lists, const GroupRec* d_grp, const int32_t* d_col,
+                      int64_t nnz, uint16_t* wcol_in, hipStream_t stream) {
+        n_teams = (int)lists.size();
+        std::vector<int32_t> l{0};
+        for (const auto& t : lists) l.push_back(l.back() + (int32_t)t.size());
+        for (const auto& t : lists) l.insert(l.end(), t.begin(), t.end());
+        int32_t* part = nullptr;
+        hipError_t e = hipSuccess;
+        auto put = [&](auto*& d, const auto* h, size_t n) {
+            if (e == hipSuccess) e = hipMalloc((void**)&d, sizeof(*d) * std::max<size_t>(n, 1));
+            if (e == hipSuccess && h && n) e = hipMemcpy(d, h, sizeof(*d) * n, hipMemcpyHostToDevice);
+        };
+        put(row_ptr, plan.row_ptr.data(), plan.row_ptr.size());
+        put(list, l.data(), l.size());
+        put(halo, plan.halo.data(), plan.halo.size());
+        put(halo_ptr, plan.halo_ptr.data(), plan.halo_ptr.size());
+        put(step_ptr, plan.step_ptr.data(), plan.step_ptr.size());
+        put(steps, plan.steps.data(), plan.steps.size());
+        put(pos, (int*)nullptr, 2 * (size_t)n_teams + 1);
+        put(slots, (unsigned long long*)nullptr, (size_t)n_slots());
+        put(part, plan.part.data(), plan.part.size());
+        own_wcol = wcol_in == nullptr;
+        wcol = wcol_in;
+        if (own_wcol) put(wcol, (uint16_t*)nullptr, (size_t)nnz);
+        if (e == hipSuccess) {
+            const int n_shares = (int)sys.size() * plan.blocks;
+            hipLaunchKernelGGL(k_team_cols, dim3((unsigned)n_shares), dim3(256), 0, stream, n_shares, plan.blocks, part, d_grp,
+                               d_col, halo_ptr, halo, wcol);
+            e = hipGetLastError();
+        }
+        if (e == hipSuccess) e = hipStreamSynchronize(stream);
+        if (part) (void)hipFree(part);
+        // the host keeps the sizes only
+        plan.part = {}; plan.row_ptr = {}; plan.step_ptr = {}; plan.steps = {}; plan.halo_ptr = {}; plan.halo = {};
+        return e;
+    }
+
+    template <typename TA>
+    void args(TeamArgs<TA>& a) const {
+        a.n_teams = n_teams;
+        a.team_blocks = plan.blocks;
+        a.team_sys = list;
+        a.sys_list = list + n_teams + 1;
+        a.team_pos = pos;
+        a.row_ptr = row_ptr;
+        a.step_ptr = step_ptr;
+        a.steps = steps;
+        a.wcol = wcol;
+        a.halo_ptr = halo_ptr;
+        a.halo = halo;
+        a.slots = slots;
+        a.abort = pos + 2 * n_teams;
+    }
+};
 
 struct TeamShape {
     const void* kernel = nullptr;  // null: no kernel holds the plan's largest share
