@@ -1,4 +1,7 @@
-// Batched solves of many independent systems sharing one device context: the
+// Batched solves of many independent systems sharing one device context.  With
+// the layout left to the library the systems are solved on resident teams
+// (pgf_team.hpp, run_teams below); an explicit layout, systems that fit no team
+// and a refused cooperative launch take the launches described next.  The
 // free-free block K_ff of a context whose mesh is a concatenation of
 // independent meshes (RVEs) is block diagonal, one block per RVE, and each
 // block is solved for NR right-hand sides (load cases / sensitivity
@@ -469,9 +472,9 @@ pgft::TeamShape batch_shape(int dim, const pgft::TeamPlan& p) {
 // A team's blocks hold their windows in LDS: as many teams as that allows, 8
 // down to 5, for all systems; if some do not fit even then, those that fit an
 // eighth of the CUs get a launch of their own and the rest at least a quarter,
-// and so on.  (32 RVEs of 64 to 160 divisions, three right-hand sides: 217 ms
-// with three of them in a second launch, BATCHT with all in one; launches with
-// tuned tiles 382 ms.)  Systems are dealt to the teams longest first.  False if
+// and so on.  (32 RVEs of 64 to 160 divisions, three right-hand sides: 222 ms
+// with three of them in a second launch, 200 ms with all in one of seven teams;
+// launches with tuned tiles 382 ms.)  Systems are dealt to the teams longest first.  False if
 // some system fits no team.
 template <int NR>
 bool make_batch_teams(pgfd::Ctx& c, const std::vector<int64_t>& sp) {

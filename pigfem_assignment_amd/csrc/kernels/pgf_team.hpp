@@ -762,10 +762,10 @@ struct TeamShape {
 // The kernel for the plan's largest share: everything in LDS and K in registers
 // where it fits, then K streamed, then r and 1/diag in memory.  us per
 // iteration of a single solve, against five launches:
-//   K in registers: 100 x 100 quads 5.9 (21.3), 333 x 333 10.2 (34.3),
-//     40^3 x 6 tets with FP32 values 12.3 (40.7);
-//   streamed: 460 x 460 quads 22.6 (49.4), 50^3 x 6 tets 36.9 (70.0);
-//   r and 1/diag in memory: 64^3 x 6 tets 100 (159), 700 x 700 quads 47.9 (93.6).
+//   K in registers: 100 x 100 quads 6.0 (21.3), 333 x 333 9.2 (34.3),
+//     40^3 x 6 tets with FP32 values 12.4 (40.7);
+//   streamed: 460 x 460 quads 21.3 (49.4), 50^3 x 6 tets 36.4 (70.0);
+//   r and 1/diag in memory: 64^3 x 6 tets 96 (159), 700 x 700 quads 44.5 (93.6).
 // A window beyond the LDS was tried with gathers through the L2 and fences:
 // 1000 x 1000 quads 212 (196), 80^3 x 6 tets 297 (279): those keep the launches.
 template <typename TA, int NR, int DIM>
