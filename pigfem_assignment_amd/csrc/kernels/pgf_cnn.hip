@@ -90,7 +90,7 @@ struct ConvArgs {
     int relu;
     bf16* out_bf;        // [dout^3][N] or null
     float* out_f;        // [dout^3][N] or null
-    int accumulate;      // out_f += instead of =
+    const float* add;    // [dout^3][N] or null: out_f = this + result
 };
 
 __device__ inline int3 tap_off(int mode, int t) {
@@ -176,10 +176,7 @@ __global__ __launch_bounds__(256) void k_conv(ConvArgs a) {
             if (a.skip) v += bf2f(a.skip[p * a.N + n]);
             if (a.relu) v = v > 0.f ? v : 0.f;
             if (a.out_bf) a.out_bf[p * a.N + n] = f2bf(v);
-            if (a.out_f) {
-                if (a.accumulate) a.out_f[p * a.N + n] += v;
-                else a.out_f[p * a.N + n] = v;
-            }
+            if (a.out_f) a.out_f[p * a.N + n] = a.add ? a.add[p * a.N + n] + v : v;
         }
     }
 }
@@ -249,40 +246,98 @@ __global__ __launch_bounds__(256) void k_wgrad(WgArgs a) {
         }
 }
 
-// gW[t][c][n] = sum over chunks of part[chunk][n][t*C + c]
-__global__ void k_wgrad_reduce(const float* part, int nchunks, int N, int TC, int C, float* gW) {
-    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= N * TC) return;
-    const int n = idx / TC, col = idx % TC;
+// gW[t][c][n] = sum over chunks of part[chunk][n][t*C + c]: 32 entries per
+// block, 8 threads an entry (one thread walking up to 1024 chunks leaves the
+// chip empty: 37 us a layer, 6 us so)
+__global__ __launch_bounds__(256) void k_wgrad_reduce(const float* __restrict__ part, int nchunks, int N, int TC, int C,
+                                                      float* __restrict__ gW) {
+    __shared__ float sh[8][32];
+    const int idx = blockIdx.x * 32 + (threadIdx.x & 31), q = threadIdx.x >> 5;
     float s = 0.f;
-    for (int k = 0; k < nchunks; ++k) s += part[((size_t)k * N + n) * TC + col];
-    const int t = col / C, c = col % C;
-    gW[((size_t)t * C + c) * N + n] = s;
+    if (idx < N * TC)
+        for (int k = q; k < nchunks; k += 8) s += part[(size_t)k * N * TC + idx];
+    sh[q][threadIdx.x & 31] = s;
+    __syncthreads();
+    if (q != 0 || idx >= N * TC) return;
+    for (int k = 1; k < 8; ++k) s += sh[k][threadIdx.x];
+    const int n = idx / TC, col = idx % TC;
+    gW[(size_t)col * N + n] = s;  // col = t*C + c
 }
 
-// bias gradient: gb[n] = sum_p g[p][n]; one block per channel, fixed order
-__global__ void k_bias_grad(const float* g, int np, int N, float* gb) {
+// g = d * (a > 0) (ReLU mask from the stored activation; act null: g = d);
+// gbf = bf16(g), g itself where asked for; and the block's sums of g per
+// channel, the bias gradient's partials, in the same pass.  Bound by memory:
+// FP32 and bf16 in, bf16 out.  A thread's four elements have the same channels
+// in every trip (1024 is a multiple of N).  The gradient as one block per
+// channel, strided over a pass of its own, took up to 336 us a layer.
+constexpr int RB_BLOCKS = 512;
+__global__ __launch_bounds__(256) void k_relu_back(int64_t n4, int N, const float4* __restrict__ d,
+                                                   const ushort4* __restrict__ act, float4* __restrict__ g,
+                                                   ushort4* __restrict__ gbf, float* __restrict__ part) {
+    __shared__ float sh[1024];
+    float4 s = {0.f, 0.f, 0.f, 0.f};
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n4; i += (int64_t)gridDim.x * 256) {
+        float4 v = d[i];
+        if (act) {
+            const ushort4 m = act[i];
+            v.x = bf2f(m.x) > 0.f ? v.x : 0.f;
+            v.y = bf2f(m.y) > 0.f ? v.y : 0.f;
+            v.z = bf2f(m.z) > 0.f ? v.z : 0.f;
+            v.w = bf2f(m.w) > 0.f ? v.w : 0.f;
+        }
+        if (g) g[i] = v;
+        gbf[i] = ushort4{f2bf(v.x), f2bf(v.y), f2bf(v.z), f2bf(v.w)};
+        s.x += v.x;
+        s.y += v.y;
+        s.z += v.z;
+        s.w += v.w;
+    }
+    ((float4*)sh)[threadIdx.x] = s;
+    __syncthreads();
+    // entry e of the block's 1024 sums has channel e % N
+    if ((int)threadIdx.x < N) {
+        float t = 0.f;
+        for (int e = threadIdx.x; e < 1024; e += N) t += sh[e];
+        part[(size_t)blockIdx.x * N + threadIdx.x] = t;
+    }
+}
+
+// gb[n] = sum over blocks of part[block][n], every layer in one launch (a block
+// each: 13 us, as much as one layer's alone)
+struct BiasLayers {
+    int blocks[N_LAYERS], N[N_LAYERS];
+    float* gb[N_LAYERS];
+};
+__global__ __launch_bounds__(256) void k_bias_reduce(const float* __restrict__ part, BiasLayers b) {
     __shared__ float sh[256];
-    const int n = blockIdx.x;
+    const int l = blockIdx.x, N = b.N[l];
+    part += (size_t)l * RB_BLOCKS * 64;
     float s = 0.f;
-    for (int p = threadIdx.x; p < np; p += blockDim.x) s += g[(size_t)p * N + n];
+    for (int e = threadIdx.x; e < b.blocks[l] * N; e += 256) s += part[e];
     sh[threadIdx.x] = s;
     __syncthreads();
-    for (int w = blockDim.x / 2; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) gb[n] = sh[0];
+    if ((int)threadIdx.x >= N) return;
+    for (int e = threadIdx.x + N; e < 256; e += N) s += sh[e];
+    b.gb[l][threadIdx.x] = s;
 }
 
-// g = d * (a > 0) (ReLU mask from the stored activation); gbf = bf16(g)
-__global__ void k_relu_back(int64_t n, const float* d, const bf16* act, float* g, bf16* gbf) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float v = bf2f(act[i]) > 0.f ? d[i] : 0.f;
-    g[i] = v;
-    gbf[i] = f2bf(v);
+// the three used channels of y [NVOX][16], and dy [NVOX][3] with the others zero
+__global__ __launch_bounds__(256) void k_pick_out(const float* __restrict__ y, float* __restrict__ y3) {
+    const int p = blockIdx.x * 256 + threadIdx.x;
+    if (p >= NVOX) return;
+    const float4 v = ((const float4*)y)[4 * (size_t)p];
+    y3[3 * (size_t)p] = v.x;
+    y3[3 * (size_t)p + 1] = v.y;
+    y3[3 * (size_t)p + 2] = v.z;
 }
+__global__ __launch_bounds__(256) void k_widen_out(const float* __restrict__ d3, float* __restrict__ dy) {
+    const int i = blockIdx.x * 256 + threadIdx.x, p = i / 4, q = i % 4;
+    if (p >= NVOX) return;
+    float4 v = {0.f, 0.f, 0.f, 0.f};
+    if (q == 0) v = float4{d3[3 * (size_t)p], d3[3 * (size_t)p + 1], d3[3 * (size_t)p + 2], 0.f};
+    ((float4*)dy)[i] = v;
+}
+
 __global__ void k_to_bf16(int64_t n, const float* x, bf16* y) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) y[i] = f2bf(x[i]);
@@ -366,6 +421,8 @@ struct pgf_net {
     float* part = nullptr;
     size_t part_size = 0;
     float* lossp = nullptr;
+    float* bpart = nullptr;  // bias-gradient partials
+    float* io = nullptr;     // [NVOX][8] staging of host inputs and outputs
     float* dy = nullptr;
     // dataset on the device
     std::vector<bf16*> ds_x;
@@ -387,7 +444,7 @@ static T* nalloc(size_t n) {
 }
 
 pgf_net::~pgf_net() {
-    void* ptrs[] = {params, grads, adam_m, adam_v, x, y, part, lossp, dy};
+    void* ptrs[] = {params, grads, adam_m, adam_v, x, y, part, lossp, dy, bpart, io};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     for (int l = 0; l < N_LAYERS; ++l) {
@@ -403,8 +460,8 @@ pgf_net::~pgf_net() {
 static std::string g_net_err;
 
 static void launch_conv(pgf_net* net, int mode, int C, int N, int din, const bf16* in, const bf16* B, const float* bias,
-                        const bf16* skip, int relu, bf16* out_bf, float* out_f, int accumulate) {
-    ConvArgs a{mode, C, N, din, dout_of(mode, din), in, B, bias, skip, relu, out_bf, out_f, accumulate};
+                        const bf16* skip, int relu, bf16* out_bf, float* out_f, const float* add) {
+    ConvArgs a{mode, C, N, din, dout_of(mode, din), in, B, bias, skip, relu, out_bf, out_f, add};
     const int dout = a.dout;
     const int tiles_pos = mode == UP ? 8 * (din * din * din / 16) : dout * dout * dout / 16;
     const int NT = N >= 64 ? 4 : (N >= 32 ? 2 : 1);
@@ -428,7 +485,7 @@ static void launch_wgrad(pgf_net* net, int l, const bf16* in, const bf16* g, flo
     hipLaunchKernelGGL(k_wgrad, dim3((waves + 3) / 4), dim3(256), 0, net->stream, a);
     NCHK(hipGetLastError());
     const int n = s.cout * TC;
-    hipLaunchKernelGGL(k_wgrad_reduce, dim3((n + 255) / 256), dim3(256), 0, net->stream, (const float*)net->part, nchunks,
+    hipLaunchKernelGGL(k_wgrad_reduce, dim3((n + 31) / 32), dim3(256), 0, net->stream, (const float*)net->part, nchunks,
                        s.cout, TC, s.cin, gW);
     NCHK(hipGetLastError());
 }
@@ -446,73 +503,68 @@ static void refresh_bf16(pgf_net* net) {
 static void forward(pgf_net* net, const bf16* x) {
     float* P = net->params;
     // a1 .. a7
-    launch_conv(net, CONV3, 8, 16, GRID, x, net->Bf[0], P + net->b_off[0], nullptr, 1, net->act[0], nullptr, 0);
-    launch_conv(net, DOWN, 16, 32, GRID, net->act[0], net->Bf[1], P + net->b_off[1], nullptr, 1, net->act[1], nullptr, 0);
-    launch_conv(net, CONV3, 32, 32, GRID / 2, net->act[1], net->Bf[2], P + net->b_off[2], nullptr, 1, net->act[2], nullptr, 0);
-    launch_conv(net, DOWN, 32, 64, GRID / 2, net->act[2], net->Bf[3], P + net->b_off[3], nullptr, 1, net->act[3], nullptr, 0);
-    launch_conv(net, CONV3, 64, 64, GRID / 4, net->act[3], net->Bf[4], P + net->b_off[4], nullptr, 1, net->act[4], nullptr, 0);
-    launch_conv(net, UP, 64, 32, GRID / 4, net->act[4], net->Bf[5], P + net->b_off[5], net->act[2], 1, net->act[5], nullptr, 0);
-    launch_conv(net, UP, 32, 16, GRID / 2, net->act[5], net->Bf[6], P + net->b_off[6], net->act[0], 1, net->act[6], nullptr, 0);
-    launch_conv(net, CONV3, 16, 16, GRID, net->act[6], net->Bf[7], P + net->b_off[7], nullptr, 0, nullptr, net->y, 0);
+    launch_conv(net, CONV3, 8, 16, GRID, x, net->Bf[0], P + net->b_off[0], nullptr, 1, net->act[0], nullptr, nullptr);
+    launch_conv(net, DOWN, 16, 32, GRID, net->act[0], net->Bf[1], P + net->b_off[1], nullptr, 1, net->act[1], nullptr, nullptr);
+    launch_conv(net, CONV3, 32, 32, GRID / 2, net->act[1], net->Bf[2], P + net->b_off[2], nullptr, 1, net->act[2], nullptr, nullptr);
+    launch_conv(net, DOWN, 32, 64, GRID / 2, net->act[2], net->Bf[3], P + net->b_off[3], nullptr, 1, net->act[3], nullptr, nullptr);
+    launch_conv(net, CONV3, 64, 64, GRID / 4, net->act[3], net->Bf[4], P + net->b_off[4], nullptr, 1, net->act[4], nullptr, nullptr);
+    launch_conv(net, UP, 64, 32, GRID / 4, net->act[4], net->Bf[5], P + net->b_off[5], net->act[2], 1, net->act[5], nullptr, nullptr);
+    launch_conv(net, UP, 32, 16, GRID / 2, net->act[5], net->Bf[6], P + net->b_off[6], net->act[0], 1, net->act[6], nullptr, nullptr);
+    launch_conv(net, CONV3, 16, 16, GRID, net->act[6], net->Bf[7], P + net->b_off[7], nullptr, 0, nullptr, net->y, nullptr);
 }
 
-static void relu_back(pgf_net* net, int l) {
-    const int64_t n = act_count(l);
-    hipLaunchKernelGGL(k_relu_back, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, net->stream, n,
-                       (const float*)net->dbuf[l], (const bf16*)net->act[l], net->gbuf[l], net->gbf[l]);
-    NCHK(hipGetLastError());
-}
+static int relu_blocks(int l) { return (int)std::min<int64_t>((act_count(l) / 4 + 255) / 256, RB_BLOCKS); }
 
-static void bias_grad(pgf_net* net, int l, const float* g) {
-    const LayerSpec& s = SPECS[l];
-    const int d = dout_of(s.mode, s.din);
-    hipLaunchKernelGGL(k_bias_grad, dim3(s.cout), dim3(256), 0, net->stream, g, d * d * d, s.cout,
-                       net->grads + net->b_off[l]);
+// layer l's gradient behind its ReLU (layer 7 has none): bf16 copy, FP32 where
+// a skip connection needs it, the bias gradient's partials
+static void relu_back(pgf_net* net, int l, const float* d) {
+    const int64_t n4 = act_count(l) / 4;
+    const int N = SPECS[l].cout;
+    hipLaunchKernelGGL(k_relu_back, dim3(relu_blocks(l)), dim3(256), 0, net->stream, n4, N, (const float4*)d,
+                       (const ushort4*)(l == 7 ? nullptr : net->act[l]), (float4*)net->gbuf[l], (ushort4*)net->gbf[l],
+                       net->bpart + (size_t)l * RB_BLOCKS * 64);
     NCHK(hipGetLastError());
 }
 
 // gradients of sum(dy . y) with respect to every parameter, dy [NVOX][16] FP32 on the device
 static void backward(pgf_net* net, const bf16* x, const float* dy) {
     float* G = net->grads;
-    const int64_t ny = (int64_t)NVOX * 16;
     // layer 7 (output conv3, no ReLU): g7 = dy
-    hipLaunchKernelGGL(k_to_bf16, dim3((unsigned)((ny + 255) / 256)), dim3(256), 0, net->stream, ny, dy, net->gbf[7]);
+    relu_back(net, 7, dy);
     launch_wgrad(net, 7, net->act[6], net->gbf[7], G + net->w_off[7]);
-    bias_grad(net, 7, dy);
     // d a7 = conv3^T(g7)
-    launch_conv(net, CONV3, 16, 16, GRID, net->gbf[7], net->Bd[7], nullptr, nullptr, 0, nullptr, net->dbuf[6], 0);
-    relu_back(net, 6);  // g6 (layer 6 = up2 into a7, skip from a1)
+    launch_conv(net, CONV3, 16, 16, GRID, net->gbf[7], net->Bd[7], nullptr, nullptr, 0, nullptr, net->dbuf[6], nullptr);
+    relu_back(net, 6, net->dbuf[6]);  // g6 (layer 6 = up2 into a7, skip from a1)
     launch_wgrad(net, 6, net->act[5], net->gbf[6], G + net->w_off[6]);
-    bias_grad(net, 6, net->gbuf[6]);
     // d a6 = up2^T(g6) (down form); skip: d a1 gets g6 (fp32)
-    launch_conv(net, DOWN, 16, 32, GRID, net->gbf[6], net->Bd[6], nullptr, nullptr, 0, nullptr, net->dbuf[5], 0);
-    relu_back(net, 5);
+    launch_conv(net, DOWN, 16, 32, GRID, net->gbf[6], net->Bd[6], nullptr, nullptr, 0, nullptr, net->dbuf[5], nullptr);
+    relu_back(net, 5, net->dbuf[5]);
     launch_wgrad(net, 5, net->act[4], net->gbf[5], G + net->w_off[5]);
-    bias_grad(net, 5, net->gbuf[5]);
-    launch_conv(net, DOWN, 32, 64, GRID / 2, net->gbf[5], net->Bd[5], nullptr, nullptr, 0, nullptr, net->dbuf[4], 0);
-    relu_back(net, 4);
+    launch_conv(net, DOWN, 32, 64, GRID / 2, net->gbf[5], net->Bd[5], nullptr, nullptr, 0, nullptr, net->dbuf[4], nullptr);
+    relu_back(net, 4, net->dbuf[4]);
     launch_wgrad(net, 4, net->act[3], net->gbf[4], G + net->w_off[4]);
-    bias_grad(net, 4, net->gbuf[4]);
-    launch_conv(net, CONV3, 64, 64, GRID / 4, net->gbf[4], net->Bd[4], nullptr, nullptr, 0, nullptr, net->dbuf[3], 0);
-    relu_back(net, 3);
+    launch_conv(net, CONV3, 64, 64, GRID / 4, net->gbf[4], net->Bd[4], nullptr, nullptr, 0, nullptr, net->dbuf[3], nullptr);
+    relu_back(net, 3, net->dbuf[3]);
     launch_wgrad(net, 3, net->act[2], net->gbf[3], G + net->w_off[3]);
-    bias_grad(net, 3, net->gbuf[3]);
     // d a3 = down2^T(g3) (up form) + g5 (skip into a6)
-    NCHK(hipMemcpyAsync(net->dbuf[2], net->gbuf[5], sizeof(float) * act_count(2), hipMemcpyDeviceToDevice, net->stream));
-    launch_conv(net, UP, 64, 32, GRID / 4, net->gbf[3], net->Bd[3], nullptr, nullptr, 0, nullptr, net->dbuf[2], 1);
-    relu_back(net, 2);
+    launch_conv(net, UP, 64, 32, GRID / 4, net->gbf[3], net->Bd[3], nullptr, nullptr, 0, nullptr, net->dbuf[2], net->gbuf[5]);
+    relu_back(net, 2, net->dbuf[2]);
     launch_wgrad(net, 2, net->act[1], net->gbf[2], G + net->w_off[2]);
-    bias_grad(net, 2, net->gbuf[2]);
-    launch_conv(net, CONV3, 32, 32, GRID / 2, net->gbf[2], net->Bd[2], nullptr, nullptr, 0, nullptr, net->dbuf[1], 0);
-    relu_back(net, 1);
+    launch_conv(net, CONV3, 32, 32, GRID / 2, net->gbf[2], net->Bd[2], nullptr, nullptr, 0, nullptr, net->dbuf[1], nullptr);
+    relu_back(net, 1, net->dbuf[1]);
     launch_wgrad(net, 1, net->act[0], net->gbf[1], G + net->w_off[1]);
-    bias_grad(net, 1, net->gbuf[1]);
     // d a1 = down2^T(g1) (up form) + g6 (skip into a7)
-    NCHK(hipMemcpyAsync(net->dbuf[0], net->gbuf[6], sizeof(float) * act_count(0), hipMemcpyDeviceToDevice, net->stream));
-    launch_conv(net, UP, 32, 16, GRID / 2, net->gbf[1], net->Bd[1], nullptr, nullptr, 0, nullptr, net->dbuf[0], 1);
-    relu_back(net, 0);
+    launch_conv(net, UP, 32, 16, GRID / 2, net->gbf[1], net->Bd[1], nullptr, nullptr, 0, nullptr, net->dbuf[0], net->gbuf[6]);
+    relu_back(net, 0, net->dbuf[0]);
     launch_wgrad(net, 0, x, net->gbf[0], G + net->w_off[0]);
-    bias_grad(net, 0, net->gbuf[0]);
+    BiasLayers b;
+    for (int l = 0; l < N_LAYERS; ++l) {
+        b.blocks[l] = relu_blocks(l);
+        b.N[l] = SPECS[l].cout;
+        b.gb[l] = G + net->b_off[l];
+    }
+    hipLaunchKernelGGL(k_bias_reduce, dim3(N_LAYERS), dim3(256), 0, net->stream, (const float*)net->bpart, b);
+    NCHK(hipGetLastError());
 }
 
 template <typename F>
@@ -527,11 +579,12 @@ static int nguard(pgf_net* net, F&& f) {
     }
 }
 
+// host input to bf16 on the device (the upload is FP32, the rounding f2bf's)
 static void upload_x(pgf_net* net, const float* xh, bf16* dst) {
-    std::vector<bf16> h((size_t)NVOX * IN_CH);
-    for (size_t i = 0; i < h.size(); ++i) h[i] = f2bf(xh[i]);
-    NCHK(hipMemcpyAsync(dst, h.data(), sizeof(bf16) * h.size(), hipMemcpyHostToDevice, net->stream));
-    NCHK(hipStreamSynchronize(net->stream));
+    const int64_t n = (int64_t)NVOX * IN_CH;
+    NCHK(hipMemcpyAsync(net->io, xh, sizeof(float) * n, hipMemcpyHostToDevice, net->stream));
+    hipLaunchKernelGGL(k_to_bf16, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, net->stream, n, (const float*)net->io, dst);
+    NCHK(hipGetLastError());
 }
 
 extern "C" {
@@ -581,8 +634,8 @@ PGF_API int pgf_net_create(uint64_t seed, pgf_net** out) {
             net->Bf[l] = nalloc<bf16>((size_t)T * s.cin * s.cout);
             net->Bd[l] = nalloc<bf16>((size_t)T * s.cin * s.cout);
             net->act[l] = nalloc<bf16>(act_count(l));
-            net->dbuf[l] = nalloc<float>(act_count(l));
-            net->gbuf[l] = nalloc<float>(act_count(l));
+            if (l < 7) net->dbuf[l] = nalloc<float>(act_count(l));
+            if (l == 5 || l == 6) net->gbuf[l] = nalloc<float>(act_count(l));  // skip connections
             net->gbf[l] = nalloc<bf16>(act_count(l));
             const int d = dout_of(s.mode, s.din);
             const int np = d * d * d;
@@ -595,6 +648,8 @@ PGF_API int pgf_net_create(uint64_t seed, pgf_net** out) {
         net->y = nalloc<float>((size_t)NVOX * 16);
         net->dy = nalloc<float>((size_t)NVOX * 16);
         net->lossp = nalloc<float>(NVOX / 256);
+        net->bpart = nalloc<float>((size_t)N_LAYERS * RB_BLOCKS * 64);
+        net->io = nalloc<float>((size_t)NVOX * IN_CH);
         refresh_bf16(net);
         NCHK(hipStreamSynchronize(net->stream));
     });
@@ -635,11 +690,10 @@ PGF_API int pgf_net_forward(pgf_net* net, const float* x, float* y) {
     return nguard(net, [&]() {
         upload_x(net, x, net->x);
         forward(net, net->x);
-        std::vector<float> h((size_t)NVOX * 16);
-        NCHK(hipMemcpyAsync(h.data(), net->y, sizeof(float) * h.size(), hipMemcpyDeviceToHost, net->stream));
+        hipLaunchKernelGGL(k_pick_out, dim3(NVOX / 256), dim3(256), 0, net->stream, (const float*)net->y, net->io);
+        NCHK(hipGetLastError());
+        NCHK(hipMemcpyAsync(y, net->io, sizeof(float) * NVOX * OUT_CH, hipMemcpyDeviceToHost, net->stream));
         NCHK(hipStreamSynchronize(net->stream));
-        for (int64_t p = 0; p < NVOX; ++p)
-            for (int c = 0; c < OUT_CH; ++c) y[p * OUT_CH + c] = h[p * 16 + c];
     });
 }
 
@@ -648,10 +702,9 @@ PGF_API int pgf_net_backward(pgf_net* net, const float* x, const float* dy, floa
     return nguard(net, [&]() {
         upload_x(net, x, net->x);
         forward(net, net->x);
-        std::vector<float> h((size_t)NVOX * 16, 0.f);
-        for (int64_t p = 0; p < NVOX; ++p)
-            for (int c = 0; c < OUT_CH; ++c) h[p * 16 + c] = dy[p * OUT_CH + c];
-        NCHK(hipMemcpyAsync(net->dy, h.data(), sizeof(float) * h.size(), hipMemcpyHostToDevice, net->stream));
+        NCHK(hipMemcpyAsync(net->io, dy, sizeof(float) * NVOX * OUT_CH, hipMemcpyHostToDevice, net->stream));
+        hipLaunchKernelGGL(k_widen_out, dim3(NVOX / 64), dim3(256), 0, net->stream, (const float*)net->io, net->dy);
+        NCHK(hipGetLastError());
         backward(net, net->x, net->dy);
         NCHK(hipMemcpyAsync(grads, net->grads, sizeof(float) * net->n_params, hipMemcpyDeviceToHost, net->stream));
         NCHK(hipStreamSynchronize(net->stream));
@@ -666,7 +719,8 @@ PGF_API int pgf_net_add_sample(pgf_net* net, const float* x, const float* t) {
         net->ds_x.push_back(dx);
         net->ds_t.push_back(dt);
         upload_x(net, x, dx);
-        NCHK(hipMemcpy(dt, t, sizeof(float) * NVOX * OUT_CH, hipMemcpyHostToDevice));
+        NCHK(hipMemcpyAsync(dt, t, sizeof(float) * NVOX * OUT_CH, hipMemcpyHostToDevice, net->stream));
+        NCHK(hipStreamSynchronize(net->stream));
     });
 }
 
