@@ -182,68 +182,162 @@ __global__ __launch_bounds__(256) void k_conv(ConvArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// Weight gradient: dW[t][c][n] = sum_p in[src(p,t)][c] * g[p][n] over the
-// layer's output positions p, as MFMA tiles (M = n, N = t*C + c, K = p) over
-// chunks of positions; partial tiles go to part[chunk][N_out][T*C], summed
-// by k_wgrad_reduce in chunk order.
+// Weight gradients dW[t][c][n] = sum_p in[src(p,t)][c] * g[p][n] over the
+// layer's output positions p, as MFMA tiles (M = 16 channels n, N = 16 channels
+// c, K = p).
+//
+// Activations are channels-last, so both operands of a product over positions
+// lie across memory; loading them element by element (2 bytes a lane) took 34
+// to 280 us a layer.  A block instead stages 128 output positions at a time in
+// LDS, transposed to [channel][x]: there a lane's four consecutive positions
+// are one 8-byte read, and the lines staged once serve every tap.  A block owns
+// one tile pair (16 c, 16 n), a wavefront the taps of one offset in z (3 x 3 x
+// 3) or in y and z (2 x 2 x 2), whose sums stay in its registers over the
+// block's stages; the partials of the blocks go to part[chunk][N][T*C] and are
+// added by k_wgrad_reduce.  6 to 21 us a layer so, 0.09 ms for all eight
+// (0.94 ms before), bound by the stages' latency: two blocks per CU.
 struct WgArgs {
-    int mode, C, N, din, dout, chunk;
+    int stages;      // stages per block
     const bf16* in;  // [din^3][C]
     const bf16* g;   // [dout^3][N]
-    float* part;     // [n_chunks][N][T*C]
+    float* part;     // [chunks][N][T*C]
 };
+constexpr int WG_POS = 128;  // positions per stage
 
-__global__ __launch_bounds__(256) void k_wgrad(WgArgs a) {
-    const int lane = threadIdx.x & 63;
-    const int wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    const int T = taps(a.mode);
-    const int TC = T * a.C;
-    const int ntn = a.N / 16, ntk = (TC + 15) / 16;
-    const int np = a.dout * a.dout * a.dout;
-    const int nchunks = np / a.chunk;
-    if (wave >= nchunks * ntn * ntk) return;
-    const int ch = wave / (ntn * ntk);
-    const int rem = wave % (ntn * ntk);
-    const int tn = rem / ntk, tk = rem % ntk;
-    const int row = lane & 15, kq = lane >> 4;
-    const int n = tn * 16 + row;              // A row (output channel)
-    const int col = tk * 16 + row;            // B column (t*C + c)
-    const int t = col / a.C, c = col - t * a.C;
-    const int3 o = tap_off(a.mode, t < T ? t : 0);
-    v4f acc = v4f{0.f, 0.f, 0.f, 0.f};
-    for (int p0 = ch * a.chunk; p0 < (ch + 1) * a.chunk; p0 += 16) {
-        short av[4], bv[4];
-        for (int i = 0; i < 4; ++i) {
-            const int p = p0 + kq * 4 + i;
-            av[i] = (short)a.g[(size_t)p * a.N + n];
-            short b = 0;
-            if (col < TC) {
-                const int x = p % a.dout, y = (p / a.dout) % a.dout, z = p / (a.dout * a.dout);
-                int sx, sy, sz;
-                bool ok;
-                if (a.mode == CONV3) {
-                    sx = x + o.x - 1; sy = y + o.y - 1; sz = z + o.z - 1;
-                    ok = sx >= 0 && sy >= 0 && sz >= 0 && sx < a.din && sy < a.din && sz < a.din;
-                } else if (a.mode == DOWN) {
-                    sx = 2 * x + o.x; sy = 2 * y + o.y; sz = 2 * z + o.z;
-                    ok = true;
-                } else {
-                    sx = x >> 1; sy = y >> 1; sz = z >> 1;
-                    ok = (x & 1) == o.x && (y & 1) == o.y && (z & 1) == o.z;
-                }
-                if (ok) b = (short)a.in[((size_t)(sz * a.din + sy) * a.din + sx) * a.C + c];
-            }
-            bv[i] = b;
-        }
-        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(v4s{av[0], av[1], av[2], av[3]}, v4s{bv[0], bv[1], bv[2], bv[3]},
-                                                        acc, 0, 0, 0);
+// 8 channels of one position into rows of a transposed tile
+__device__ inline void put8(bf16* tile, int ld, int x, uint4 v) {
+    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        tile[(2 * i) * ld + x] = (bf16)(w[i] & 0xffffu);
+        tile[(2 * i + 1) * ld + x] = (bf16)(w[i] >> 16);
     }
-    // lane holds rows (n) tn*16 + kq*4 + i, column tk*16 + row
-    if (col < TC)
-        for (int i = 0; i < 4; ++i) {
-            const int nn = tn * 16 + kq * 4 + i;
-            a.part[((size_t)ch * a.N + nn) * TC + col] = acc[i];
+}
+__device__ inline v4s frag(uint32_t a, uint32_t b) {
+    union { uint32_t u[2]; v4s v; } f;
+    f.u[0] = a;
+    f.u[1] = b;
+    return f.v;
+}
+__device__ inline v4s frag_at(const bf16* p) {
+    const uint2 v = *(const uint2*)p;
+    return frag(v.x, v.y);
+}
+
+template <int C, int N, int D>
+__global__ __launch_bounds__(192) void k_wgrad3(WgArgs a) {
+    constexpr int R = WG_POS / D, LI = (R + 2) * 3, LD = D + 4, LG = WG_POS + 4, TC = 27 * C;
+    constexpr int CH = C < 16 ? C : 16, H8 = CH / 8;  // staged input channels, in groups of 8
+    constexpr int CT = C < 16 ? 1 : C / 16, NT = N / 16;
+    __shared__ __align__(16) bf16 s_in[LI][CH][LD], s_g[16][LG];
+    const int lane = threadIdx.x & 63, oz = threadIdx.x >> 6, row = lane & 15, kq = lane >> 4;
+    const int ct = blockIdx.x % CT, nt = blockIdx.x / CT % NT, chunk = blockIdx.x / (CT * NT);
+    v4f acc[3][3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int j = 0; j < 3; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+    // columns outside the grid (x + 1 of 0 and beyond D) stay zero
+    for (int i = threadIdx.x; i < LI * CH * LD / 2; i += 192) ((uint32_t*)s_in)[i] = 0u;
+    for (int st = chunk * a.stages; st < (chunk + 1) * a.stages; ++st) {
+        const int z = st / (D / R), y0 = st % (D / R) * R;
+        __syncthreads();
+        for (int i = threadIdx.x; i < LI * D * H8; i += 192) {
+            const int h = i % H8, x = i / H8 % D, l = i / (H8 * D), lz = z + l / (R + 2) - 1, ly = y0 + l % (R + 2) - 1;
+            uint4 v = {0u, 0u, 0u, 0u};
+            if ((unsigned)lz < (unsigned)D && (unsigned)ly < (unsigned)D)
+                v = *(const uint4*)(a.in + ((size_t)(lz * D + ly) * D + x) * C + ct * CH + h * 8);
+            put8(&s_in[l][h * 8][0], LD, x + 1, v);
         }
+        for (int i = threadIdx.x; i < WG_POS * 2; i += 192) {
+            const int h = i & 1, p = i >> 1;
+            put8(&s_g[h * 8][0], LG, p, *(const uint4*)(a.g + ((size_t)(z * D + y0) * D + p) * N + nt * 16 + h * 8));
+        }
+        __syncthreads();
+#pragma unroll 2
+        for (int k = 0; k < WG_POS / 16; ++k) {
+            const int p = k * 16 + kq * 4, r = p / D, x = p % D;
+            const v4s av = frag_at(&s_g[row][p]);
+#pragma unroll
+            for (int oy = 0; oy < 3; ++oy) {
+                // inputs x - 1 .. x + 6 of the tap's line: the three x offsets
+                const bf16* q = &s_in[oz * (R + 2) + r + oy][row % CH][x];
+                const uint2 lo = *(const uint2*)q, hi = *(const uint2*)(q + 4);
+                const v4s b0 = frag(lo.x, lo.y);
+                const v4s b1 = frag(__builtin_amdgcn_alignbit(lo.y, lo.x, 16), __builtin_amdgcn_alignbit(hi.x, lo.y, 16));
+                const v4s b2 = frag(lo.y, hi.x);
+                if (C >= 16) {
+                    acc[oy][0] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, b0, acc[oy][0], 0, 0, 0);
+                    acc[oy][1] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, b1, acc[oy][1], 0, 0, 0);
+                    acc[oy][2] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, b2, acc[oy][2], 0, 0, 0);
+                } else {
+                    // 8 channels: x offsets 0 and 1 side by side, then 2 alone
+                    const v4s b01 = row < 8 ? b0 : b1;
+                    acc[oy][0] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, b01, acc[oy][0], 0, 0, 0);
+                    acc[oy][1] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, b2, acc[oy][1], 0, 0, 0);
+                }
+            }
+        }
+    }
+    // lane holds channels n = nt*16 + kq*4 + i, column `row`
+#pragma unroll
+    for (int oy = 0; oy < 3; ++oy)
+#pragma unroll
+        for (int j = 0; j < (C >= 16 ? 3 : 2); ++j) {
+            const int ox = C >= 16 ? j : (j == 0 ? row >> 3 : 2), c = C >= 16 ? ct * 16 + row : row & 7;
+            if (C < 16 && j == 1 && row >= 8) continue;
+            const int t = ox + 3 * oy + 9 * oz;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                a.part[((size_t)chunk * N + nt * 16 + kq * 4 + i) * TC + t * C + c] = acc[oy][j][i];
+        }
+}
+
+// 2 x 2 x 2 stride 2 between a fine grid (2H)^3 with CF channels and a coarse
+// one H^3 with CQ: DOWN has in fine and g coarse, UP in coarse and g fine.
+template <int CF, int CQ, int H, bool IS_UP>
+__global__ __launch_bounds__(256) void k_wgrad2(WgArgs a) {
+    constexpr int R = WG_POS / H, LD = H + 4, LG = WG_POS + 4, D = 2 * H;
+    constexpr int C = IS_UP ? CQ : CF, N = IS_UP ? CF : CQ, TC = 8 * C;
+    constexpr int FT = CF / 16, QT = CQ / 16;
+    __shared__ __align__(16) bf16 s_f[R * 4][2][16][LD], s_q[16][LG];
+    const bf16* fine = IS_UP ? a.g : a.in;
+    const bf16* coarse = IS_UP ? a.in : a.g;
+    const int lane = threadIdx.x & 63, oyz = threadIdx.x >> 6, row = lane & 15, kq = lane >> 4;
+    const int ft = blockIdx.x % FT, qt = blockIdx.x / FT % QT, chunk = blockIdx.x / (FT * QT);
+    v4f acc[2];
+    acc[0] = acc[1] = v4f{0.f, 0.f, 0.f, 0.f};
+    for (int st = chunk * a.stages; st < (chunk + 1) * a.stages; ++st) {
+        const int z = st / (H / R), y0 = st % (H / R) * R;
+        __syncthreads();
+        for (int i = threadIdx.x; i < R * 4 * D * 2; i += 256) {
+            const int h = i & 1, x = (i >> 1) % D, l = (i >> 1) / D, r = l >> 2, oy = l & 1, o2 = (l >> 1) & 1;
+            const size_t p = ((size_t)(2 * z + o2) * D + 2 * (y0 + r) + oy) * D + x;
+            put8(&s_f[l][x & 1][h * 8][0], LD, x >> 1, *(const uint4*)(fine + p * CF + ft * 16 + h * 8));
+        }
+        for (int i = threadIdx.x; i < WG_POS * 2; i += 256) {
+            const int h = i & 1, p = i >> 1;
+            put8(&s_q[h * 8][0], LG, p, *(const uint4*)(coarse + ((size_t)(z * H + y0) * H + p) * CQ + qt * 16 + h * 8));
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < WG_POS / 16; ++k) {
+            const int p = k * 16 + kq * 4, r = p / H, x = p % H;
+            const v4s qv = frag_at(&s_q[row][p]);
+#pragma unroll
+            for (int ox = 0; ox < 2; ++ox) {
+                const v4s fv = frag_at(&s_f[r * 4 + oyz][ox][row][x]);
+                acc[ox] = IS_UP ? __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(fv, qv, acc[ox], 0, 0, 0)
+                                : __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(qv, fv, acc[ox], 0, 0, 0);
+            }
+        }
+    }
+    const int nt = IS_UP ? ft : qt, c = (IS_UP ? qt : ft) * 16 + row;
+#pragma unroll
+    for (int ox = 0; ox < 2; ++ox)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            a.part[((size_t)chunk * N + nt * 16 + kq * 4 + i) * TC + (ox + 2 * oyz) * C + c] = acc[ox][i];
 }
 
 // gW[t][c][n] = sum over chunks of part[chunk][n][t*C + c]: 32 entries per
@@ -473,20 +567,39 @@ static void launch_conv(pgf_net* net, int mode, int C, int N, int din, const bf1
     NCHK(hipGetLastError());
 }
 
+// blocks of a weight gradient: tile pairs times chunks of its stages (about 512,
+// two per CU)
+struct WgShape {
+    int tiles, chunks, stages;
+};
+static WgShape wgrad_shape(int l) {
+    const LayerSpec& s = SPECS[l];
+    const int h = s.mode == UP ? s.din : dout_of(s.mode, s.din);  // positions of the sum: the coarser grid
+    const int tiles = std::max(s.cin / 16, 1) * (s.cout / 16), stages = h * h * h / WG_POS;
+    const int per = std::max(1, tiles * stages / 512);
+    return {tiles, stages / per, per};
+}
+
 static void launch_wgrad(pgf_net* net, int l, const bf16* in, const bf16* g, float* gW) {
     const LayerSpec& s = SPECS[l];
-    const int T = taps(s.mode), TC = T * s.cin;
-    const int dout = dout_of(s.mode, s.din);
-    const int np = dout * dout * dout;
-    const int chunk = std::min(np >= 65536 ? 1024 : 256, np);
-    const int nchunks = np / chunk;
-    WgArgs a{s.mode, s.cin, s.cout, s.din, dout, chunk, in, g, net->part};
-    const int waves = nchunks * (s.cout / 16) * ((TC + 15) / 16);
-    hipLaunchKernelGGL(k_wgrad, dim3((waves + 3) / 4), dim3(256), 0, net->stream, a);
+    const WgShape w = wgrad_shape(l);
+    const WgArgs a{w.stages, in, g, net->part};
+    const dim3 grid(w.tiles * w.chunks);
+    hipStream_t st = net->stream;
+    switch (l) {
+        case 0: hipLaunchKernelGGL((k_wgrad3<8, 16, GRID>), grid, dim3(192), 0, st, a); break;
+        case 1: hipLaunchKernelGGL((k_wgrad2<16, 32, GRID / 2, false>), grid, dim3(256), 0, st, a); break;
+        case 2: hipLaunchKernelGGL((k_wgrad3<32, 32, GRID / 2>), grid, dim3(192), 0, st, a); break;
+        case 3: hipLaunchKernelGGL((k_wgrad2<32, 64, GRID / 4, false>), grid, dim3(256), 0, st, a); break;
+        case 4: hipLaunchKernelGGL((k_wgrad3<64, 64, GRID / 4>), grid, dim3(192), 0, st, a); break;
+        case 5: hipLaunchKernelGGL((k_wgrad2<32, 64, GRID / 4, true>), grid, dim3(256), 0, st, a); break;
+        case 6: hipLaunchKernelGGL((k_wgrad2<16, 32, GRID / 2, true>), grid, dim3(256), 0, st, a); break;
+        default: hipLaunchKernelGGL((k_wgrad3<16, 16, GRID>), grid, dim3(192), 0, st, a); break;
+    }
     NCHK(hipGetLastError());
-    const int n = s.cout * TC;
-    hipLaunchKernelGGL(k_wgrad_reduce, dim3((n + 31) / 32), dim3(256), 0, net->stream, (const float*)net->part, nchunks,
-                       s.cout, TC, s.cin, gW);
+    const int TC = taps(s.mode) * s.cin, n = s.cout * TC;
+    hipLaunchKernelGGL(k_wgrad_reduce, dim3((n + 31) / 32), dim3(256), 0, st, (const float*)net->part, w.chunks, s.cout, TC,
+                       s.cin, gW);
     NCHK(hipGetLastError());
 }
 
@@ -637,10 +750,7 @@ PGF_API int pgf_net_create(uint64_t seed, pgf_net** out) {
             if (l < 7) net->dbuf[l] = nalloc<float>(act_count(l));
             if (l == 5 || l == 6) net->gbuf[l] = nalloc<float>(act_count(l));  // skip connections
             net->gbf[l] = nalloc<bf16>(act_count(l));
-            const int d = dout_of(s.mode, s.din);
-            const int np = d * d * d;
-            const int chunk = std::min(np >= 65536 ? 1024 : 256, np);
-            part = std::max(part, (size_t)(np / chunk) * s.cout * (size_t)T * s.cin);
+            part = std::max(part, (size_t)wgrad_shape(l).chunks * s.cout * (size_t)T * s.cin);
         }
         net->part = nalloc<float>(part);
         net->part_size = part;
