@@ -74,111 +74,230 @@ __device__ __host__ inline float bf2f(bf16 h) {
 
 // ---------------------------------------------------------------------------
 // Implicit-GEMM convolution, forward form.
-//   out[p][n] = bias[n] + sum_{t,c} in[src(p,t)][c] * B[n][t*C + c]
+//   out[p][n] = sum_{t,c} in[src(p,t)][c] * B[n][t*C + c]
 // CONV3: src = p + off(t) - 1 (zero outside); DOWN: src = 2p + off(t);
-// UP: tiles are grouped by output parity class cls, the only tap is t = cls
-// and src = p / 2.  One wavefront computes 16 output positions (consecutive
-// along x; for UP consecutive input positions of one parity class) times
-// 16*NT output channels.  Epilogue: + bias, + skip (bf16, same shape as out),
-// ReLU, store bf16 and/or FP32 (or add into FP32).
+// UP: the output's parity is the tap, t = parity, and src = p / 2.  Epilogue of
+// the forward pass: + bias, + skip (bf16, same shape as out), ReLU; of the data
+// gradients (BACK): + the skip connection's gradient, the mask of the ReLU in
+// front of it, and the sums per channel, which are that layer's bias gradient.
+//
+// MFMA tiles with M = 16 channels, N = 16 positions along x, so that a lane
+// ends with four consecutive channels of one position: 8- and 16-byte stores.
+// The weights lie in fragment order (k_weights_bf16), 512 contiguous bytes a
+// step.  The layers are small (one to four waves per SIMD), so latency bounds
+// them: sizes are template parameters, the steps of the sum (16 wide) are
+// unrolled and loaded KB steps ahead of their products.  4.5 to 20 us a layer,
+// 64 us for a forward pass; loaded step by step, 9 to 105 and 0.28 ms.
 struct ConvArgs {
-    int mode, C, N, din, dout;
-    const bf16* in;      // [din^3][C]
-    const bf16* B;       // [N][T*C]
-    const float* bias;   // [N] or null
-    const bf16* skip;    // [dout^3][N] or null
-    int relu;
+    const bf16* in;      // [DIN^3][C]
+    const bf16* B;       // fragments of [N][T*C]
     bf16* out_bf;        // [dout^3][N] or null
     float* out_f;        // [dout^3][N] or null
-    const float* add;    // [dout^3][N] or null: out_f = this + result
+    // forward
+    const float* bias;   // [N]
+    const bf16* skip;    // [dout^3][N] or null
+    int relu;
+    // data gradient
+    const float* add;    // [dout^3][N] or null
+    const bf16* act;     // [dout^3][N]
+    float* bpart;        // [blocks][N] sums
 };
 
-__device__ inline int3 tap_off(int mode, int t) {
-    if (mode == CONV3) return make_int3(t % 3, (t / 3) % 3, t / 9);
-    return make_int3(t & 1, (t >> 1) & 1, t >> 2);
+__device__ inline v4s frag(uint32_t a, uint32_t b) {
+    union { uint32_t u[2]; v4s v; } f;
+    f.u[0] = a;
+    f.u[1] = b;
+    return f.v;
+}
+__device__ inline v4s frag_at(const bf16* p) {
+    const uint2 v = *(const uint2*)p;
+    return frag(v.x, v.y);
 }
 
-template <int NT>
-__global__ __launch_bounds__(256) void k_conv(ConvArgs a) {
-    const int lane = threadIdx.x & 63;
-    const int wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    const int T = taps(a.mode);
-    const int n_tiles_pos = a.mode == UP ? 8 * (a.din * a.din * a.din / 16) : a.dout * a.dout * a.dout / 16;
-    const int n_tiles_ch = a.N / (16 * NT);
-    if (wave >= n_tiles_pos * n_tiles_ch) return;
-    const int tpos = wave / n_tiles_ch, tch = wave % n_tiles_ch;
-    const int row = lane & 15, kq = lane >> 4;
-    // output position of this lane's A row (m = row)
-    int cls = 0, px, py, pz, ix = 0, iy = 0, iz = 0;
-    if (a.mode == UP) {
-        const int per = a.din * a.din * a.din / 16;
-        cls = tpos / per;
-        const int i = (tpos % per) * 16 + row;
-        ix = i % a.din; iy = (i / a.din) % a.din; iz = i / (a.din * a.din);
-        px = 2 * ix + (cls & 1); py = 2 * iy + ((cls >> 1) & 1); pz = 2 * iz + (cls >> 2);
+// channels n .. n + 3 of the output position whose first channel is element e
+template <bool BACK>
+__device__ inline void conv_out(const ConvArgs& a, size_t e, int n, v4f acc, float4& bs) {
+    float4 v = {acc[0], acc[1], acc[2], acc[3]};
+    if (!BACK) {
+        const float4 b = *(const float4*)(a.bias + n);
+        v = float4{v.x + b.x, v.y + b.y, v.z + b.z, v.w + b.w};
+        if (a.skip) {
+            const ushort4 k = *(const ushort4*)(a.skip + e);
+            v = float4{v.x + bf2f(k.x), v.y + bf2f(k.y), v.z + bf2f(k.z), v.w + bf2f(k.w)};
+        }
+        if (a.relu) v = float4{v.x > 0.f ? v.x : 0.f, v.y > 0.f ? v.y : 0.f, v.z > 0.f ? v.z : 0.f, v.w > 0.f ? v.w : 0.f};
     } else {
-        const int p = tpos * 16 + row;
-        px = p % a.dout; py = (p / a.dout) % a.dout; pz = p / (a.dout * a.dout);
-    }
-    const int K = a.mode == UP ? a.C : T * a.C;
-    const int ldb = T * a.C;
-    const int boff = a.mode == UP ? cls * a.C : 0;
-    v4f acc[NT];
-    for (int j = 0; j < NT; ++j) acc[j] = v4f{0.f, 0.f, 0.f, 0.f};
-    for (int k0 = 0; k0 < K; k0 += 16) {
-        const int kk = k0 + kq * 4;  // this lane's 4 consecutive k
-        v4s av = v4s{0, 0, 0, 0};
-        if (kk < K) {
-            int src = -1, c;
-            if (a.mode == UP) {
-                c = kk;
-                src = (iz * a.din + iy) * a.din + ix;
-            } else {
-                const int t = kk / a.C;
-                c = kk - t * a.C;
-                const int3 o = tap_off(a.mode, t);
-                int sx, sy, sz;
-                if (a.mode == CONV3) { sx = px + o.x - 1; sy = py + o.y - 1; sz = pz + o.z - 1; }
-                else { sx = 2 * px + o.x; sy = 2 * py + o.y; sz = 2 * pz + o.z; }
-                if (sx >= 0 && sy >= 0 && sz >= 0 && sx < a.din && sy < a.din && sz < a.din) src = (sz * a.din + sy) * a.din + sx;
-            }
-            if (src >= 0) {
-                const uint2 v = *reinterpret_cast<const uint2*>(a.in + (size_t)src * a.C + c);
-                av = v4s{(short)(v.x & 0xffff), (short)(v.x >> 16), (short)(v.y & 0xffff), (short)(v.y >> 16)};
-            }
+        if (a.add) {
+            const float4 d = *(const float4*)(a.add + e);
+            v = float4{d.x + v.x, d.y + v.y, d.z + v.z, d.w + v.w};
         }
-        for (int j = 0; j < NT; ++j) {
-            const int n = (tch * NT + j) * 16 + row;
-            v4s bv = v4s{0, 0, 0, 0};
-            if (kk < K) {
-                const uint2 v = *reinterpret_cast<const uint2*>(a.B + (size_t)n * ldb + boff + kk);
-                bv = v4s{(short)(v.x & 0xffff), (short)(v.x >> 16), (short)(v.y & 0xffff), (short)(v.y >> 16)};
-            }
-            acc[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, bv, acc[j], 0, 0, 0);
-        }
+        const ushort4 m = *(const ushort4*)(a.act + e);
+        v = float4{bf2f(m.x) > 0.f ? v.x : 0.f, bf2f(m.y) > 0.f ? v.y : 0.f, bf2f(m.z) > 0.f ? v.z : 0.f,
+                   bf2f(m.w) > 0.f ? v.w : 0.f};
+        bs = float4{bs.x + v.x, bs.y + v.y, bs.z + v.z, bs.w + v.w};
     }
-    // epilogue: lane holds rows m = kq*4 + i, column n = row
+    if (a.out_bf) *(ushort4*)(a.out_bf + e) = ushort4{f2bf(v.x), f2bf(v.y), f2bf(v.z), f2bf(v.w)};
+    if (a.out_f) *(float4*)(a.out_f + e) = v;
+}
+
+// the block's sums of the channels n0 .. n0 + 16 NT of bs, to dst
+template <int NT>
+__device__ inline void conv_bias_sums(float4 (&bs)[NT], float* dst) {
+    __shared__ float sb[4][16 * NT];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
     for (int j = 0; j < NT; ++j) {
-        const int n = (tch * NT + j) * 16 + row;
-        const float bn = a.bias ? a.bias[n] : 0.f;
-        for (int i = 0; i < 4; ++i) {
-            const int m = kq * 4 + i;
-            size_t p;
-            if (a.mode == UP) {
-                const int per = a.din * a.din * a.din / 16;
-                const int ii = (tpos % per) * 16 + m;
-                const int jx = ii % a.din, jy = (ii / a.din) % a.din, jz = ii / (a.din * a.din);
-                p = ((size_t)(2 * jz + (cls >> 2)) * a.dout + 2 * jy + ((cls >> 1) & 1)) * a.dout + 2 * jx + (cls & 1);
-            } else {
-                p = (size_t)tpos * 16 + m;
-            }
-            float v = acc[j][i] + bn;
-            if (a.skip) v += bf2f(a.skip[p * a.N + n]);
-            if (a.relu) v = v > 0.f ? v : 0.f;
-            if (a.out_bf) a.out_bf[p * a.N + n] = f2bf(v);
-            if (a.out_f) a.out_f[p * a.N + n] = a.add ? a.add[p * a.N + n] + v : v;
+#pragma unroll
+        for (int m = 1; m < 16; m *= 2) {
+            bs[j].x += __shfl_xor(bs[j].x, m);
+            bs[j].y += __shfl_xor(bs[j].y, m);
+            bs[j].z += __shfl_xor(bs[j].z, m);
+            bs[j].w += __shfl_xor(bs[j].w, m);
+        }
+        if ((lane & 15) == 0) *(float4*)&sb[wave][j * 16 + (lane >> 4) * 4] = bs[j];
+    }
+    __syncthreads();
+    const int n = threadIdx.x;
+    if (n < 16 * NT) dst[n] = sb[0][n] + sb[1][n] + sb[2][n] + sb[3][n];
+}
+
+// CONV3.  A block takes YB lines of a plane and 16 channels: the lines around
+// them go to LDS once, with the zeros outside the grid, so a tap is an offset
+// within the block's lines, while the weights travel to registers; the loads
+// are one latency, and every input is read from memory 18 / YB times instead
+// of 27.  Positions are padded by 8 bytes from 32 channels on (bank conflicts).
+template <bool BACK, int C, int N, int D, int YB>
+__global__ __launch_bounds__(256) void k_conv3(ConvArgs a) {
+    constexpr int KS = (27 * C + 15) / 16, KB = 9, NB = (KS + KB - 1) / KB, NCT = N / 16;
+    constexpr int LI = (YB + 2) * 3, PS = C + (C >= 32 ? 4 : 0), LINE = (D + 2) * PS;
+    constexpr int XT = D / 16, WY = 4 / XT, PT = YB / WY, H8 = C / 8, LOADS = (LI * D * H8 + 255) / 256;
+    __shared__ __align__(16) bf16 s_in[LI * LINE];
+    const int lane = threadIdx.x & 63, row = lane & 15, kq = lane >> 4, wave = threadIdx.x >> 6;
+    const int tch = blockIdx.x % NCT, y0 = blockIdx.x / NCT % (D / YB) * YB, z = blockIdx.x / NCT / (D / YB);
+    v4s w[KS];
+#pragma unroll
+    for (int s = 0; s < KS; ++s) w[s] = frag_at(a.B + ((size_t)(tch * KS + s) * 64 + lane) * 4);
+    uint4 v[LOADS];
+#pragma unroll
+    for (int k = 0; k < LOADS; ++k) {
+        const int i = k * 256 + threadIdx.x, h = i % H8, x = i / H8 % D, l = i / (H8 * D);
+        const int ly = y0 + l % (YB + 2) - 1, lz = z + l / (YB + 2) - 1;
+        v[k] = uint4{0u, 0u, 0u, 0u};
+        if (l < LI && (unsigned)ly < (unsigned)D && (unsigned)lz < (unsigned)D)
+            v[k] = *(const uint4*)(a.in + ((size_t)(lz * D + ly) * D + x) * C + h * 8);
+    }
+    for (int i = threadIdx.x; i < LI * 2 * (C / 4); i += 256) {
+        const int c4 = i % (C / 4), side = i / (C / 4) & 1, l = i / (C / 4 * 2);
+        *(uint2*)&s_in[l * LINE + side * (D + 1) * PS + c4 * 4] = uint2{0u, 0u};
+    }
+#pragma unroll
+    for (int k = 0; k < LOADS; ++k) {
+        const int i = k * 256 + threadIdx.x, h = i % H8, x = i / H8 % D, l = i / (H8 * D);
+        if (l < LI) {
+            bf16* q = &s_in[l * LINE + (x + 1) * PS + h * 8];
+            *(uint2*)q = uint2{v[k].x, v[k].y};
+            *(uint2*)(q + 4) = uint2{v[k].z, v[k].w};
         }
     }
+    __syncthreads();
+    const int x = wave % XT * 16 + row, wy = wave / XT * PT;
+    float4 bs[1] = {{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll 1
+    for (int t = wy; t < wy + PT; ++t) {
+        const bf16* base = &s_in[t * LINE + x * PS + (C >= 16 ? kq : kq & 1) * 4];
+        auto off = [&](int tap) { return (tap / 9 * (YB + 2) + tap / 3 % 3) * LINE + tap % 3 * PS; };
+        v4s av[2][KB];
+        auto fetch = [&](int b) {
+#pragma unroll
+            for (int i = 0; i < KB; ++i) {
+                const int s = b * KB + i;
+                if (s >= KS) break;
+                if (C >= 16) {
+                    av[b & 1][i] = frag_at(base + off(s * 16 / C) + s * 16 % C);
+                } else {  // 8 channels: two taps a step, the last alone
+                    const int o0 = off(2 * s), o1 = 2 * s + 1 < 27 ? off(2 * s + 1) : o0;
+                    const v4s f = frag_at(base + (kq < 2 ? o0 : o1));
+                    av[b & 1][i] = 2 * s + 1 < 27 || kq < 2 ? f : v4s{0, 0, 0, 0};
+                }
+            }
+        };
+        v4f acc = {0.f, 0.f, 0.f, 0.f};
+        fetch(0);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            if (b + 1 < NB) fetch(b + 1);
+            __builtin_amdgcn_sched_barrier(0);  // else the loads sink to their products
+#pragma unroll
+            for (int i = 0; i < KB; ++i)
+                if (b * KB + i < KS) acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(w[b * KB + i], av[b & 1][i], acc, 0, 0, 0);
+        }
+        const int n = tch * 16 + kq * 4;
+        conv_out<BACK>(a, ((size_t)(z * D + y0 + t) * D + x) * N + n, n, acc, bs[0]);
+    }
+    if (BACK) conv_bias_sums<1>(bs, a.bpart + (size_t)(blockIdx.x / NCT) * N + tch * 16);
+}
+
+// DOWN and UP, no input read twice: fragments straight from memory.  A
+// wavefront takes one tile of positions (UP: of the input's, both parities in
+// x) and 16 NT channels.
+template <bool BACK, int MODE, int C, int N, int DIN, int NT>
+__global__ __launch_bounds__(256) void k_conv2(ConvArgs a) {
+    constexpr int S = MODE == DOWN ? DIN / 2 : DIN, DOUT = dout_of(MODE, DIN), CS = C / 16, KST = 8 * CS;
+    constexpr int KS = MODE == UP ? CS : KST, KB = KS < 8 ? KS : 8, NB = KS / KB;
+    constexpr int XT = S / 16, NCT = N / (16 * NT), CLS = MODE == UP ? 2 : 1;
+    const int lane = threadIdx.x & 63, row = lane & 15, kq = lane >> 4;
+    // x tile fastest, then y, z, for UP the parity in y and z
+    const int tch = blockIdx.x % NCT;
+    int u = blockIdx.x / NCT * 4 + (threadIdx.x >> 6);
+    const int x = u % XT * 16 + row;
+    u /= XT;
+    const int y = u % S, z = u / S % S, par = u / (S * S);  // par = oy + 2 oz
+    const bf16* src = a.in + ((size_t)((MODE == DOWN ? 2 * z : z) * DIN + (MODE == DOWN ? 2 * y : y)) * DIN +
+                              (MODE == DOWN ? 2 * x : x)) * C + kq * 4;
+    const bf16* wts = a.B + ((size_t)(tch * NT * KST + 2 * par * CS) * 64 + lane) * 4;
+    v4s av[2][KB], bv[2][KB][NT][CLS];
+    auto fetch = [&](int b) {
+#pragma unroll
+        for (int i = 0; i < KB; ++i) {
+            const int s = b * KB + i, t = s / CS;
+            av[b & 1][i] = frag_at(src + (MODE == UP ? 0 : (((t >> 2) * DIN + (t >> 1 & 1)) * DIN + (t & 1)) * C) + s % CS * 16);
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+#pragma unroll
+                for (int c = 0; c < CLS; ++c) bv[b & 1][i][j][c] = frag_at(wts + (size_t)(j * KST + c * CS + s) * 256);
+        }
+    };
+    v4f acc[NT][CLS];
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int c = 0; c < CLS; ++c) acc[j][c] = v4f{0.f, 0.f, 0.f, 0.f};
+    fetch(0);
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        if (b + 1 < NB) fetch(b + 1);
+        __builtin_amdgcn_sched_barrier(0);  // else the loads sink to their products
+#pragma unroll
+        for (int i = 0; i < KB; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+#pragma unroll
+                for (int c = 0; c < CLS; ++c)
+                    acc[j][c] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(bv[b & 1][i][j][c], av[b & 1][i], acc[j][c], 0, 0, 0);
+    }
+    float4 bs[NT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+        bs[j] = float4{0.f, 0.f, 0.f, 0.f};
+        const int n = (tch * NT + j) * 16 + kq * 4;
+#pragma unroll
+        for (int c = 0; c < CLS; ++c) {
+            const size_t p = MODE == UP ? (size_t)((2 * z + (par >> 1)) * DOUT + 2 * y + (par & 1)) * DOUT + 2 * x + c
+                                        : (size_t)(z * DOUT + y) * DOUT + x;
+            conv_out<BACK>(a, p * N + n, n, acc[j][c], bs[j]);
+        }
+    }
+    if (BACK) conv_bias_sums<NT>(bs, a.bpart + (size_t)(blockIdx.x / NCT) * N + tch * NT * 16);
 }
 
 // ---------------------------------------------------------------------------
@@ -213,17 +332,6 @@ __device__ inline void put8(bf16* tile, int ld, int x, uint4 v) {
         tile[(2 * i + 1) * ld + x] = (bf16)(w[i] >> 16);
     }
 }
-__device__ inline v4s frag(uint32_t a, uint32_t b) {
-    union { uint32_t u[2]; v4s v; } f;
-    f.u[0] = a;
-    f.u[1] = b;
-    return f.v;
-}
-__device__ inline v4s frag_at(const bf16* p) {
-    const uint2 v = *(const uint2*)p;
-    return frag(v.x, v.y);
-}
-
 template <int C, int N, int D>
 __global__ __launch_bounds__(192) void k_wgrad3(WgArgs a) {
     constexpr int R = WG_POS / D, LI = (R + 2) * 3, LD = D + 4, LG = WG_POS + 4, TC = 27 * C;
@@ -340,46 +448,46 @@ __global__ __launch_bounds__(256) void k_wgrad2(WgArgs a) {
             a.part[((size_t)chunk * N + nt * 16 + kq * 4 + i) * TC + (ox + 2 * oyz) * C + c] = acc[ox][i];
 }
 
-// gW[t][c][n] = sum over chunks of part[chunk][n][t*C + c]: 32 entries per
-// block, 8 threads an entry (one thread walking up to 1024 chunks leaves the
-// chip empty: 37 us a layer, 6 us so)
-__global__ __launch_bounds__(256) void k_wgrad_reduce(const float* __restrict__ part, int nchunks, int N, int TC, int C,
-                                                      float* __restrict__ gW) {
+// gW[t][c][n] = sum over chunks of part[chunk][n][t*C + c], every layer in one
+// launch: 32 entries per block, 8 threads an entry.  Bound by memory: the
+// partials, 62 MB in 14 us (eight launches of 10 us before).
+struct WgLayers {
+    int first[N_LAYERS + 1];  // blocks
+    int chunks[N_LAYERS], N[N_LAYERS], TC[N_LAYERS];
+    const float* part[N_LAYERS];
+    float* gW[N_LAYERS];
+};
+__global__ __launch_bounds__(256) void k_wgrad_reduce(WgLayers w) {
     __shared__ float sh[8][32];
-    const int idx = blockIdx.x * 32 + (threadIdx.x & 31), q = threadIdx.x >> 5;
+    int l = 0;
+    while ((int)blockIdx.x >= w.first[l + 1]) ++l;
+    const int nchunks = w.chunks[l], N = w.N[l], TC = w.TC[l];
+    const float* part = w.part[l];
+    const int idx = (blockIdx.x - w.first[l]) * 32 + (threadIdx.x & 31), q = threadIdx.x >> 5;
     float s = 0.f;
-    if (idx < N * TC)
+    if (idx < N * TC) {
+#pragma unroll 8
         for (int k = q; k < nchunks; k += 8) s += part[(size_t)k * N * TC + idx];
+    }
     sh[q][threadIdx.x & 31] = s;
     __syncthreads();
     if (q != 0 || idx >= N * TC) return;
     for (int k = 1; k < 8; ++k) s += sh[k][threadIdx.x];
     const int n = idx / TC, col = idx % TC;
-    gW[(size_t)col * N + n] = s;  // col = t*C + c
+    w.gW[l][(size_t)col * N + n] = s;  // col = t*C + c
 }
 
-// g = d * (a > 0) (ReLU mask from the stored activation; act null: g = d);
-// gbf = bf16(g), g itself where asked for; and the block's sums of g per
-// channel, the bias gradient's partials, in the same pass.  Bound by memory:
-// FP32 and bf16 in, bf16 out.  A thread's four elements have the same channels
-// in every trip (1024 is a multiple of N).  The gradient as one block per
-// channel, strided over a pass of its own, took up to 336 us a layer.
+// bf16(d) of the output layer's gradient and the block's sums of d per channel,
+// its bias gradient's partials (the other layers' come from the convolutions).
+// Bound by memory.  A thread's four elements have the same channels in every
+// trip (1024 is a multiple of N).
 constexpr int RB_BLOCKS = 512;
-__global__ __launch_bounds__(256) void k_relu_back(int64_t n4, int N, const float4* __restrict__ d,
-                                                   const ushort4* __restrict__ act, float4* __restrict__ g,
-                                                   ushort4* __restrict__ gbf, float* __restrict__ part) {
+__global__ __launch_bounds__(256) void k_out_back(int64_t n4, int N, const float4* __restrict__ d,
+                                                  ushort4* __restrict__ gbf, float* __restrict__ part) {
     __shared__ float sh[1024];
     float4 s = {0.f, 0.f, 0.f, 0.f};
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n4; i += (int64_t)gridDim.x * 256) {
-        float4 v = d[i];
-        if (act) {
-            const ushort4 m = act[i];
-            v.x = bf2f(m.x) > 0.f ? v.x : 0.f;
-            v.y = bf2f(m.y) > 0.f ? v.y : 0.f;
-            v.z = bf2f(m.z) > 0.f ? v.z : 0.f;
-            v.w = bf2f(m.w) > 0.f ? v.w : 0.f;
-        }
-        if (g) g[i] = v;
+        const float4 v = d[i];
         gbf[i] = ushort4{f2bf(v.x), f2bf(v.y), f2bf(v.z), f2bf(v.w)};
         s.x += v.x;
         s.y += v.y;
@@ -397,21 +505,23 @@ __global__ __launch_bounds__(256) void k_relu_back(int64_t n4, int N, const floa
 }
 
 // gb[n] = sum over blocks of part[block][n], every layer in one launch (a block
-// each: 13 us, as much as one layer's alone)
+// each)
 struct BiasLayers {
     int blocks[N_LAYERS], N[N_LAYERS];
     float* gb[N_LAYERS];
 };
-__global__ __launch_bounds__(256) void k_bias_reduce(const float* __restrict__ part, BiasLayers b) {
-    __shared__ float sh[256];
+constexpr int BIAS_PART = 512 * 64;  // floats per layer, the most any has (blocks x channels)
+__global__ __launch_bounds__(1024) void k_bias_reduce(const float* __restrict__ part, BiasLayers b) {
+    __shared__ float sh[1024];
     const int l = blockIdx.x, N = b.N[l];
-    part += (size_t)l * RB_BLOCKS * 64;
+    part += (size_t)l * BIAS_PART;
     float s = 0.f;
-    for (int e = threadIdx.x; e < b.blocks[l] * N; e += 256) s += part[e];
+#pragma unroll 4
+    for (int e = threadIdx.x; e < b.blocks[l] * N; e += 1024) s += part[e];
     sh[threadIdx.x] = s;
     __syncthreads();
     if ((int)threadIdx.x >= N) return;
-    for (int e = threadIdx.x + N; e < 256; e += N) s += sh[e];
+    for (int e = threadIdx.x + N; e < 1024; e += N) s += sh[e];
     b.gb[l][threadIdx.x] = s;
 }
 
@@ -440,14 +550,20 @@ __global__ void k_to_bf16(int64_t n, const float* x, bf16* y) {
 // bf16 weight copies from the FP32 master W[t][c][n]:
 //   Bf[n][t*C + c] = W[t][c][n]             (forward)
 //   Bd[c][t*N + n] = W[flip(t)][c][n]       (data gradient; flip = 26 - t for conv3)
+// both as fragments: 16 rows by 16 columns, the columns padded to 16, a lane's
+// four consecutive columns of a row side by side.
+__host__ __device__ constexpr int frag_count(int rows, int cols) { return (rows + 15) / 16 * ((cols + 15) / 16) * 256; }
+__device__ inline int frag_index(int r, int k, int cols) {
+    return ((r >> 4) * ((cols + 15) >> 4) + (k >> 4)) * 256 + ((k & 15) >> 2) * 64 + (r & 15) * 4 + (k & 3);
+}
 __global__ void k_weights_bf16(int mode, int T, int C, int N, const float* W, bf16* Bf, bf16* Bd) {
     const int idx = blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= T * C * N) return;
     const int t = idx / (C * N), c = (idx / N) % C, n = idx % N;
     const bf16 h = f2bf(W[idx]);
-    Bf[(size_t)n * T * C + t * C + c] = h;
+    Bf[frag_index(n, t * C + c, T * C)] = h;
     const int tf = mode == CONV3 ? 26 - t : t;
-    Bd[(size_t)c * T * N + tf * N + n] = h;
+    Bd[frag_index(c, tf * N + n, T * N)] = h;
 }
 
 // Adam (FP32): m = b1 m + (1-b1) g; v = b2 v + (1-b2) g^2; w -= lr mhat / (sqrt(vhat) + eps)
@@ -510,10 +626,10 @@ struct pgf_net {
     bf16* act[N_LAYERS] = {};  // act[l] = output of layer l (l < 7); act input separately
     bf16* x = nullptr;
     float* y = nullptr;
-    float *dbuf[N_LAYERS] = {}, *gbuf[N_LAYERS] = {};  // d (fp32 grad wrt layer output), g (after ReLU mask)
+    float* gbuf[N_LAYERS] = {};  // gradient behind the ReLU, FP32 where a skip connection needs it
     bf16* gbf[N_LAYERS] = {};
-    float* part = nullptr;
-    size_t part_size = 0;
+    float* part = nullptr;       // weight-gradient partials, layer after layer
+    size_t part_off[N_LAYERS];
     float* lossp = nullptr;
     float* bpart = nullptr;  // bias-gradient partials
     float* io = nullptr;     // [NVOX][8] staging of host inputs and outputs
@@ -542,7 +658,7 @@ pgf_net::~pgf_net() {
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     for (int l = 0; l < N_LAYERS; ++l) {
-        void* q[] = {Bf[l], Bd[l], act[l], dbuf[l], gbuf[l], gbf[l]};
+        void* q[] = {Bf[l], Bd[l], act[l], gbuf[l], gbf[l]};
         for (void* p : q)
             if (p) (void)hipFree(p);
     }
@@ -553,19 +669,39 @@ pgf_net::~pgf_net() {
 
 static std::string g_net_err;
 
-static void launch_conv(pgf_net* net, int mode, int C, int N, int din, const bf16* in, const bf16* B, const float* bias,
-                        const bf16* skip, int relu, bf16* out_bf, float* out_f, const float* add) {
-    ConvArgs a{mode, C, N, din, dout_of(mode, din), in, B, bias, skip, relu, out_bf, out_f, add};
-    const int dout = a.dout;
-    const int tiles_pos = mode == UP ? 8 * (din * din * din / 16) : dout * dout * dout / 16;
-    const int NT = N >= 64 ? 4 : (N >= 32 ? 2 : 1);
-    const int waves = tiles_pos * (N / (16 * NT));
-    const int blocks = (waves + 3) / 4;
-    if (NT == 4) hipLaunchKernelGGL(k_conv<4>, dim3(blocks), dim3(256), 0, net->stream, a);
-    else if (NT == 2) hipLaunchKernelGGL(k_conv<2>, dim3(blocks), dim3(256), 0, net->stream, a);
-    else hipLaunchKernelGGL(k_conv<1>, dim3(blocks), dim3(256), 0, net->stream, a);
+// One of the layer forms, both ways; returns the rows of bias partials that the
+// data gradient leaves.  Four lines per block: 9.2, 20, 10.8 us for the first
+// three below, against 10.9, 20, 12.9 with two and 9.6, 21, 10.4 with eight.
+// Two channel tiles per wavefront for down_fine, 4.8 us against 5.3, one where
+// two leave half the chip's wavefront slots empty.
+template <int C, int N, int D, int YB>
+static int conv3(pgf_net* net, const ConvArgs& a) {
+    const int rows = D / YB * D;
+    const dim3 grid(rows * (N / 16));
+    if (!a.act) hipLaunchKernelGGL((k_conv3<false, C, N, D, YB>), grid, dim3(256), 0, net->stream, a);
+    // (the network's input has no gradient)
+    else if constexpr (C != IN_CH) hipLaunchKernelGGL((k_conv3<true, C, N, D, YB>), grid, dim3(256), 0, net->stream, a);
     NCHK(hipGetLastError());
+    return rows;
 }
+template <int MODE, int C, int N, int DIN, int NT>
+static int conv2(pgf_net* net, const ConvArgs& a) {
+    constexpr int S = MODE == DOWN ? DIN / 2 : DIN;
+    const int rows = S * S * S / 64 * (MODE == UP ? 4 : 1);
+    const dim3 grid(rows * (N / (16 * NT)));
+    if (a.act) hipLaunchKernelGGL((k_conv2<true, MODE, C, N, DIN, NT>), grid, dim3(256), 0, net->stream, a);
+    else hipLaunchKernelGGL((k_conv2<false, MODE, C, N, DIN, NT>), grid, dim3(256), 0, net->stream, a);
+    NCHK(hipGetLastError());
+    return rows;
+}
+static int conv_first(pgf_net* net, const ConvArgs& a) { return conv3<IN_CH, 16, GRID, 4>(net, a); }
+static int conv_fine(pgf_net* net, const ConvArgs& a) { return conv3<16, 16, GRID, 4>(net, a); }
+static int conv_mid(pgf_net* net, const ConvArgs& a) { return conv3<32, 32, GRID / 2, 4>(net, a); }
+static int conv_coarse(pgf_net* net, const ConvArgs& a) { return conv3<64, 64, GRID / 4, 4>(net, a); }
+static int down_fine(pgf_net* net, const ConvArgs& a) { return conv2<DOWN, 16, 32, GRID, 2>(net, a); }
+static int down_mid(pgf_net* net, const ConvArgs& a) { return conv2<DOWN, 32, 64, GRID / 2, 1>(net, a); }
+static int up_coarse(pgf_net* net, const ConvArgs& a) { return conv2<UP, 64, 32, GRID / 4, 1>(net, a); }
+static int up_mid(pgf_net* net, const ConvArgs& a) { return conv2<UP, 32, 16, GRID / 2, 1>(net, a); }
 
 // blocks of a weight gradient: tile pairs times chunks of its stages (about 512,
 // two per CU)
@@ -580,10 +716,10 @@ static WgShape wgrad_shape(int l) {
     return {tiles, stages / per, per};
 }
 
-static void launch_wgrad(pgf_net* net, int l, const bf16* in, const bf16* g, float* gW) {
-    const LayerSpec& s = SPECS[l];
+// layer l's partials, from its input; k_wgrad_reduce adds them up
+static void launch_wgrad(pgf_net* net, int l, const bf16* in) {
     const WgShape w = wgrad_shape(l);
-    const WgArgs a{w.stages, in, g, net->part};
+    const WgArgs a{w.stages, in, net->gbf[l], net->part + net->part_off[l]};
     const dim3 grid(w.tiles * w.chunks);
     hipStream_t st = net->stream;
     switch (l) {
@@ -596,10 +732,6 @@ static void launch_wgrad(pgf_net* net, int l, const bf16* in, const bf16* g, flo
         case 6: hipLaunchKernelGGL((k_wgrad2<16, 32, GRID / 2, true>), grid, dim3(256), 0, st, a); break;
         default: hipLaunchKernelGGL((k_wgrad3<16, 16, GRID>), grid, dim3(192), 0, st, a); break;
     }
-    NCHK(hipGetLastError());
-    const int TC = taps(s.mode) * s.cin, n = s.cout * TC;
-    hipLaunchKernelGGL(k_wgrad_reduce, dim3((n + 31) / 32), dim3(256), 0, st, (const float*)net->part, w.chunks, s.cout, TC,
-                       s.cin, gW);
     NCHK(hipGetLastError());
 }
 
@@ -614,69 +746,68 @@ static void refresh_bf16(pgf_net* net) {
 }
 
 static void forward(pgf_net* net, const bf16* x) {
-    float* P = net->params;
+    auto& act = net->act;
     // a1 .. a7
-    launch_conv(net, CONV3, 8, 16, GRID, x, net->Bf[0], P + net->b_off[0], nullptr, 1, net->act[0], nullptr, nullptr);
-    launch_conv(net, DOWN, 16, 32, GRID, net->act[0], net->Bf[1], P + net->b_off[1], nullptr, 1, net->act[1], nullptr, nullptr);
-    launch_conv(net, CONV3, 32, 32, GRID / 2, net->act[1], net->Bf[2], P + net->b_off[2], nullptr, 1, net->act[2], nullptr, nullptr);
-    launch_conv(net, DOWN, 32, 64, GRID / 2, net->act[2], net->Bf[3], P + net->b_off[3], nullptr, 1, net->act[3], nullptr, nullptr);
-    launch_conv(net, CONV3, 64, 64, GRID / 4, net->act[3], net->Bf[4], P + net->b_off[4], nullptr, 1, net->act[4], nullptr, nullptr);
-    launch_conv(net, UP, 64, 32, GRID / 4, net->act[4], net->Bf[5], P + net->b_off[5], net->act[2], 1, net->act[5], nullptr, nullptr);
-    launch_conv(net, UP, 32, 16, GRID / 2, net->act[5], net->Bf[6], P + net->b_off[6], net->act[0], 1, net->act[6], nullptr, nullptr);
-    launch_conv(net, CONV3, 16, 16, GRID, net->act[6], net->Bf[7], P + net->b_off[7], nullptr, 0, nullptr, net->y, nullptr);
-}
-
-static int relu_blocks(int l) { return (int)std::min<int64_t>((act_count(l) / 4 + 255) / 256, RB_BLOCKS); }
-
-// layer l's gradient behind its ReLU (layer 7 has none): bf16 copy, FP32 where
-// a skip connection needs it, the bias gradient's partials
-static void relu_back(pgf_net* net, int l, const float* d) {
-    const int64_t n4 = act_count(l) / 4;
-    const int N = SPECS[l].cout;
-    hipLaunchKernelGGL(k_relu_back, dim3(relu_blocks(l)), dim3(256), 0, net->stream, n4, N, (const float4*)d,
-                       (const ushort4*)(l == 7 ? nullptr : net->act[l]), (float4*)net->gbuf[l], (ushort4*)net->gbf[l],
-                       net->bpart + (size_t)l * RB_BLOCKS * 64);
-    NCHK(hipGetLastError());
+    auto args = [&](int l, const bf16* in, const bf16* skip) {
+        return ConvArgs{in, net->Bf[l], l < 7 ? act[l] : nullptr, l < 7 ? nullptr : net->y, net->params + net->b_off[l],
+                        skip, l < 7, nullptr, nullptr, nullptr};
+    };
+    conv_first(net, args(0, x, nullptr));
+    down_fine(net, args(1, act[0], nullptr));
+    conv_mid(net, args(2, act[1], nullptr));
+    down_mid(net, args(3, act[2], nullptr));
+    conv_coarse(net, args(4, act[3], nullptr));
+    up_coarse(net, args(5, act[4], act[2]));
+    up_mid(net, args(6, act[5], act[0]));
+    conv_fine(net, args(7, act[6], nullptr));
 }
 
 // gradients of sum(dy . y) with respect to every parameter, dy [NVOX][16] FP32 on the device
 static void backward(pgf_net* net, const bf16* x, const float* dy) {
     float* G = net->grads;
-    // layer 7 (output conv3, no ReLU): g7 = dy
-    relu_back(net, 7, dy);
-    launch_wgrad(net, 7, net->act[6], net->gbf[7], G + net->w_off[7]);
-    // d a7 = conv3^T(g7)
-    launch_conv(net, CONV3, 16, 16, GRID, net->gbf[7], net->Bd[7], nullptr, nullptr, 0, nullptr, net->dbuf[6], nullptr);
-    relu_back(net, 6, net->dbuf[6]);  // g6 (layer 6 = up2 into a7, skip from a1)
-    launch_wgrad(net, 6, net->act[5], net->gbf[6], G + net->w_off[6]);
-    // d a6 = up2^T(g6) (down form); skip: d a1 gets g6 (fp32)
-    launch_conv(net, DOWN, 16, 32, GRID, net->gbf[6], net->Bd[6], nullptr, nullptr, 0, nullptr, net->dbuf[5], nullptr);
-    relu_back(net, 5, net->dbuf[5]);
-    launch_wgrad(net, 5, net->act[4], net->gbf[5], G + net->w_off[5]);
-    launch_conv(net, DOWN, 32, 64, GRID / 2, net->gbf[5], net->Bd[5], nullptr, nullptr, 0, nullptr, net->dbuf[4], nullptr);
-    relu_back(net, 4, net->dbuf[4]);
-    launch_wgrad(net, 4, net->act[3], net->gbf[4], G + net->w_off[4]);
-    launch_conv(net, CONV3, 64, 64, GRID / 4, net->gbf[4], net->Bd[4], nullptr, nullptr, 0, nullptr, net->dbuf[3], nullptr);
-    relu_back(net, 3, net->dbuf[3]);
-    launch_wgrad(net, 3, net->act[2], net->gbf[3], G + net->w_off[3]);
-    // d a3 = down2^T(g3) (up form) + g5 (skip into a6)
-    launch_conv(net, UP, 64, 32, GRID / 4, net->gbf[3], net->Bd[3], nullptr, nullptr, 0, nullptr, net->dbuf[2], net->gbuf[5]);
-    relu_back(net, 2, net->dbuf[2]);
-    launch_wgrad(net, 2, net->act[1], net->gbf[2], G + net->w_off[2]);
-    launch_conv(net, CONV3, 32, 32, GRID / 2, net->gbf[2], net->Bd[2], nullptr, nullptr, 0, nullptr, net->dbuf[1], nullptr);
-    relu_back(net, 1, net->dbuf[1]);
-    launch_wgrad(net, 1, net->act[0], net->gbf[1], G + net->w_off[1]);
-    // d a1 = down2^T(g1) (up form) + g6 (skip into a7)
-    launch_conv(net, UP, 32, 16, GRID / 2, net->gbf[1], net->Bd[1], nullptr, nullptr, 0, nullptr, net->dbuf[0], net->gbuf[6]);
-    relu_back(net, 0, net->dbuf[0]);
-    launch_wgrad(net, 0, x, net->gbf[0], G + net->w_off[0]);
+    auto& act = net->act;
     BiasLayers b;
+    // g7 = dy (the output layer has no ReLU)
+    b.blocks[7] = RB_BLOCKS;
+    hipLaunchKernelGGL(k_out_back, dim3(RB_BLOCKS), dim3(256), 0, net->stream, act_count(7) / 4, SPECS[7].cout,
+                       (const float4*)dy, (ushort4*)net->gbf[7], net->bpart + (size_t)7 * BIAS_PART);
+    NCHK(hipGetLastError());
+    // the gradient of layer l's output, from layer l + 1's: + that of a skip
+    // connection (FP32, of the layer it leads to), behind layer l's ReLU
+    auto args = [&](int l, const float* add) {
+        return ConvArgs{net->gbf[l + 1], net->Bd[l + 1], net->gbf[l], net->gbuf[l], nullptr, nullptr, 0, add, act[l],
+                        net->bpart + (size_t)l * BIAS_PART};
+    };
+    launch_wgrad(net, 7, act[6]);
+    b.blocks[6] = conv_fine(net, args(6, nullptr));  // layer 6: up2 into a7, skip from a1
+    launch_wgrad(net, 6, act[5]);
+    b.blocks[5] = down_fine(net, args(5, nullptr));  // up2^T, down form
+    launch_wgrad(net, 5, act[4]);
+    b.blocks[4] = down_mid(net, args(4, nullptr));
+    launch_wgrad(net, 4, act[3]);
+    b.blocks[3] = conv_coarse(net, args(3, nullptr));
+    launch_wgrad(net, 3, act[2]);
+    b.blocks[2] = up_coarse(net, args(2, net->gbuf[5]));  // down2^T, up form; skip into a6
+    launch_wgrad(net, 2, act[1]);
+    b.blocks[1] = conv_mid(net, args(1, nullptr));
+    launch_wgrad(net, 1, act[0]);
+    b.blocks[0] = up_mid(net, args(0, net->gbuf[6]));  // skip into a7
+    launch_wgrad(net, 0, x);
+    WgLayers w;
+    w.first[0] = 0;
     for (int l = 0; l < N_LAYERS; ++l) {
-        b.blocks[l] = relu_blocks(l);
-        b.N[l] = SPECS[l].cout;
+        const LayerSpec& s = SPECS[l];
+        w.chunks[l] = wgrad_shape(l).chunks;
+        w.N[l] = b.N[l] = s.cout;
+        w.TC[l] = taps(s.mode) * s.cin;
+        w.part[l] = net->part + net->part_off[l];
+        w.gW[l] = G + net->w_off[l];
+        w.first[l + 1] = w.first[l] + (s.cout * w.TC[l] + 31) / 32;
         b.gb[l] = G + net->b_off[l];
     }
-    hipLaunchKernelGGL(k_bias_reduce, dim3(N_LAYERS), dim3(256), 0, net->stream, (const float*)net->bpart, b);
+    hipLaunchKernelGGL(k_wgrad_reduce, dim3(w.first[N_LAYERS]), dim3(256), 0, net->stream, w);
+    NCHK(hipGetLastError());
+    hipLaunchKernelGGL(k_bias_reduce, dim3(N_LAYERS), dim3(1024), 0, net->stream, (const float*)net->bpart, b);
     NCHK(hipGetLastError());
 }
 
@@ -744,21 +875,24 @@ PGF_API int pgf_net_create(uint64_t seed, pgf_net** out) {
         for (int l = 0; l < N_LAYERS; ++l) {
             const LayerSpec& s = SPECS[l];
             const int T = taps(s.mode);
-            net->Bf[l] = nalloc<bf16>((size_t)T * s.cin * s.cout);
-            net->Bd[l] = nalloc<bf16>((size_t)T * s.cin * s.cout);
+            const int nf = frag_count(s.cout, T * s.cin), nd = frag_count(s.cin, T * s.cout);
+            net->Bf[l] = nalloc<bf16>(nf);
+            net->Bd[l] = nalloc<bf16>(nd);
+            // the padding stays zero
+            NCHK(hipMemsetAsync(net->Bf[l], 0, sizeof(bf16) * nf, net->stream));
+            NCHK(hipMemsetAsync(net->Bd[l], 0, sizeof(bf16) * nd, net->stream));
             net->act[l] = nalloc<bf16>(act_count(l));
-            if (l < 7) net->dbuf[l] = nalloc<float>(act_count(l));
             if (l == 5 || l == 6) net->gbuf[l] = nalloc<float>(act_count(l));  // skip connections
             net->gbf[l] = nalloc<bf16>(act_count(l));
-            part = std::max(part, (size_t)wgrad_shape(l).chunks * s.cout * (size_t)T * s.cin);
+            net->part_off[l] = part;
+            part += (size_t)wgrad_shape(l).chunks * s.cout * T * s.cin;
         }
         net->part = nalloc<float>(part);
-        net->part_size = part;
         net->x = nalloc<bf16>((size_t)NVOX * IN_CH);
         net->y = nalloc<float>((size_t)NVOX * 16);
         net->dy = nalloc<float>((size_t)NVOX * 16);
         net->lossp = nalloc<float>(NVOX / 256);
-        net->bpart = nalloc<float>((size_t)N_LAYERS * RB_BLOCKS * 64);
+        net->bpart = nalloc<float>((size_t)N_LAYERS * BIAS_PART);
         net->io = nalloc<float>((size_t)NVOX * IN_CH);
         refresh_bf16(net);
         NCHK(hipStreamSynchronize(net->stream));
