@@ -647,7 +647,7 @@ bool run_teams(pgfd::Ctx& c, const std::vector<int64_t>& sp, const double* b, do
         base += (int64_t)t.sys.size() * NR * pgft::T_N;
     }
     BCHK(hipEventRecord(ev.e[1], c.stream));
-    BCHK(hipMemcpyAsync(x, dx, sizeof(double) * nv, hipMemcpyDeviceToHost, c.stream));
+    BCHK(c.copy.down(x, dx, sizeof(double) * nv, c.stream));
     BCHK(hipMemcpyAsync(st.data(), state, sizeof(double) * base, hipMemcpyDeviceToHost, c.stream));
     BCHK(hipStreamSynchronize(c.stream));
     float ms;
@@ -917,8 +917,7 @@ PGF_API int pgf_rhs_prescribed(pgf_ctx* h, int32_t nrhs, const double* up, doubl
                            (const int32_t*)c->rowptr, (const int32_t*)c->rowsplit, (const int32_t*)c->colidx,
                            (const double*)c->K, (const double*)dup, db);
         BCHK(hipGetLastError());
-        BCHK(hipStreamSynchronize(c->stream));
-        BCHK(hipMemcpy(b, db, sizeof(double) * nrhs * nf, hipMemcpyDeviceToHost));
+        BCHK(c->copy.down(b, db, sizeof(double) * nrhs * nf, c->stream));
         (void)hipFree(dup);
         (void)hipFree(db);
         return 0;
@@ -944,8 +943,7 @@ PGF_API int pgf_reactions(pgf_ctx* h, int32_t nrhs, const double* uf, const doub
                            (const int32_t*)c->rowptr, (const int32_t*)c->colidx, (const double*)c->K, (const double*)duf,
                            (const double*)dup, dR);
         BCHK(hipGetLastError());
-        BCHK(hipStreamSynchronize(c->stream));
-        BCHK(hipMemcpy(R, dR, sizeof(double) * nrhs * np, hipMemcpyDeviceToHost));
+        BCHK(c->copy.down(R, dR, sizeof(double) * nrhs * np, c->stream));
         (void)hipFree(duf);
         (void)hipFree(dup);
         (void)hipFree(dR);

@@ -31,6 +31,7 @@
 #include <string>
 #include <vector>
 
+#include "pgf_copy.hpp"
 #include "../../../include/pgfem_learn.h"
 
 namespace pgfn {
@@ -618,6 +619,7 @@ using namespace pgfn;
 struct pgf_net {
     std::string err;
     hipStream_t stream = nullptr;
+    pgfd::HostCopy copy;
     int64_t n_params = 0;
     int64_t w_off[N_LAYERS], b_off[N_LAYERS];
     float *params = nullptr, *grads = nullptr, *adam_m = nullptr, *adam_v = nullptr;
@@ -838,6 +840,7 @@ PGF_API int pgf_net_create(uint64_t seed, pgf_net** out) {
     pgf_net* net = new pgf_net();
     int rc = nguard(nullptr, [&]() {
         NCHK(hipStreamCreateWithFlags(&net->stream, hipStreamNonBlocking));
+        NCHK(net->copy.create());
         int64_t off = 0;
         for (int l = 0; l < N_LAYERS; ++l) {
             const LayerSpec& s = SPECS[l];
@@ -917,7 +920,7 @@ PGF_API int pgf_net_num_params(pgf_net* net, int64_t* n) {
 
 PGF_API int pgf_net_get_params(pgf_net* net, float* w) {
     if (!net || !w) return PGF_EARG;
-    return nguard(net, [&]() { NCHK(hipMemcpy(w, net->params, sizeof(float) * net->n_params, hipMemcpyDeviceToHost)); });
+    return nguard(net, [&]() { NCHK(net->copy.down(w, net->params, sizeof(float) * net->n_params, net->stream)); });
 }
 
 PGF_API int pgf_net_set_params(pgf_net* net, const float* w) {
@@ -936,8 +939,7 @@ PGF_API int pgf_net_forward(pgf_net* net, const float* x, float* y) {
         forward(net, net->x);
         hipLaunchKernelGGL(k_pick_out, dim3(NVOX / 256), dim3(256), 0, net->stream, (const float*)net->y, net->io);
         NCHK(hipGetLastError());
-        NCHK(hipMemcpyAsync(y, net->io, sizeof(float) * NVOX * OUT_CH, hipMemcpyDeviceToHost, net->stream));
-        NCHK(hipStreamSynchronize(net->stream));
+        NCHK(net->copy.down(y, net->io, sizeof(float) * NVOX * OUT_CH, net->stream));
     });
 }
 
@@ -950,8 +952,7 @@ PGF_API int pgf_net_backward(pgf_net* net, const float* x, const float* dy, floa
         hipLaunchKernelGGL(k_widen_out, dim3(NVOX / 64), dim3(256), 0, net->stream, (const float*)net->io, net->dy);
         NCHK(hipGetLastError());
         backward(net, net->x, net->dy);
-        NCHK(hipMemcpyAsync(grads, net->grads, sizeof(float) * net->n_params, hipMemcpyDeviceToHost, net->stream));
-        NCHK(hipStreamSynchronize(net->stream));
+        NCHK(net->copy.down(grads, net->grads, sizeof(float) * net->n_params, net->stream));
     });
 }
 

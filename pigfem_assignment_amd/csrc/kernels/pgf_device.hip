@@ -755,6 +755,7 @@ PGF_API int pgf_create(const pgf_mesh_desc* d, pgf_ctx** out) {
         c->nnz_ff = 0;
         for (int64_t r = 0; r < d->n_free; ++r) c->nnz_ff += pat.rowsplit[r];
         HIPCHK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
+        HIPCHK(c->copy.create());
         // ---- elements in colour order ----
         std::vector<int64_t> ucount(pat.n_colors + 1, 0), ccount(pat.n_colors + 1, 0);
         for (int64_t e = 0; e < d->n_elem; ++e) {
@@ -1219,8 +1220,7 @@ PGF_API int pgf_volume_average_noalloc(pgf_ctx* c, const double* eps_bar, int32_
 PGF_API int pgf_get_solution(pgf_ctx* c, double* u) {
     if (!c || !u) return PGF_EARG;
     return guard(c, [&]() -> int {
-        HIPCHK(hipMemcpyAsync(u, c->U, sizeof(double) * c->dim * c->n_all, hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(hipStreamSynchronize(c->stream));
+        HIPCHK(c->copy.down(u, c->U, sizeof(double) * c->dim * c->n_all, c->stream));
         return 0;
     });
 }
@@ -1262,21 +1262,21 @@ PGF_API int pgf_assemble(pgf_ctx* c, double dt, uint32_t flags) {
 PGF_API int pgf_get_matrix(pgf_ctx* c, double* vals) {
     if (!c || !vals) return PGF_EARG;
     return guard(c, [&]() -> int {
-        HIPCHK(hipMemcpy(vals, c->K, sizeof(double) * c->nnz, hipMemcpyDeviceToHost));
+        HIPCHK(c->copy.down(vals, c->K, sizeof(double) * c->nnz, c->stream));
         return 0;
     });
 }
 PGF_API int pgf_get_matrix32(pgf_ctx* c, float* vals) {
     if (!c || !vals) return PGF_EARG;
     return guard(c, [&]() -> int {
-        HIPCHK(hipMemcpy(vals, c->K32, sizeof(float) * c->nnz, hipMemcpyDeviceToHost));
+        HIPCHK(c->copy.down(vals, c->K32, sizeof(float) * c->nnz, c->stream));
         return 0;
     });
 }
 PGF_API int pgf_get_internal_force(pgf_ctx* c, double* p) {
     if (!c || !p) return PGF_EARG;
     return guard(c, [&]() -> int {
-        HIPCHK(hipMemcpy(p, c->P, sizeof(double) * c->n_rows, hipMemcpyDeviceToHost));
+        HIPCHK(c->copy.down(p, c->P, sizeof(double) * c->n_rows, c->stream));
         return 0;
     });
 }
@@ -1310,9 +1310,9 @@ PGF_API int pgf_get_isv(pgf_ctx* c, double* dt, double* dc, uint8_t* fl) {
     if (!c) return PGF_EARG;
     return guard(c, [&]() -> int {
         if (c->n_cpt) {
-            if (dt) HIPCHK(hipMemcpy(dt, c->dmax_trial, sizeof(double) * c->n_cpt, hipMemcpyDeviceToHost));
-            if (dc) HIPCHK(hipMemcpy(dc, c->dmax_conv, sizeof(double) * c->n_cpt, hipMemcpyDeviceToHost));
-            if (fl) HIPCHK(hipMemcpy(fl, c->flags, c->n_cpt, hipMemcpyDeviceToHost));
+            if (dt) HIPCHK(c->copy.down(dt, c->dmax_trial, sizeof(double) * c->n_cpt, c->stream));
+            if (dc) HIPCHK(c->copy.down(dc, c->dmax_conv, sizeof(double) * c->n_cpt, c->stream));
+            if (fl) HIPCHK(c->copy.down(fl, c->flags, c->n_cpt, c->stream));
         }
         return 0;
     });
@@ -1334,8 +1334,7 @@ PGF_API int pgf_spmv(pgf_ctx* c, const double* x, double* y) {
         HIPCHK(hipMemcpyAsync(c->x, x, sizeof(double) * c->n_free, hipMemcpyHostToDevice, c->stream));
         pgfd::enqueue_spmv<double, double>(*c, c->K, c->x, c->q);
         HIPCHK(hipGetLastError());
-        HIPCHK(hipMemcpyAsync(y, c->q, sizeof(double) * c->n_free, hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(hipStreamSynchronize(c->stream));
+        HIPCHK(c->copy.down(y, c->q, sizeof(double) * c->n_free, c->stream));
         return 0;
     });
 }
@@ -1353,7 +1352,7 @@ PGF_API int pgf_pcg(pgf_ctx* c, const double* b, double* x, const double* x0, do
         if (precision == 32) pgfd::run_pcg<float>(*c, c->K32, c->res, x0 != nullptr, rtol, maxit, &si);
         else pgfd::run_pcg<double>(*c, c->K, c->res, x0 != nullptr, rtol, maxit, &si);
         if (info) *info = si;
-        HIPCHK(hipMemcpy(x, c->x, sizeof(double) * n, hipMemcpyDeviceToHost));
+        HIPCHK(c->copy.down(x, c->x, sizeof(double) * n, c->stream));
         return 0;
     });
 }

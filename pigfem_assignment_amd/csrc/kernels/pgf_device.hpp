@@ -6,6 +6,7 @@
 #include <string>
 #include <vector>
 
+#include "pgf_copy.hpp"
 #include "pgf_kernels.hpp"
 #include "pgf_team.hpp"
 
@@ -18,6 +19,7 @@ struct LearnState;  // learned initial guess state (pgf_cnn.hip)
 struct Ctx {
     std::string err;
     hipStream_t stream = nullptr;
+    HostCopy copy;
     int dim = 0, kind = 0, n_colors = 0;
     double tet_scale = 1.0;
     int64_t n_nodes = 0, n_all = 0, n_elem = 0, n_uncut = 0, n_cut = 0, n_free = 0, n_pres = 0, n_rows = 0,
