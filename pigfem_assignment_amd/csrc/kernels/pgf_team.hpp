@@ -12,7 +12,8 @@
 //    reads all slots until none is empty and adds them in slot order, so every
 //    block has the same total and takes the same decisions.  No
 //    read-modify-write: a single arrival counter costs ~60 ns per block on one
-//    line (15 us at 256 blocks); this exchange takes 2.0 to 2.6 us.
+//    line (15 us at 256 blocks); this exchange takes 1.6 us with 79 blocks, 2.1
+//    to 2.7 with 240.
 //  * "empty" is a NaN pattern no sum is published as.  Slots rotate over three
 //    buffers: a block empties its slot of the buffer after next right after it
 //    has read a sum, when every block has left the sum that last used it.
@@ -53,7 +54,7 @@
 namespace pgft {
 
 constexpr int TT = TEAM_THREADS;                  // 512: 256 registers a lane for K entries
-constexpr int MAX_TEAM = 256;                     // blocks per team (four slots per lane of the reading wavefront)
+constexpr int MAX_TEAM = 256;                     // blocks per team (one pass of loads for one or two values)
 constexpr unsigned long long EMPTY = ~0ull;       // slot not yet published
 constexpr unsigned long long WAIT_TICKS = 2000000000ull;  // 20 s of the 100 MHz wall clock
 constexpr size_t LDS_MAX = 158 * 1024;            // dynamic LDS a block may take (160 KiB less the static part)
@@ -130,8 +131,9 @@ __device__ inline void slot_store(unsigned long long* p, unsigned long long v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// ---- sums over consecutive lanes by data-parallel primitives (every lane
-// gets the sum): lanes ^1, ^2, 7 - i, 15 - i of a row of 16
+// ---- sums over lanes without LDS.  By data-parallel primitives: lanes ^1,
+// ^2, 7 - i, 15 - i of a row of 16 (every lane gets the sum), ^4, ^8; by
+// exchange of rows and halves: 16 and 32 apart.
 template <int CTRL>
 __device__ inline double dpp(double v) {
     const long long u = __double_as_longlong(v);
@@ -147,11 +149,51 @@ __device__ inline double lane_sum(double v) {
     if (G >= 16) v += dpp<0x140>(v);
     return v;
 }
-__device__ inline double wave_sum(double v) {
-    v = lane_sum<16>(v);
-    v += __shfl_xor(v, 16, 64);
-    v += __shfl_xor(v, 32, 64);
-    return v;
+__device__ inline double xor4(double v) { return dpp<0x1B>(dpp<0x141>(v)); }
+__device__ inline double xor8(double v) { return dpp<0x128>(v); }
+// even rows (halves) get the sum of a, odd ones that of b, over the two
+template <int APART>
+__device__ inline double swap_add(double a, double b) {
+    const unsigned long long ua = __double_as_longlong(a), ub = __double_as_longlong(b);
+    auto swap = [](unsigned x, unsigned y) {
+        if constexpr (APART == 16) return __builtin_amdgcn_permlane16_swap(x, y, false, false);
+        else return __builtin_amdgcn_permlane32_swap(x, y, false, false);
+    };
+    const auto lo = swap((unsigned)ua, (unsigned)ub), hi = swap((unsigned)(ua >> 32), (unsigned)(ub >> 32));
+    return __longlong_as_double((long long)((unsigned long long)hi[0] << 32 | lo[0])) +
+           __longlong_as_double((long long)((unsigned long long)hi[1] << 32 | lo[1]));
+}
+constexpr int padded(int nv) { return nv <= 2 ? nv : nv <= 4 ? 4 : 8; }
+// sums of v[0..NV) over the wavefront: every lane gets that of value
+// lane / (64 / padded(NV)).  Each exchange halves the values a lane carries:
+// 10 additions for 6 values, not 36, and no step through LDS (333 x 333 quads
+// 9.3 -> 8.3 us per iteration, 64^3 x 6 tets 96 -> 94.7, with the loads below).
+template <int NV>
+__device__ inline double wave_sums(const double (&v)[NV]) {
+    constexpr int VP = padded(NV);
+    double w[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) w[k] = k < NV ? v[k] : 0.0;
+    if (VP == 8)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) w[k] = swap_add<32>(w[k], w[k + 4]);
+    else if (VP == 4)
+#pragma unroll
+        for (int k = 0; k < 2; ++k) w[k] = swap_add<32>(w[k], w[k + 2]);
+    else
+        w[0] = swap_add<32>(w[0], w[VP - 1]);
+    if (VP == 8)
+#pragma unroll
+        for (int k = 0; k < 2; ++k) w[k] = swap_add<16>(w[k], w[k + 2]);
+    else
+        w[0] = swap_add<16>(w[0], w[VP == 4 ? 1 : 0]);
+    if (VP == 8) {
+        const bool odd = threadIdx.x & 8;
+        w[0] = (odd ? w[1] : w[0]) + xor8(odd ? w[0] : w[1]);
+    } else {
+        w[0] += xor8(w[0]);
+    }
+    return lane_sum<8>(w[0]);
 }
 
 // a value all lanes agree on, in scalar registers
@@ -164,13 +206,13 @@ __device__ inline double uniform(double v) {
 // One block's end of the team's sums.
 template <int NR>
 struct TeamSum {
-    static constexpr int W = slot_values<NR>(), TW = TT / 64;
-    static_assert(TW <= 16, "one row of lanes adds the wavefronts");
+    static constexpr int TW = TT / 64;
+    static_assert(TW == 8 && COPIES == 8 && SLOT == 8, "eight lanes add the wavefronts, publish and empty a value");
     unsigned long long* slots;  // this team's [COPIES][3][nb][SLOT]
     int nb, me, copy;
     unsigned phase;
-    double (*red)[W];           // [16][W] LDS, rows from TW on zero
-    double* tot;                // [W] LDS
+    double (*red)[SLOT];        // [TW][SLOT] LDS
+    double* tot;                // [SLOT] LDS
     int* bad;                   // LDS: the team gave up
     int* abort;
 
@@ -179,83 +221,89 @@ struct TeamSum {
     // the first run `meanwhile`.
     template <int NV, typename F>
     __device__ bool operator()(double (&v)[NV], bool publish, F&& meanwhile) {
-        const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-#pragma unroll
-        for (int k = 0; k < NV; ++k) v[k] = wave_sum(v[k]);
-        if (lane == 0)
-#pragma unroll
-            for (int k = 0; k < NV; ++k) red[w][k] = v[k];
+        constexpr int L = 64 / padded(NV);  // lanes a value has
+        int lane = threadIdx.x & 63;
+        // (kept out of the compiler's sight, which otherwise computes every
+        // address below before the iteration and spills K entries for it)
+        asm volatile("" : "+v"(lane));
+        const int w = threadIdx.x >> 6, k = lane / L, j = lane % L;
+        const double mine = wave_sums<NV>(v);
+        if (j == 0 && k < NV) red[w][k] = mine;
         // every wavefront's pairs have left it before the publication
         if (publish) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
         if (w == 0) {
-            double s[NV];
-#pragma unroll
-            for (int k = 0; k < NV; ++k) s[k] = lane_sum<16>(red[lane & 15][k]);
+            // of the block, in the first eight lanes of each value
+            const double s = lane_sum<8>(j < TW && k < NV ? red[j][k] : 0.0);
             if (nb > 1) exchange<NV>(s, lane);
-            if (lane == 0)
-#pragma unroll
-                for (int k = 0; k < NV; ++k) tot[k] = s[k];
+            else if (j == 0 && k < NV) tot[k] = s;
         } else {
             meanwhile();
         }
         __syncthreads();
 #pragma unroll
-        for (int k = 0; k < NV; ++k) v[k] = uniform(tot[k]);
+        for (int i = 0; i < NV; ++i) v[i] = uniform(tot[i]);
         return __builtin_amdgcn_readfirstlane(*bad) == 0;
     }
 
+    // One store publishes every value in every copy, and the lanes of a load
+    // read whole slots: with a load per value and 64 slots each, the sum of six
+    // values over 42 blocks took 4.1 us and that of three 2.9 (six systems of 3
+    // right-hand sides 11.2 -> 8.6 us per iteration, 32 larger ones 75.6 -> 63.6).
     template <int NV>
-    __device__ void exchange(double (&s)[NV], int lane) {
+    __device__ void exchange(double s, int lane) {
+        constexpr int VP = padded(NV), L = 64 / VP;
+        constexpr int LOADS = std::min(MAX_TEAM / L, NR == 1 ? 8 : 16);  // at a time
         const int64_t per = team_slots(nb), at = (int64_t)(phase % 3) * nb * SLOT;
         const unsigned long long* buf = slots + copy * per + at;
         // the emptied slot of the next buffer is in memory before this
         // publication, after which another block may look for it
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        if (lane < COPIES)
-#pragma unroll
-            for (int k = 0; k < NV; ++k) {
-                unsigned long long u = __double_as_longlong(s[k]);
-                if (u == EMPTY) u = 0x7ff8000000000000ull;
-                slot_store(&slots[lane * per + at + (int64_t)me * SLOT + k], u);
-            }
-        unsigned long long got[MAX_TEAM / 64][NV];
+        if (lane % L < COPIES && lane / L < NV) {
+            unsigned long long u = __double_as_longlong(s);
+            if (u == EMPTY) u = 0x7ff8000000000000ull;
+            slot_store(&slots[lane % L * per + at + (int64_t)me * SLOT + lane / L], u);
+        }
+        // value lane % VP of blocks lane / VP, + L, ...
+        const int k = lane % VP;
+        const uint32_t mine = lane / VP * SLOT + k;
+        double sum = 0.0;
         const unsigned long long t0 = wall_clock64();
-        for (unsigned round = 0;; ++round) {
-            bool all = true;
+        for (int m0 = 0; m0 < nb; m0 += LOADS * L) {
+            unsigned long long got[LOADS];
+            for (unsigned round = 0;; ++round) {
+                bool all = true;
 #pragma unroll
-            for (int i = 0; i < MAX_TEAM / 64; ++i) {
-                const int m = lane + 64 * i;
-#pragma unroll
-                for (int k = 0; k < NV; ++k) got[i][k] = m < nb ? slot_load(&buf[(size_t)m * SLOT + k]) : 0ull;
-            }
-#pragma unroll
-            for (int i = 0; i < MAX_TEAM / 64; ++i)
-#pragma unroll
-                for (int k = 0; k < NV; ++k) all = all && got[i][k] != EMPTY;
-            if (__all(all)) break;
-            if ((round & 255u) == 255u && wall_clock64() - t0 > WAIT_TICKS) {
-                if (lane == 0) {
-                    *bad = 1;
-                    __hip_atomic_store(abort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                for (int i = 0; i < LOADS; ++i) {
+                    got[i] = 0ull;
+                    const int m = m0 + i * L;  // (of the wavefront)
+                    if (m < nb && m + lane / VP < nb && k < NV) got[i] = slot_load(buf + m * SLOT + mine);
                 }
-                break;
+#pragma unroll
+                for (int i = 0; i < LOADS; ++i) all = all && got[i] != EMPTY;
+                if (__all(all)) break;
+                if ((round & 255u) == 255u && wall_clock64() - t0 > WAIT_TICKS) {
+                    if (lane == 0) {
+                        *bad = 1;
+                        __hip_atomic_store(abort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    }
+                    break;
+                }
             }
+#pragma unroll
+            for (int i = 0; i < LOADS; ++i) sum += __longlong_as_double((long long)got[i]);
         }
         // nothing after this is read before the slots were
         asm volatile("" ::: "memory");
-#pragma unroll
-        for (int k = 0; k < NV; ++k) {
-            double a = 0.0;
-#pragma unroll
-            for (int i = 0; i < MAX_TEAM / 64; ++i) a += __longlong_as_double(got[i][k]);
-            s[k] = wave_sum(a);
-        }
-        if (lane < COPIES) {
-            unsigned long long* nxt = slots + lane * per + ((int64_t)((phase + 2) % 3) * nb + me) * SLOT;
-#pragma unroll
-            for (int k = 0; k < W; ++k) slot_store(&nxt[k], EMPTY);
-        }
+        if (VP == 1) sum += dpp<0xB1>(sum);
+        if (VP <= 2) sum += dpp<0x4E>(sum);
+        if (VP <= 4) sum += xor4(sum);
+        sum += xor8(sum);
+        sum = swap_add<16>(sum, sum);
+        sum = swap_add<32>(sum, sum);
+        if (lane < NV) tot[lane] = sum;
+        // all values of this block's next slot but one, in all copies
+        slot_store(&slots[lane / SLOT * per + ((int64_t)((phase + 2) % 3) * nb + me) * SLOT + lane % SLOT], EMPTY);
         ++phase;
     }
 };
@@ -281,7 +329,7 @@ __global__ __launch_bounds__(TT) void k_team_pcg(TeamArgs<TA> a) {
     constexpr int RB = ALL ? 1 : 4;  // rows per trip: operands in memory want several on the way
     constexpr int W = slot_values<NR>();
     extern __shared__ __align__(16) unsigned char s_dyn[];
-    __shared__ double s_red[16][W], s_tot[W];
+    __shared__ double s_red[TT / 64][SLOT], s_tot[SLOT];
     __shared__ int s_bad;
     const int t = threadIdx.x, sub = t % G;
     int team = blockIdx.x % a.n_teams, me = blockIdx.x / a.n_teams;
@@ -290,7 +338,6 @@ __global__ __launch_bounds__(TT) void k_team_pcg(TeamArgs<TA> a) {
     if (a.n_teams == 1 && a.team_blocks % 8 == 0) me = (blockIdx.x % 8) * (a.team_blocks / 8) + blockIdx.x / 8;
     TeamSum<NR> sum{a.slots + team * COPIES * team_slots(a.team_blocks), a.team_blocks, me,
                     (int)(blockIdx.x % COPIES), 0u, s_red, s_tot, &s_bad, a.abort};
-    if (t < 16 * W) (&s_red[0][0])[t] = 0.0;
     if (t == 0) s_bad = 0;
     __syncthreads();
     const __amdgpu_buffer_rsrc_t zrs =
