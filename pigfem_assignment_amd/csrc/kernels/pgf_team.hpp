@@ -356,11 +356,17 @@ __global__ __launch_bounds__(TT) void k_team_pcg(TeamArgs<TA> a) {
         const int nh = (int)(a.halo_ptr[share + 1] - h0);
         const int nw = nrow + nh;
         // LDS: p of the window by right-hand side [NR][nw], then q (z from the
-        // update on) and r [NR][nrow], 1/diag [nrow]
+        // update on) and r [NR][nrow], 1/diag [nrow]; the halo's columns [nh]
+        // where K is in registers
         double* Lp = (double*)s_dyn;
         double* Lq = Lp + (size_t)nw * NR;
         double* Lr = Lq + (size_t)nrow * NR;
         double* Ld = Lr + (size_t)nrow * NR;
+        uint32_t* Lh = (uint32_t*)(Ld + nrow);
+        if (KEEP > 0) {
+            for (int i = t; i < nh; i += TT) Lh[i] = (uint32_t)a.halo[h0 + i];
+            __syncthreads();
+        }
         double* xg = a.x + row0;
         double* rg = a.r + row0;
         const double2* zg = a.zp + row0;
@@ -475,7 +481,10 @@ __global__ __launch_bounds__(TT) void k_team_pcg(TeamArgs<TA> a) {
                 uint32_t col[HB];
                 double2 e[HB][NR];
 #pragma unroll
-                for (int k = 0; k < HB; ++k) col[k] = (uint32_t)a.halo[h0 + min(i0 + k * TT, nh - 1)];
+                for (int k = 0; k < HB; ++k) {
+                    const int i = min(i0 + k * TT, nh - 1);
+                    col[k] = KEEP > 0 ? Lh[i] : (uint32_t)a.halo[h0 + i];
+                }
 #pragma unroll
                 for (int k = 0; k < HB; ++k)
 #pragma unroll
@@ -809,22 +818,26 @@ struct TeamShape {
 // The kernel for the plan's largest share: everything in LDS and K in registers
 // where it fits, then K streamed, then r and 1/diag in memory.  us per
 // iteration of a single solve, against five launches:
-//   K in registers: 100 x 100 quads 6.0 (21.3), 333 x 333 9.2 (34.3),
-//     40^3 x 6 tets with FP32 values 12.4 (40.7);
-//   streamed: 460 x 460 quads 21.3 (49.4), 50^3 x 6 tets 36.4 (70.0);
-//   r and 1/diag in memory: 64^3 x 6 tets 96 (159), 700 x 700 quads 44.5 (93.6).
+//   K in registers: 100 x 100 quads 5.3 (21.3), 333 x 333 8.3 (34.3),
+//     40^3 x 6 tets with FP32 values 11.7 (40.7);
+//   streamed: 460 x 460 quads 20.2 (49.4), 50^3 x 6 tets 34.6 (70.0);
+//   r and 1/diag in memory: 64^3 x 6 tets 94.5 (159), 700 x 700 quads 43.6 (93.6).
+// The halo's columns in LDS, beside K in registers, are 3 to 5 % of an iteration
+// (100 x 100 quads 5.51 -> 5.32, 333 x 333 8.66 -> 8.26, 20^3 x 6 tets 7.22 ->
+// 6.94); fetched ahead into registers they cost spills (8 columns a lane: 6.1,
+// 9.1, 8.2).
 // A window beyond the LDS was tried with gathers through the L2 and fences:
 // 1000 x 1000 quads 212 (196), 80^3 x 6 tets 297 (279): those keep the launches.
 template <typename TA, int NR, int DIM>
 TeamShape team_shape(const TeamPlan& p) {
     const size_t win = sizeof(double) * NR * (size_t)p.max_window, row = sizeof(double) * (size_t)p.max_rows;
-    const size_t all = win + row * (2 * NR + 1), pq = win + row * NR;
+    const size_t all = win + row * (2 * NR + 1), pq = win + row * NR, halo = sizeof(uint32_t) * (size_t)p.max_window;
     constexpr int K = max_keep<TA, NR, DIM>();
     TeamShape s;
     if (p.max_window > MAX_WINDOW || pq > LDS_MAX) return s;
     if (all > LDS_MAX) s = {reinterpret_cast<const void*>(&k_team_pcg<TA, NR, DIM, WIN_PQ, 0>), (unsigned)pq};
-    else if (p.max_passes > K) s = {reinterpret_cast<const void*>(&k_team_pcg<TA, NR, DIM, WIN_ALL, 0>), (unsigned)all};
-    else s = {reinterpret_cast<const void*>(&k_team_pcg<TA, NR, DIM, WIN_ALL, K>), (unsigned)all};
+    else if (p.max_passes > K || all + halo > LDS_MAX) s = {reinterpret_cast<const void*>(&k_team_pcg<TA, NR, DIM, WIN_ALL, 0>), (unsigned)all};
+    else s = {reinterpret_cast<const void*>(&k_team_pcg<TA, NR, DIM, WIN_ALL, K>), (unsigned)(all + halo)};
     return s;
 }
 
