@@ -532,22 +532,25 @@ def bench_c3(args):
     F = batch.macro_strain_rhs(ctx, B)
     ctx.assemble(L.PGF_ASM_JAC)
     X, its, rel, ms_solve, tune = ctx.batch_pcg(B.sys_ptr, F, rtol=1e-8)
-    print("# C3 batched PCG (graph replays): %.1f ms" % ms_solve, flush=True)
+    print("# C3 batched PCG: %.1f ms" % ms_solve, flush=True)
     ms_persist, same = None, None
     if args.c3_persistent:
-        # the same solve as one persistent cooperative launch (bit-identical)
+        # an explicit layout by graph replays and as one persistent
+        # cooperative launch (bit-identical)
         try:
-            Xp, itp, _, ms_persist, _ = ctx.batch_pcg(B.sys_ptr, F, rtol=1e-8, tune=tune, persistent=True)
-            same = bool(np.array_equal(Xp, X) and np.array_equal(itp, its))
-            del Xp
+            lay = (8, 512)
+            Xg, itg, _, ms_graph, _ = ctx.batch_pcg(B.sys_ptr, F, rtol=1e-8, tune=lay)
+            Xp, itp, _, ms_persist, _ = ctx.batch_pcg(B.sys_ptr, F, rtol=1e-8, tune=lay, persistent=True)
+            same = bool(np.array_equal(Xp, Xg) and np.array_equal(itp, itg))
+            del Xp, Xg
             print("# C3 batched PCG as one persistent launch: %.1f ms (graph replays %.1f ms), identical results %s"
-                  % (ms_persist, ms_solve, same), flush=True)
+                  % (ms_persist, ms_graph, same), flush=True)
         except RuntimeError as e:
             print("# C3 persistent launch refused: %s" % e, flush=True)
     Ce = batch.homogenized_stiffness(ctx, B, X, B.elem_ptr)
     print("# C3 assembly %.2f ms (%.3e elem/s); batched PCG 3 cases x %d RVEs: %.1f ms, iterations %d..%d, "
-          "tuned (threads/row, rows/tile) %s" % (ms_asm, B.n_elem / (ms_asm * 1e-3), len(parts), ms_solve,
-                                                 its.min(), its.max(), tune), flush=True)
+          "layout (threads/row, rows/tile; 0, 0: resident teams) %s" % (ms_asm, B.n_elem / (ms_asm * 1e-3), len(parts),
+                                                                       ms_solve, its.min(), its.max(), tune), flush=True)
     extra = {"batched_solve_ms": ms_solve, "batched_solve_persistent_ms": ms_persist,
              "persistent_equals_graph": same, "iterations_min": int(its.min()), "iterations_max": int(its.max()),
              "iterations_total": int(its.sum()), "autotuned": list(tune), "gather_layout": slots,

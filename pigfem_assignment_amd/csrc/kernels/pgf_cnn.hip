@@ -4,11 +4,12 @@
 // with this file's own kernels.
 //
 //  * every convolution is an implicit GEMM on bf16 MFMA tiles
-//    (v_mfma_f32_16x16x16bf16_1k, FP32 accumulation), one wavefront per
-//    16-position x 16*NT-channel output tile;
-//  * activations are stored channels-last in bf16; gradients are FP32 with a
-//    bf16 copy as MFMA operand; weights are FP32 masters with bf16 copies per
-//    step (forward layout [Cout][T*Cin], data-gradient layout [Cin][T*Cout]);
+//    (v_mfma_f32_16x16x16bf16_1k, FP32 accumulation);
+//  * activations are stored channels-last in bf16; gradients leave their FP32
+//    sums behind the ReLU mask as bf16 MFMA operands, FP32 where a skip
+//    connection adds them on; weights are FP32 masters with bf16 copies per
+//    step in fragment order (forward matrix [Cout][T*Cin], data-gradient matrix
+//    [Cin][T*Cout]);
 //  * Adam in FP32.
 //
 // Layers (64^3 x 8 input):
