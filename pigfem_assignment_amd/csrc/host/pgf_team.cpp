@@ -2,6 +2,7 @@
 #include "pgf_team.hpp"
 
 #include <algorithm>
+#include <exception>
 #include <omp.h>
 
 namespace pgft {
@@ -43,12 +44,15 @@ bool make_team_plan(int dim, const std::vector<GroupRec>& grp, const std::vector
     std::vector<std::vector<int32_t>> found(n_shares);
     std::vector<std::vector<StepRec>> steps(n_shares);
     int rows = 0, passes = 0, window = 0;
+    // an exception must not leave a parallel region: the first is thrown on behind it
+    std::exception_ptr failed;
 #pragma omp parallel num_threads(std::min(omp_get_max_threads(), 16)) reduction(max : rows, passes, window)
     {
         // the share that last met each column of its system, per thread
-        std::vector<int32_t> seen((size_t)sys_rows, -1);
+        std::vector<int32_t> seen;
 #pragma omp for schedule(dynamic, 4)
-        for (int k = 0; k < n_shares; ++k) {
+        for (int k = 0; k < n_shares; ++k) try {
+            if (seen.empty()) seen.assign((size_t)sys_rows, -1);
             const int32_t* pt = &plan.part[(size_t)(k / blocks) * (blocks + 1) + k % blocks];
             const int32_t r0 = grp[pt[0]].row, r1 = grp[pt[1]].row, first = grp[sys[k / blocks].lo].row;
             rows = std::max(rows, r1 - r0);
@@ -88,8 +92,12 @@ bool make_team_plan(int dim, const std::vector<GroupRec>& grp, const std::vector
             std::sort(h.begin(), h.end());
             share_window[k] = r1 - r0 + (int32_t)h.size();
             window = std::max(window, share_window[k]);
+        } catch (...) {
+#pragma omp critical(pgf_team_plan)
+            if (!failed) failed = std::current_exception();
         }
     }
+    if (failed) std::rethrow_exception(failed);
     plan.max_rows = rows;
     plan.max_passes = passes;
     plan.max_window = window;

@@ -556,8 +556,9 @@ bool make_batch_teams(pgfd::Ctx& c, const std::vector<int64_t>& sp) {
         if (plan(small, stage[0], t)) take(t);
     }
     if (!left.empty()) return false;
+    std::vector<int64_t> key = sp;  // (may throw: before the teams change)
     c.batch_teams = std::move(teams);
-    c.batch_sys = sp;
+    c.batch_sys.swap(key);
     c.batch_nrhs = NR;
     return true;
 }
@@ -999,6 +1000,9 @@ static int batch_pcg(pgf_ctx* h, int32_t n_sys, const int64_t* sys_ptr, int32_t 
         c->err = e;
         if (e.rfind("persistent", 0) == 0) return PGF_EUNSUPPORTED;
         return e.rfind("HIP", 0) == 0 ? PGF_EDEVICE : PGF_EARG;
+    } catch (const std::exception& e) {  // the context's allocations, host memory
+        c->err = e.what();
+        return PGF_EDEVICE;
     }
 }
 
