@@ -475,11 +475,20 @@ pgft::TeamShape batch_shape(int dim, const pgft::TeamPlan& p) {
 // and so on.  (32 RVEs of 64 to 160 divisions, three right-hand sides: 222 ms
 // with three of them in a second launch, 200 ms with all in one of seven teams;
 // launches with tuned tiles 382 ms.)  Systems are dealt to the teams longest first.  False if
-// some system fits no team.
+// some system fits no team; the context remembers that for the last such
+// ranges, and keeps what it has laid out for others.
 template <int NR>
 bool make_batch_teams(pgfd::Ctx& c, const std::vector<int64_t>& sp) {
     if (!c.batch_teams.empty() && c.batch_nrhs == NR && c.batch_sys == sp) return true;
-    c.batch_teams.clear();
+    if (c.unfit_nrhs >> NR & 1 && c.unfit_sys == sp) return false;
+    auto unfit = [&] {
+        if (c.unfit_sys != sp) {
+            c.unfit_nrhs = 0;
+            c.unfit_sys = sp;
+        }
+        c.unfit_nrhs |= 1u << NR;
+        return false;
+    };
     const int n_sys = (int)sp.size() - 1, lg = pgft::TEAM_THREADS / pgft::team_lanes(c.dim);
     std::vector<pgft::SysGroups> grp(n_sys);
     std::vector<int32_t> left;
@@ -489,7 +498,7 @@ bool make_batch_teams(pgfd::Ctx& c, const std::vector<int64_t>& sp) {
                                     [](const pgft::GroupRec& g, int64_t r) { return g.row < r; });
         };
         const auto lo = at(sp[s]), hi = at(sp[s + 1]);
-        if (lo->row != sp[s] || hi->row != sp[s + 1]) return false;  // a row group across two systems
+        if (lo->row != sp[s] || hi->row != sp[s + 1]) return unfit();  // a row group across two systems
         grp[s] = {lo - c.h_grp.begin(), hi - c.h_grp.begin()};
         if (sp[s + 1] > sp[s]) left.push_back(s);
     }
@@ -540,6 +549,19 @@ bool make_batch_teams(pgfd::Ctx& c, const std::vector<int64_t>& sp) {
         left.swap(rest);
         teams.push_back(std::move(t));
     };
+    // One system that fits no team takes the batch to the launches, so where the
+    // largest may be one (more rows than half of what a team of the smallest
+    // size holds) it is tried alone on all CUs before anything else: planning
+    // every team for 31 cells of 64 to 94 and one of 520 first made each call
+    // 308 ms, against 289 without teams.
+    const int32_t big = left.empty() ? 0 : *std::max_element(left.begin(), left.end(), [&](int32_t a, int32_t b) {
+        return grp[a].hi - grp[a].lo < grp[b].hi - grp[b].lo;
+    });
+    if (!left.empty() && 2 * (sp[big + 1] - sp[big]) > fit * std::max(c.n_cu / 8, 1)) {
+        pgft::Team t;
+        if (!plan({big}, 1, t)) return unfit();
+    }
+    c.batch_teams.clear();
     static const std::vector<int> stages[] = {{8, 7, 6, 5}, {4, 3}, {2}, {1}};
     for (const std::vector<int>& stage : stages) {
         if (left.empty()) break;
@@ -555,7 +577,7 @@ bool make_batch_teams(pgfd::Ctx& c, const std::vector<int64_t>& sp) {
         pgft::Team t;
         if (plan(small, stage[0], t)) take(t);
     }
-    if (!left.empty()) return false;
+    if (!left.empty()) return unfit();
     std::vector<int64_t> key = sp;  // (may throw: before the teams change)
     c.batch_teams = std::move(teams);
     c.batch_sys.swap(key);
@@ -972,8 +994,8 @@ static int batch_pcg(pgf_ctx* h, int32_t n_sys, const int64_t* sys_ptr, int32_t 
             if (sp[s + 1] < sp[s]) throw std::string("system ranges must be ascending");
         // the free-free block must be block diagonal over these ranges
         // (the rows of a group have one column list; ranges that the context
-        // laid its teams out for were found block diagonal then)
-        if (c->batch_sys != sp) {
+        // has tried to lay teams out for were found block diagonal then)
+        if (c->batch_sys != sp && c->unfit_sys != sp) {
             int s = 0;
             for (int64_t g = 0; g < c->n_grp; ++g) {
                 const pgft::GroupRec& gr = c->h_grp[g];

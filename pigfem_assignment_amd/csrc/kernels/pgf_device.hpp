@@ -95,6 +95,10 @@ struct Ctx {
     std::vector<pgft::Team> batch_teams;
     std::vector<int64_t> batch_sys;
     int batch_nrhs = 0;
+    // the last ranges with a system that fits no team, for these numbers of
+    // right-hand sides (bit n: n of them)
+    std::vector<int64_t> unfit_sys;
+    unsigned unfit_nrhs = 0;
     int n_cu = 0;
     double* partial = nullptr;     // block partial sums
     double* scal = nullptr;        // device scalars: PCG state (pgft::T_N), residual norm

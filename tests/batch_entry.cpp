@@ -1,8 +1,12 @@
 // Calls pgf_batch_pcg where no GPU is visible, on a context made by hand: what
-// the C entry does when memory of the host or the device runs out.
+// the C entry does when memory of the host or the device runs out, and what it
+// does again on a repeated call.
 //   batch_entry workspace        teams laid out already, the solve's device memory fails
 //   batch_entry plan BYTES       one system of 400 x 400 rows, host blocks of BYTES or more fail
-// Prints the status, or dies of an exception that leaves the entry.
+//   batch_entry unfit            a system of 800 x 800 rows, four right-hand sides: fits no team; twice
+// Prints the status and the host bytes that each call allocated, or dies of an
+// exception that leaves the entry.
+#include <atomic>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -12,7 +16,9 @@
 #include "../pigfem_assignment_amd/csrc/kernels/pgf_device.hpp"
 
 static size_t g_limit = ~(size_t)0;
+static std::atomic<size_t> g_bytes{0};
 void* operator new(size_t n) {
+    g_bytes += n;
     void* p = n >= g_limit ? nullptr : std::malloc(n);
     if (!p) throw std::bad_alloc();
     return p;
@@ -44,22 +50,25 @@ static void grid_pattern(pgf_ctx& c, int n) {
 
 int main(int argc, char** argv) {
     pgf_ctx* c = new pgf_ctx();
-    const bool workspace = argc > 1 && !std::strcmp(argv[1], "workspace");
-    const int n = workspace ? 4 : 400;
+    const char* mode = argc > 1 ? argv[1] : "";
+    const bool unfit = !std::strcmp(mode, "unfit");
+    const int n = !std::strcmp(mode, "workspace") ? 4 : unfit ? 800 : 400, nrhs = unfit ? 4 : 1;
     grid_pattern(*c, n);
     const int64_t sys[2] = {0, c->n_free};
-    double* b = (double*)std::calloc((size_t)n * n, sizeof(double));
-    double* x = (double*)std::calloc((size_t)n * n, sizeof(double));
-    if (workspace) {
+    double* b = (double*)std::calloc((size_t)n * n * nrhs, sizeof(double));
+    double* x = (double*)std::calloc((size_t)n * n * nrhs, sizeof(double));
+    if (!std::strcmp(mode, "workspace")) {
         c->batch_teams.emplace_back();
         c->batch_sys = {0, c->n_free};
         c->batch_nrhs = 1;
-    } else {
-        g_limit = (size_t)std::atoll(argv[2]);
     }
-    const int rc = pgf_batch_pcg(c, 1, sys, 1, b, x, 1e-8, 10, nullptr, nullptr, nullptr, nullptr);
-    g_limit = ~(size_t)0;
-    std::printf("status %d: %s\n", rc, pgf_last_error(c));
+    for (int call = 0; call < (unfit ? 2 : 1); ++call) {
+        if (argc > 2) g_limit = (size_t)std::atoll(argv[2]);
+        g_bytes = 0;
+        const int rc = pgf_batch_pcg(c, 1, sys, nrhs, b, x, 1e-8, 10, nullptr, nullptr, nullptr, nullptr);
+        g_limit = ~(size_t)0;
+        std::printf("status %d, %zu bytes: %s\n", rc, (size_t)g_bytes, pgf_last_error(c));
+    }
     std::fflush(stdout);
     std::_Exit(0);  // (the context holds nothing of the device)
 }
