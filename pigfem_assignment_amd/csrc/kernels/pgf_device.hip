@@ -451,6 +451,12 @@ __global__ __launch_bounds__(256) void k_cg_init(int64_t n, const double* b, dou
     }
 }
 
+// A converged recurrence goes on where it stopped, to a smaller tolerance.
+__global__ void k_cg_resume(double tol2, double* scal, int* done) {
+    scal[S_TOL2] = tol2;
+    *done = 0;
+}
+
 template <typename TA>
 __global__ __launch_bounds__(256) void k_diag_inv(int64_t n, const int32_t* __restrict__ diag, const TA* __restrict__ A,
                                                   double* __restrict__ dinv) {
@@ -535,22 +541,28 @@ struct Progress {
 // at a time; the device flag stops the recurrence, the host only polls the
 // pinned scalars between chunks.
 template <typename TA>
-static void pcg_launches(Ctx& c, const TA* A, const double* b, bool x0, double rtol, int maxit) {
+static void pcg_launches(Ctx& c, const TA* A, const double* b, bool x0, bool resume, double rtol, int maxit) {
     const int64_t n = c.n_free;
     double *z = (double*)c.zp, *p = z + n;
     int* done = (int*)(c.scal + S_NSCAL + 4);
-    hipLaunchKernelGGL(k_diag_inv<TA>, dim3(grid_for(n)), dim3(256), 0, c.stream, n, (const int32_t*)c.diag, A, c.dinv);
-    if (!x0) fill_async<double>(c, c.x, n, 0.0);
-    hipLaunchKernelGGL(k_cg_init, dim3(grid_for(n)), dim3(256), 0, c.stream, n, b, c.r, z, p,
-                       x0 ? (const double*)c.q : nullptr, (const double*)c.dinv, c.scal, c.partial, c.counter, done,
-                       rtol * rtol, (double)maxit);
+    int it = 0;
+    if (resume) {
+        hipLaunchKernelGGL(k_cg_resume, dim3(1), dim3(1), 0, c.stream, rtol * rtol, c.scal, done);
+        it = (int)c.h_scal[pgft::T_IT];
+    } else {
+        hipLaunchKernelGGL(k_diag_inv<TA>, dim3(grid_for(n)), dim3(256), 0, c.stream, n, (const int32_t*)c.diag, A, c.dinv);
+        if (!x0) fill_async<double>(c, c.x, n, 0.0);
+        hipLaunchKernelGGL(k_cg_init, dim3(grid_for(n)), dim3(256), 0, c.stream, n, b, c.r, z, p,
+                           x0 ? (const double*)c.q : nullptr, (const double*)c.dinv, c.scal, c.partial, c.counter, done,
+                           rtol * rtol, (double)maxit);
+    }
     const int G = c.dim == 3 ? 16 : 8;
     const unsigned ga = (unsigned)std::max<int64_t>(1, std::min<int64_t>((c.n_grp * G + 255) / 256, CG_SPMV_BLOCKS));
     const unsigned gu = (unsigned)std::max<int64_t>(1, std::min<int64_t>((n + 255) / 256, CG_UPD_BLOCKS));
     double* part_a = c.partial;                   // [ga] p.q
     double* part_u = c.partial + CG_SPMV_BLOCKS;  // [2][gu] rz, rr
     Progress progress;
-    for (int it = 0; it < std::max(maxit, 1);) {
+    while (it < std::max(maxit, 1)) {
         for (int k = 0; k < 32; ++k, ++it) {
             hipLaunchKernelGGL(k_cg_pupd, dim3(gu), dim3(256), 0, c.stream, n, (const double*)z, p, (const double*)c.scal,
                                (const int*)done);
@@ -581,13 +593,21 @@ static void pcg_launches(Ctx& c, const TA* A, const double* b, bool x0, double r
     c.h_scal[pgft::T_IT] = its;
 }
 
+// A converged solve goes on where it stopped, to a smaller tolerance.
+__global__ void k_team_resume(double tol2, double* state, int* pos) {
+    state[pgft::T_TOL] = tol2 * state[pgft::T_RR0];
+    state[pgft::T_DONE] = 0.0;
+    pos[0] = 0;
+    pos[1] = 1;
+}
+
 // The solve on the context's team; false if there is none or the device gives
 // no cooperative launch.  A launch runs at most TEAM_ITS iterations, so the
 // host sees a long solve's progress.
 constexpr int TEAM_ITS = 2048;
 
 template <typename TA>
-static bool pcg_team(Ctx& c, const TA* A, const double* b, bool x0, double rtol, int maxit) {
+static bool pcg_team(Ctx& c, const TA* A, const double* b, bool x0, bool resume, double rtol, int maxit) {
     if (!c.team.fits) return false;
     const pgft::TeamShape shape =
         c.dim == 3 ? pgft::team_shape<TA, 1, 3>(c.team.plan) : pgft::team_shape<TA, 1, 2>(c.team.plan);
@@ -610,13 +630,14 @@ static bool pcg_team(Ctx& c, const TA* A, const double* b, bool x0, double rtol,
     void* args[] = {(void*)&a};
     const int64_t n_slots = c.team.n_slots();
     Progress progress;
-    hipLaunchKernelGGL(k_fill<int>, dim3(1), dim3(64), 0, c.stream, c.team.pos, (int64_t)3, 0);
+    if (resume) hipLaunchKernelGGL(k_team_resume, dim3(1), dim3(1), 0, c.stream, a.tol2, c.scal, c.team.pos);
+    else hipLaunchKernelGGL(k_fill<int>, dim3(1), dim3(64), 0, c.stream, c.team.pos, (int64_t)3, 0);
     for (bool first = true;; first = false) {
         hipLaunchKernelGGL(k_fill<unsigned long long>, dim3((unsigned)((n_slots + 255) / 256)), dim3(256), 0, c.stream,
                            c.team.slots, n_slots, pgft::EMPTY);
         const hipError_t e = hipLaunchCooperativeKernel(shape.kernel, dim3((unsigned)c.team.plan.blocks), dim3(pgft::TT), args,
                                                         shape.lds, c.stream);
-        if (first && (e == hipErrorIllegalState || e == hipErrorCooperativeLaunchTooLarge)) {
+        if (first && !resume && (e == hipErrorIllegalState || e == hipErrorCooperativeLaunchTooLarge)) {
             (void)hipGetLastError();
             return false;
         }
@@ -633,8 +654,11 @@ static bool pcg_team(Ctx& c, const TA* A, const double* b, bool x0, double rtol,
 }
 
 // Jacobi-PCG on K_ff: x from x0 (then c.x holds it) or zero, b a device vector.
+// With spare (a vector that may be b), a solve that has met rtol goes on to aim;
+// where its iterations run out above rtol, x is the iterate that met it.
 template <typename TA>
-static void run_pcg(Ctx& c, const TA* A, const double* b, bool x0, double rtol, int maxit, pgf_solve_info* info) {
+static void run_pcg(Ctx& c, const TA* A, const double* b, bool x0, double rtol, int maxit, pgf_solve_info* info,
+                    double aim = 0.0, double* spare = nullptr) {
     *info = pgf_solve_info{0, 1, 0.0, 0.0};
     if (c.n_free == 0) return;
     hipEvent_t e0, e1;
@@ -642,17 +666,30 @@ static void run_pcg(Ctx& c, const TA* A, const double* b, bool x0, double rtol, 
     HIPCHK(hipEventCreate(&e1));
     HIPCHK(hipEventRecord(e0, c.stream));
     if (x0) enqueue_spmv<TA, double>(c, A, c.x, c.q);
-    if (!pcg_team<TA>(c, A, b, x0, rtol, maxit)) pcg_launches<TA>(c, A, b, x0, rtol, maxit);
+    const bool on_team = pcg_team<TA>(c, A, b, x0, false, rtol, maxit);
+    if (!on_team) pcg_launches<TA>(c, A, b, x0, false, rtol, maxit);
+    auto rr = [&] { return c.h_scal[pgft::T_RR]; };
+    const double rr0 = c.h_scal[pgft::T_RR0];
+    auto met = [&](double tol) { return rr0 == 0 || rr() <= tol * tol * rr0; };
+    info->converged = met(rtol);
+    if (spare && info->converged && !met(aim) && c.h_scal[pgft::T_IT] < maxit) {
+        const double rr1 = rr();
+        hipLaunchKernelGGL(k_copy, dim3(grid_for(c.n_free)), dim3(256), 0, c.stream, c.n_free, (const double*)c.x, spare);
+        if (on_team) (void)pcg_team<TA>(c, A, b, x0, true, aim, maxit);
+        else pcg_launches<TA>(c, A, b, x0, true, aim, maxit);
+        if (!met(rtol)) {
+            hipLaunchKernelGGL(k_copy, dim3(grid_for(c.n_free)), dim3(256), 0, c.stream, c.n_free, (const double*)spare, c.x);
+            c.h_scal[pgft::T_RR] = rr1;
+        }
+    }
     HIPCHK(hipEventRecord(e1, c.stream));
     HIPCHK(hipEventSynchronize(e1));
     float ms = 0.f;
     HIPCHK(hipEventElapsedTime(&ms, e0, e1));
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
-    const double rr = c.h_scal[pgft::T_RR], rr0 = c.h_scal[pgft::T_RR0];
     info->iterations = (int)c.h_scal[pgft::T_IT];
-    info->rel_residual = rr0 > 0 ? std::sqrt(rr / rr0) : 0.0;
-    info->converged = rr0 == 0 || rr <= rtol * rtol * rr0;
+    info->rel_residual = rr0 > 0 ? std::sqrt(rr() / rr0) : 0.0;
     info->ms = ms;
 }
 
@@ -1431,11 +1468,11 @@ PGF_API int pgf_newton_step(pgf_ctx* c, double frac, const pgf_newton_opts* o, p
                 const int maxit32 = o->fp32_maxit > 0 ? std::min(o->fp32_maxit, o->lin_maxit) : o->lin_maxit;
                 // the residual of these solves dips and rises around the
                 // tolerance, and whether a dip just meets it decides the
-                // refined step's accuracy within a factor of ten; asking for
-                // a tenth more keeps the sums' order from costing accuracy
+                // refined step's accuracy within a factor of ten; going on
+                // for a tenth more keeps the sums' order from costing accuracy
                 // (200 x 200 quads, 20 circles: displacement error 2.7e-9
                 // against 2.4e-9 to 1.6e-8 by the order of the sums)
-                pgfd::run_pcg<float>(*c, c->K32, c->res, g, 0.9 * lin_tol, maxit32, &si);
+                pgfd::run_pcg<float>(*c, c->K32, c->res, g, lin_tol, maxit32, &si, 0.9 * lin_tol, c->res);
                 if (!si.converged) {
                     fallback = it + 1;
                     HIPCHK(hipEventRecord(a0, c->stream));

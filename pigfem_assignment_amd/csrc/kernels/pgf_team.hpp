@@ -644,13 +644,13 @@ __global__ __launch_bounds__(TT) void k_team_pcg(TeamArgs<TA> a) {
                 ++it[c];
                 if (!(rr[c] > tol[c]) || it[c] >= a.maxit || (a.single && !isfinite(rr[c]))) {
                     act[c] = false;
-                    beta[c] = 0.0;  // its direction stays put while other right-hand sides run
+                    if (NR > 1) beta[c] = 0.0;  // its direction stays put while other right-hand sides run
                 }
                 any = any || act[c];
             }
             --left;
         }
-        if (any && ALL)  // to be resumed
+        if (ALL && (any || a.single))  // to be resumed
             for (int i = t; i < nrow; i += TT)
                 for (int c = 0; c < NR; ++c) rg[c * a.ld + i] = Lr[c * nrow + i];
         if (me == 0 && t == 0)
