@@ -1134,29 +1134,45 @@ __global__ void k_round32(int64_t n, const double* __restrict__ src, float* __re
 // Homogenised response of an RVE (SubscaleModel::homogenize_stress_strain,
 // src/SubscaleModel.cpp:42-196): over every volumetric point of the elements
 // of a segment, sum w * sigma with sigma = D (eps(u) + eps_bar), w * eps(u)
-// and w.  Segment k (elements [seg[k], seg[k+1])) is split evenly over vb
+// and w.  Segment k (elements [seg[k], seg[k+1])) is split evenly over its
 // blocks; each block writes one partial per quantity, and k_vol_finish adds a
 // segment's partials in a fixed order (deterministic).
 //
 // Bound by memory latency: per element one connectivity record and four nodes.
-// vb gives every thread about one element as long as the launch stays within
-// VOL_LAUNCH blocks (701 x 701 quads in one segment: 1.66 ms with 64 blocks a
-// segment, 41 us with 1920).  The block's cut elements are listed and taken by
+// A segment has about a block per 2^shift of its elements, 256 as long as that
+// makes no more than VOL_LAUNCH blocks and one per segment: every thread about
+// one element (701 x 701 quads in one segment: 1.66 ms with 64 blocks, 41 us
+// with 1920).  Blocks follow the segment's own length, not the mean one: a call
+// with 999 segments of one element and one of 490,402 took 2.82 ms with two
+// blocks each, 0.084 ms so; the search for the block's segment costs 1,000 equal
+// ones 5 us (65 -> 70).  The block's cut elements are listed and taken by
 // 32 (2D) or 16 (3D) lanes each, one point per lane: one thread walking its
 // points holds up the other 63, and one wavefront taking them one after the
 // other still needs 64 us.
-constexpr int VOL_LAUNCH = 4096;
+constexpr int64_t VOL_LAUNCH = 4096;
 
-int vol_blocks(int n_seg, int64_t n_elem) {
-    const int64_t want = (n_elem / std::max(n_seg, 1) + 255) / 256;
-    return (int)std::max<int64_t>(1, std::min<int64_t>({want, VOL_LAUNCH / n_seg, 2048}));
+int vol_shift(int64_t n_elem) {
+    int s = 8;
+    while (n_elem >> s > VOL_LAUNCH) ++s;
+    return s;
 }
+// first block of segment k: one per segment and one per multiple of 2^shift
+// elements before it
+__device__ __host__ inline int64_t vol_first(const int64_t* seg, int k, int shift) { return k + ((seg[k] - seg[0]) >> shift); }
 
 template <int DIM>
-__global__ __launch_bounds__(256) void k_vol_partials(AsmArgs a, int vb, const double* __restrict__ eps_bar,
+__global__ __launch_bounds__(256) void k_vol_partials(AsmArgs a, int n_seg, int shift,
+                                                      const double* __restrict__ eps_bar,
                                                       const int64_t* __restrict__ seg, double* __restrict__ part) {
     constexpr int S = DIM == 2 ? 3 : 6, NQ = DIM == 2 ? 4 : 1, W = 2 * S + 1;
-    const int k = blockIdx.x / vb, b = blockIdx.x % vb;
+    int k = 0;  // the last segment whose first block is this one or before it
+    for (int hi = n_seg; hi - k > 1;) {
+        const int m = (k + hi) >> 1;
+        if (vol_first(seg, m, shift) <= (int64_t)blockIdx.x) k = m;
+        else hi = m;
+    }
+    const int64_t first = vol_first(seg, k, shift);
+    const int vb = (int)(vol_first(seg, k + 1, shift) - first), b = (int)((int64_t)blockIdx.x - first);
     const int64_t e0 = seg[k], len = seg[k + 1] - e0;
     const int64_t c0 = e0 + len * b / vb, c1 = e0 + len * (b + 1) / vb;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -1250,10 +1266,13 @@ __global__ __launch_bounds__(256) void k_vol_partials(AsmArgs a, int vb, const d
 // out[k] = (averaged stress [S], averaged fluctuation strain [S], volume): one
 // block per segment
 template <int DIM>
-__global__ __launch_bounds__(256) void k_vol_finish(int vb, const double* __restrict__ part, double* __restrict__ out) {
+__global__ __launch_bounds__(256) void k_vol_finish(int shift, const int64_t* __restrict__ seg,
+                                                    const double* __restrict__ part, double* __restrict__ out) {
     constexpr int S = DIM == 2 ? 3 : 6, W = 2 * S + 1;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const double* p = part + (int64_t)blockIdx.x * vb * W;
+    const int64_t first = vol_first(seg, blockIdx.x, shift);
+    const int vb = (int)(vol_first(seg, blockIdx.x + 1, shift) - first);
+    const double* p = part + first * W;
     double acc[W];
     for (int i = 0; i < W; ++i) acc[i] = 0.0;
     for (int b = threadIdx.x; b < vb; b += 256)
@@ -1367,18 +1386,21 @@ static void launch_dim(Ctx& c, const pgfk::AsmArgs& a, bool jac, bool func, bool
     if (func && (fp32 || !jac)) launch_gather<DIM, false, true, double>(c, a);
 }
 
-int volume_average_blocks(int n_seg, int64_t n_elem) { return pgfk::vol_blocks(n_seg, n_elem); }
+int64_t volume_average_blocks(int n_seg, const int64_t* seg) {
+    return pgfk::vol_first(seg, n_seg, pgfk::vol_shift(seg[n_seg] - seg[0]));
+}
 
-void enqueue_volume_average(Ctx& c, const double* d_eps_bar, int n_seg, int vb, const int64_t* d_seg, double* d_part,
-                            double* d_out) {
+void enqueue_volume_average(Ctx& c, const double* d_eps_bar, int n_seg, const int64_t* seg, const int64_t* d_seg,
+                            double* d_part, double* d_out) {
     const pgfk::AsmArgs a = c.asm_args();
-    const dim3 grid((unsigned)(n_seg * vb)), blk(256);
+    const int shift = pgfk::vol_shift(seg[n_seg] - seg[0]);
+    const dim3 grid((unsigned)volume_average_blocks(n_seg, seg)), blk(256);
     if (c.dim == 2) {
-        hipLaunchKernelGGL((pgfk::k_vol_partials<2>), grid, blk, 0, c.stream, a, vb, d_eps_bar, d_seg, d_part);
-        hipLaunchKernelGGL((pgfk::k_vol_finish<2>), dim3((unsigned)n_seg), blk, 0, c.stream, vb, d_part, d_out);
+        hipLaunchKernelGGL((pgfk::k_vol_partials<2>), grid, blk, 0, c.stream, a, n_seg, shift, d_eps_bar, d_seg, d_part);
+        hipLaunchKernelGGL((pgfk::k_vol_finish<2>), dim3((unsigned)n_seg), blk, 0, c.stream, shift, d_seg, d_part, d_out);
     } else {
-        hipLaunchKernelGGL((pgfk::k_vol_partials<3>), grid, blk, 0, c.stream, a, vb, d_eps_bar, d_seg, d_part);
-        hipLaunchKernelGGL((pgfk::k_vol_finish<3>), dim3((unsigned)n_seg), blk, 0, c.stream, vb, d_part, d_out);
+        hipLaunchKernelGGL((pgfk::k_vol_partials<3>), grid, blk, 0, c.stream, a, n_seg, shift, d_eps_bar, d_seg, d_part);
+        hipLaunchKernelGGL((pgfk::k_vol_finish<3>), dim3((unsigned)n_seg), blk, 0, c.stream, shift, d_seg, d_part, d_out);
     }
 }
 

@@ -1209,15 +1209,14 @@ PGF_API int pgf_volume_average(pgf_ctx* c, const double* eps_bar, int32_t n_seg,
             if (seg_elem[k] < 0 || seg_elem[k] > seg_elem[k + 1] || seg_elem[k + 1] > c->n_elem)
                 throw pgf::Error(PGF_EARG, "element segments must be ordered ranges inside [0, n_elem]");
         const int S = c->dim == 2 ? 3 : 6, W = 2 * S + 1;
-        const int vb = pgfd::volume_average_blocks(n_seg, seg_elem[n_seg] - seg_elem[0]);
         // eps_bar [8] | segments [n_seg + 1] | out [n_seg][W] | partials
-        double* de = c->workspace(8 + n_seg + 1 + (int64_t)n_seg * (vb + 1) * W);
+        double* de = c->workspace(8 + n_seg + 1 + (n_seg + pgfd::volume_average_blocks(n_seg, seg_elem)) * W);
         int64_t* ds = (int64_t*)(de + 8);
         double* dout = de + 8 + n_seg + 1;
         double* dpart = dout + (int64_t)n_seg * W;
         HIPCHK(hipMemcpyAsync(de, eps_bar, sizeof(double) * S, hipMemcpyHostToDevice, c->stream));
         HIPCHK(hipMemcpyAsync(ds, seg_elem, sizeof(int64_t) * (n_seg + 1), hipMemcpyHostToDevice, c->stream));
-        pgfd::enqueue_volume_average(*c, de, n_seg, vb, ds, dpart, dout);
+        pgfd::enqueue_volume_average(*c, de, n_seg, seg_elem, ds, dpart, dout);
         HIPCHK(hipGetLastError());
         HIPCHK(hipMemcpyAsync(out, dout, sizeof(double) * n_seg * W, hipMemcpyDeviceToHost, c->stream));
         HIPCHK(hipStreamSynchronize(c->stream));
@@ -1245,8 +1244,7 @@ PGF_API int pgf_volume_average_noalloc(pgf_ctx* c, const double* eps_bar, int32_
         double* dpart = dout + (size_t)PGF_NOALLOC_MAX_SEG * 13;
         HIPCHK(hipMemcpyAsync(de, eps_bar, sizeof(double) * S, hipMemcpyHostToDevice, c->stream));
         HIPCHK(hipMemcpyAsync(ds, seg_elem, sizeof(int64_t) * (n_seg + 1), hipMemcpyHostToDevice, c->stream));
-        pgfd::enqueue_volume_average(*c, de, n_seg, pgfd::volume_average_blocks(n_seg, seg_elem[n_seg] - seg_elem[0]), ds,
-                                     dpart, dout);
+        pgfd::enqueue_volume_average(*c, de, n_seg, seg_elem, ds, dpart, dout);
         HIPCHK(hipGetLastError());
         HIPCHK(hipMemcpyAsync(out, dout, sizeof(double) * n_seg * W, hipMemcpyDeviceToHost, c->stream));
         HIPCHK(hipStreamSynchronize(c->stream));

@@ -120,12 +120,12 @@ struct Ctx {
 template <typename T>
 void fill_async(Ctx& c, T* p, int64_t n, T v);
 void enqueue_assembly(Ctx& c, double dt, uint32_t flags);
-// homogenised response per element segment: blocks per segment for n_seg
-// segments of n_elem elements in all, at most max(VOL_LAUNCH, n_seg) in the launch;
-// partials [n_seg * vb][2S+1], out [n_seg][2S+1]
-int volume_average_blocks(int n_seg, int64_t n_elem);
-void enqueue_volume_average(Ctx& c, const double* d_eps_bar, int n_seg, int vb, const int64_t* d_seg, double* d_part,
-                            double* d_out);
+// homogenised response per element segment (seg: host array [n_seg + 1], d_seg
+// its device copy); blocks of the launch, at most n_seg + 4096; partials
+// [blocks][2S+1], out [n_seg][2S+1]
+int64_t volume_average_blocks(int n_seg, const int64_t* seg);
+void enqueue_volume_average(Ctx& c, const double* d_eps_bar, int n_seg, const int64_t* seg, const int64_t* d_seg,
+                            double* d_part, double* d_out);
 // the current device's scratch of the allocation-free entry point
 double* noalloc_scratch();
 // nodal field U from a dof vector (free part x, prescribed part up or zero)
