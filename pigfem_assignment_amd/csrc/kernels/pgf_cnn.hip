@@ -841,7 +841,6 @@ PGF_API int pgf_net_create(uint64_t seed, pgf_net** out) {
     pgf_net* net = new pgf_net();
     int rc = nguard(nullptr, [&]() {
         NCHK(hipStreamCreateWithFlags(&net->stream, hipStreamNonBlocking));
-        NCHK(net->copy.create());
         int64_t off = 0;
         for (int l = 0; l < N_LAYERS; ++l) {
             const LayerSpec& s = SPECS[l];

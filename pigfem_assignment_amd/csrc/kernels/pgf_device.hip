@@ -606,8 +606,39 @@ __global__ void k_team_resume(double tol2, double* state, int* pos) {
 // host sees a long solve's progress.
 constexpr int TEAM_ITS = 2048;
 
+// The team is laid out by the context's first solve: contexts that only
+// assemble, average or solve batches have none (with the pinned buffer it was
+// 0.6 of the 3.7 ms that creating 100 x 100 quads takes, 5 of 42 at 333 x 333, 10
+// of 158 at 48^3 x 6 tets, 8 of 136 for 32 cells of 64 to 157).  None where
+// memory for it is short: the launches need less.
+static void make_team(Ctx& c) {
+    c.team_tried = true;
+    // a block per CU, fewer where a block's threads would outnumber the lanes
+    // its rows can use
+    const int64_t lanes = c.n_grp * pgft::team_lanes(c.dim);
+    const int blocks = (int)std::max<int64_t>(1, std::min<int64_t>({(lanes + pgft::TT - 1) / pgft::TT, c.n_cu, pgft::MAX_TEAM}));
+    pgft::Team t;
+    try {
+        t.sys = {0};
+        t.fits = pgft::make_team_plan(c.dim, c.h_grp, {{0, c.n_grp}}, c.h_colidx.data(), blocks,
+                                      pgft::LDS_MAX / sizeof(double), t.plan) &&
+                 pgft::team_shape<double, 1, 2>(t.plan).kernel != nullptr;
+        if (!t.fits) return;
+        const hipError_t e = t.upload({{0}}, c.grp, c.colidx, c.nnz, nullptr, c.stream);
+        if (e == hipErrorOutOfMemory) {
+            (void)hipGetLastError();
+            return;
+        }
+        HIPCHK(e);
+    } catch (const std::bad_alloc&) {
+        return;
+    }
+    c.team = std::move(t);
+}
+
 template <typename TA>
 static bool pcg_team(Ctx& c, const TA* A, const double* b, bool x0, bool resume, double rtol, int maxit) {
+    if (!c.team_tried) make_team(c);
     if (!c.team.fits) return false;
     const pgft::TeamShape shape =
         c.dim == 3 ? pgft::team_shape<TA, 1, 3>(c.team.plan) : pgft::team_shape<TA, 1, 2>(c.team.plan);
@@ -792,7 +823,6 @@ PGF_API int pgf_create(const pgf_mesh_desc* d, pgf_ctx** out) {
         c->nnz_ff = 0;
         for (int64_t r = 0; r < d->n_free; ++r) c->nnz_ff += pat.rowsplit[r];
         HIPCHK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
-        HIPCHK(c->copy.create());
         // ---- elements in colour order ----
         std::vector<int64_t> ucount(pat.n_colors + 1, 0), ccount(pat.n_colors + 1, 0);
         for (int64_t e = 0; e < d->n_elem; ++e) {
@@ -1111,20 +1141,11 @@ PGF_API int pgf_create(const pgf_mesh_desc* d, pgf_ctx** out) {
             grp.push_back(pgft::GroupRec{(int32_t)c->n_free, 0, 0, 0});
             c->grp = pgfd::dupload(grp.data(), (int64_t)grp.size());
             c->diag = pgfd::dupload(diag.data(), (int64_t)diag.size());
-            // the PCG team: a block per CU, fewer where a block's threads
-            // would outnumber the lanes its rows can use
             int dev = 0;
             HIPCHK(hipGetDevice(&dev));
             HIPCHK(hipDeviceGetAttribute(&c->n_cu, hipDeviceAttributeMultiprocessorCount, dev));
-            const int64_t lanes = c->n_grp * pgft::team_lanes(c->dim);
-            const int blocks = (int)std::max<int64_t>(1, std::min<int64_t>({(lanes + pgft::TT - 1) / pgft::TT, c->n_cu, pgft::MAX_TEAM}));
-            c->team.sys = {0};
-            c->team.fits = pgft::make_team_plan(c->dim, grp, {{0, c->n_grp}}, pat.colidx.data(), blocks,
-                                                pgft::LDS_MAX / sizeof(double), c->team.plan) &&
-                           pgft::team_shape<double, 1, 2>(c->team.plan).kernel != nullptr;
         }
         c->colidx = pgfd::dupload(pat.colidx.data(), c->nnz);
-        if (c->team.fits) HIPCHK(c->team.upload({{0}}, c->grp, c->colidx, c->nnz, nullptr, c->stream));
         c->K = pgfd::dalloc<double>(c->nnz);
         c->K32 = pgfd::dalloc<float>(c->nnz);
         c->P = pgfd::dalloc<double>(c->n_rows);

@@ -89,7 +89,8 @@ struct Ctx {
     std::vector<pgft::GroupRec> h_grp;  // [n_grp + 1] host copy (shares of a batch)
     pgft::GroupRec* grp = nullptr;
     int32_t* diag = nullptr;       // entry of each free row's diagonal, -1 without one
-    pgft::Team team;               // of K_ff as one system
+    pgft::Team team;               // of K_ff as one system, from its first solve on
+    bool team_tried = false;
     // teams of the last batched solve with automatic choice, by its systems
     // and right-hand sides
     std::vector<pgft::Team> batch_teams;

@@ -726,6 +726,7 @@ struct Team {
     bool own_wcol = false;
     int* pos = nullptr;              // [n_teams][2], then the abort flag
     unsigned long long* slots = nullptr;
+    char* block = nullptr;           // holds the other arrays
     Team() = default;
     Team(Team&& o) noexcept { *this = std::move(o); }
     Team& operator=(Team&& o) noexcept {
@@ -743,53 +744,64 @@ struct Team {
         std::swap(own_wcol, o.own_wcol);
         std::swap(pos, o.pos);
         std::swap(slots, o.slots);
+        std::swap(block, o.block);
         return *this;
     }
     ~Team() {
-        void* p[] = {row_ptr, list, halo, halo_ptr, step_ptr, steps, own_wcol ? wcol : nullptr, pos, slots};
+        void* p[] = {block, own_wcol ? wcol : nullptr, pos, slots};
         for (void* q : p)
             if (q) (void)hipFree(q);
     }
     int64_t n_slots() const { return (int64_t)n_teams * COPIES * team_slots(plan.blocks); }
 
-    // Device arrays of a made plan; lists[t]: places in `sys` that team t
-    // solves, in its order.  wcol_in: the array to fill, or null for one of
-    // nnz entries of its own.
+    // Device arrays of a made plan: what the host laid out in one block and one
+    // copy (seven of each: a new context's first solve of 100 x 100 quads 10.4 ms,
+    // 6.7 so).  lists[t]: places in `sys` that team t solves, in its order.
+    // wcol_in: the array to fill, or null for one of nnz entries of its own.
     hipError_t upload(const std::vector<std::vector<int32_t>>& lists, const GroupRec* d_grp, const int32_t* d_col,
                       int64_t nnz, uint16_t* wcol_in, hipStream_t stream) {
         n_teams = (int)lists.size();
         std::vector<int32_t> l{0};
         for (const auto& t : lists) l.push_back(l.back() + (int32_t)t.size());
         for (const auto& t : lists) l.insert(l.end(), t.begin(), t.end());
-        int32_t* part = nullptr;
-        hipError_t e = hipSuccess;
-        auto put = [&](auto*& d, const auto* h, size_t n) {
-            if (e == hipSuccess) e = hipMalloc((void**)&d, sizeof(*d) * std::max<size_t>(n, 1));
-            if (e == hipSuccess && h && n) e = hipMemcpy(d, h, sizeof(*d) * n, hipMemcpyHostToDevice);
+        std::vector<char> host;
+        auto put = [&](const auto& v) {  // returns its place
+            const size_t at = host.size(), n = sizeof(v[0]) * v.size();
+            host.resize(at + (n + 255) / 256 * 256);
+            std::copy_n((const char*)v.data(), n, host.data() + at);
+            return at;
         };
-        put(row_ptr, plan.row_ptr.data(), plan.row_ptr.size());
-        put(list, l.data(), l.size());
-        put(halo, plan.halo.data(), plan.halo.size());
-        put(halo_ptr, plan.halo_ptr.data(), plan.halo_ptr.size());
-        put(step_ptr, plan.step_ptr.data(), plan.step_ptr.size());
-        put(steps, plan.steps.data(), plan.steps.size());
-        put(pos, (int*)nullptr, 2 * (size_t)n_teams + 1);
-        put(slots, (unsigned long long*)nullptr, (size_t)n_slots());
-        put(part, plan.part.data(), plan.part.size());
+        const size_t at_row = put(plan.row_ptr), at_list = put(l), at_halo = put(plan.halo), at_hptr = put(plan.halo_ptr),
+                     at_sptr = put(plan.step_ptr), at_steps = put(plan.steps), at_part = put(plan.part);
+        hipError_t e = hipSuccess;
+        auto alloc = [&](auto*& d, size_t n) {
+            if (e == hipSuccess) e = hipMalloc((void**)&d, sizeof(*d) * std::max<size_t>(n, 1));
+            if (e != hipSuccess) d = nullptr;
+        };
+        alloc(block, host.size());
+        alloc(pos, 2 * (size_t)n_teams + 1);
+        alloc(slots, (size_t)n_slots());
         own_wcol = wcol_in == nullptr;
         wcol = wcol_in;
-        if (own_wcol) put(wcol, (uint16_t*)nullptr, (size_t)nnz);
+        if (own_wcol) alloc(wcol, (size_t)nnz);
+        if (e != hipSuccess) return e;
+        row_ptr = (int32_t*)(block + at_row);
+        list = (int32_t*)(block + at_list);
+        halo = (int32_t*)(block + at_halo);
+        halo_ptr = (int64_t*)(block + at_hptr);
+        step_ptr = (int64_t*)(block + at_sptr);
+        steps = (StepRec*)(block + at_steps);
+        e = hipMemcpyAsync(block, host.data(), host.size(), hipMemcpyHostToDevice, stream);
         if (e == hipSuccess) {
             const int n_shares = (int)sys.size() * plan.blocks;
-            hipLaunchKernelGGL(k_team_cols, dim3((unsigned)n_shares), dim3(256), 0, stream, n_shares, plan.blocks, part, d_grp,
-                               d_col, halo_ptr, halo, wcol);
+            hipLaunchKernelGGL(k_team_cols, dim3((unsigned)n_shares), dim3(256), 0, stream, n_shares, plan.blocks,
+                               (const int32_t*)(block + at_part), d_grp, d_col, halo_ptr, halo, wcol);
             e = hipGetLastError();
         }
-        if (e == hipSuccess) e = hipStreamSynchronize(stream);
-        if (part) (void)hipFree(part);
+        const hipError_t done = hipStreamSynchronize(stream);  // (the host's copy goes)
         // the host keeps the sizes only
         plan.part = {}; plan.row_ptr = {}; plan.step_ptr = {}; plan.steps = {}; plan.halo_ptr = {}; plan.halo = {};
-        return e;
+        return e == hipSuccess ? done : e;
     }
 
     template <typename TA>
