@@ -468,6 +468,12 @@ pgft::TeamShape batch_shape(int dim, const pgft::TeamPlan& p) {
     return dim == 3 ? pgft::team_shape<double, NR, 3>(p) : pgft::team_shape<double, NR, 2>(p);
 }
 
+bool out_of_memory(hipError_t e) {
+    if (e != hipErrorOutOfMemory) return false;
+    (void)hipGetLastError();
+    return true;
+}
+
 // Teams for the batch, kept with the context for calls with the same systems.
 // A team's blocks hold their windows in LDS: as many teams as that allows, 8
 // down to 5, for all systems; if some do not fit even then, those that fit an
@@ -475,8 +481,9 @@ pgft::TeamShape batch_shape(int dim, const pgft::TeamPlan& p) {
 // and so on.  (32 RVEs of 64 to 160 divisions, three right-hand sides: 222 ms
 // with three of them in a second launch, 200 ms with all in one of seven teams;
 // launches with tuned tiles 382 ms.)  Systems are dealt to the teams longest first.  False if
-// some system fits no team; the context remembers that for the last such
-// ranges, and keeps what it has laid out for others.
+// some system fits no team (the context remembers that for the last such
+// ranges, and keeps what it has laid out for others) or memory is short: the
+// launches need less.
 template <int NR>
 bool make_batch_teams(pgfd::Ctx& c, const std::vector<int64_t>& sp) {
     if (!c.batch_teams.empty() && c.batch_nrhs == NR && c.batch_sys == sp) return true;
@@ -541,13 +548,16 @@ bool make_batch_teams(pgfd::Ctx& c, const std::vector<int64_t>& sp) {
             lists[k].push_back(i);
             load[k] += cost(i);
         }
-        BCHK(t.upload(lists, c.grp, c.colidx, c.nnz, wcol, c.stream));
+        const hipError_t e = t.upload(lists, c.grp, c.colidx, c.nnz, wcol, c.stream);
+        if (out_of_memory(e)) return false;
+        BCHK(e);
         wcol = t.wcol;
         std::vector<int32_t> rest;
         for (int s : left)
             if (!std::binary_search(t.sys.begin(), t.sys.end(), s)) rest.push_back(s);
         left.swap(rest);
         teams.push_back(std::move(t));
+        return true;
     };
     // One system that fits no team takes the batch to the launches, so where the
     // largest may be one (more rows than half of what a team of the smallest
@@ -568,14 +578,15 @@ bool make_batch_teams(pgfd::Ctx& c, const std::vector<int64_t>& sp) {
         std::vector<int32_t> small;  // systems that fit the stage's smallest team
         for (size_t i = 0; i < stage.size() && !left.empty(); ++i) {
             pgft::Team t;
-            if (plan(left, stage[i], t)) take(t);
-            else if (i == 0)
+            if (plan(left, stage[i], t)) {
+                if (!take(t)) return false;
+            } else if (i == 0)
                 for (size_t k = 0; k < left.size(); ++k)
                     if (t.plan.sys_window[k] * 4ll / 3 <= fit) small.push_back(left[k]);
         }
         if (left.empty() || small.empty()) continue;
         pgft::Team t;
-        if (plan(small, stage[0], t)) take(t);
+        if (plan(small, stage[0], t) && !take(t)) return false;
     }
     if (!left.empty()) return unfit();
     std::vector<int64_t> key = sp;  // (may throw: before the teams change)
@@ -586,13 +597,19 @@ bool make_batch_teams(pgfd::Ctx& c, const std::vector<int64_t>& sp) {
 }
 
 // Device memory of one solve: kept with the context up to KEEP_BYTES, else of
-// the call.
+// the call; p is null where there is none.
 struct BatchWork {
     static constexpr int64_t KEEP_BYTES = 256ll << 20;
     double *p = nullptr, *own = nullptr;
     BatchWork(pgfd::Ctx& c, int64_t doubles) {
-        if (doubles * (int64_t)sizeof(double) <= KEEP_BYTES) p = c.workspace(doubles);
-        else p = own = balloc<double>((size_t)doubles);
+        if (doubles * (int64_t)sizeof(double) <= KEEP_BYTES) {
+            p = c.workspace(doubles, true);
+            return;
+        }
+        const hipError_t e = hipMalloc((void**)&own, sizeof(double) * (size_t)doubles);
+        if (e != hipSuccess) own = nullptr;
+        if (!out_of_memory(e)) BCHK(e);
+        p = own;
     }
     ~BatchWork() {
         if (own) (void)hipFree(own);
@@ -609,9 +626,15 @@ bool run_teams(pgfd::Ctx& c, const std::vector<int64_t>& sp, const double* b, do
                int32_t* iters, double* relres, double* ms_out, int* rc) {
     const int n_sys = (int)sp.size() - 1;
     const int64_t nf = c.n_free, nv = nf * NR;
-    if (nf == 0 || nv * (int64_t)sizeof(double2) > 0xffffffffll || !make_batch_teams<NR>(c, sp)) return false;
+    if (nf == 0 || nv * (int64_t)sizeof(double2) > 0xffffffffll) return false;
+    try {
+        if (!make_batch_teams<NR>(c, sp)) return false;
+    } catch (const std::bad_alloc&) {
+        return false;
+    }
     // x, r [NR][n] (r first holds b) | (z, p) pairs | 1/diag | states
     BatchWork work(c, 4 * nv + nf + (int64_t)n_sys * NR * pgft::T_N);
+    if (!work.p) return false;
     double *dx = work.p, *dr = dx + nv, *dz = dr + nv, *dd = dz + 2 * nv, *state = dd + nf;
     BCHK(hipMemcpyAsync(dr, b, sizeof(double) * nv, hipMemcpyHostToDevice, c.stream));
     struct Events {

@@ -76,12 +76,18 @@ void fill_async(Ctx& c, T* p, int64_t n, T v) {
 template void fill_async<double>(Ctx&, double*, int64_t, double);
 template void fill_async<float>(Ctx&, float*, int64_t, float);
 
-double* Ctx::workspace(int64_t doubles) {
+double* Ctx::workspace(int64_t doubles, bool or_null) {
     if (doubles > work_n) {
         if (work) HIPCHK(hipFree(work));
         work = nullptr;
         work_n = 0;
-        work = dalloc<double>(doubles);
+        const hipError_t e = hipMalloc((void**)&work, sizeof(double) * (size_t)doubles);
+        if (e != hipSuccess) work = nullptr;
+        if (e == hipErrorOutOfMemory && or_null) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        HIPCHK(e);
         work_n = doubles;
     }
     return work;

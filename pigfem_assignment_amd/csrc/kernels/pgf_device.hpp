@@ -109,7 +109,7 @@ struct Ctx {
     // and freed with the context
     double* work = nullptr;
     int64_t work_n = 0;
-    double* workspace(int64_t doubles);
+    double* workspace(int64_t doubles, bool or_null = false);  // or_null: without memory for it, null
     bool have_guess = false;
     hipEvent_t* timing_events = nullptr;  // when set: cut pass start, gather start, gather end
     LearnState* learn = nullptr;
