@@ -601,7 +601,10 @@ __global__ __launch_bounds__(TT) void k_team_pcg(TeamArgs<TA> a) {
                     if (i >= nrow) continue;
 #pragma unroll
                     for (int c = 0; c < NR; ++c) {
-                        if (!act[c]) continue;
+                        if (NR > 1 && !act[c]) {  // q back to z, which p is
+                            Lq[c * nrow + i] = pi[k][c];
+                            continue;
+                        }
                         const double rn = ri[k][c] - alpha[c] * qi[k][c];
                         const double zi = di[k] * rn;
                         if (ALL) Lr[c * nrow + i] = rn;
@@ -644,7 +647,9 @@ __global__ __launch_bounds__(TT) void k_team_pcg(TeamArgs<TA> a) {
                 ++it[c];
                 if (!(rr[c] > tol[c]) || it[c] >= a.maxit || (a.single && !isfinite(rr[c]))) {
                     act[c] = false;
-                    if (NR > 1) beta[c] = 0.0;  // its direction stays put while other right-hand sides run
+                    // while other right-hand sides run, its p is the last z, of the
+                    // rows and of the halo alike
+                    if (NR > 1) beta[c] = 0.0;
                 }
                 any = any || act[c];
             }
