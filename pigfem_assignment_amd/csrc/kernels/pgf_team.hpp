@@ -37,9 +37,11 @@
 //    than a step take consecutive steps of one lane group, so no lane waits in
 //    a loop over a neighbour's long row, and every block has about as many.
 //
-// Every wait ends: a wait that has seen no change for WAIT_TICKS raises the
-// abort flag, all blocks leave and the host reports a device error.  The
-// launch is cooperative, so all blocks are resident.
+// Every wait ends: a block leaves that has waited for one sum longer than
+// WAIT_TICKS, and raises the abort flag, by which the host reports a device
+// error.  No block looks at the flag: the others of its team, which are at the
+// same sum or the next, run into the limit by themselves.  The launch is
+// cooperative, so all blocks are resident.
 #pragma once
 
 #include <hip/hip_runtime.h>
