@@ -41,10 +41,7 @@ typedef short v4s __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef uint16_t bf16;
 
-#ifndef PGF_CNN_GRID
-#define PGF_CNN_GRID 64
-#endif
-constexpr int GRID = PGF_CNN_GRID;
+constexpr int GRID = 64;  // the interface's; the kernels' tiles are laid out for it
 constexpr int NVOX = GRID * GRID * GRID;
 constexpr int IN_CH = 8;
 constexpr int OUT_CH = 3;
@@ -172,6 +169,7 @@ template <bool BACK, int C, int N, int D, int YB>
 __global__ __launch_bounds__(256) void k_conv3(ConvArgs a) {
     constexpr int KS = (27 * C + 15) / 16, KB = 9, NB = (KS + KB - 1) / KB, NCT = N / 16;
     constexpr int LI = (YB + 2) * 3, PS = C + (C >= 32 ? 4 : 0), LINE = (D + 2) * PS;
+    static_assert(D % 16 == 0 && 64 % D == 0 && D % YB == 0, "four wavefronts share whole lines of 16-position tiles");
     constexpr int XT = D / 16, WY = 4 / XT, PT = YB / WY, H8 = C / 8, LOADS = (LI * D * H8 + 255) / 256;
     __shared__ __align__(16) bf16 s_in[LI * LINE];
     const int lane = threadIdx.x & 63, row = lane & 15, kq = lane >> 4, wave = threadIdx.x >> 6;
@@ -246,6 +244,7 @@ template <bool BACK, int MODE, int C, int N, int DIN, int NT>
 __global__ __launch_bounds__(256) void k_conv2(ConvArgs a) {
     constexpr int S = MODE == DOWN ? DIN / 2 : DIN, DOUT = dout_of(MODE, DIN), CS = C / 16, KST = 8 * CS;
     constexpr int KS = MODE == UP ? CS : KST, KB = KS < 8 ? KS : 8, NB = KS / KB;
+    static_assert(S % 16 == 0 && S * S * S % 64 == 0, "whole tiles of 16 positions along x, four to a block");
     constexpr int XT = S / 16, NCT = N / (16 * NT), CLS = MODE == UP ? 2 : 1;
     const int lane = threadIdx.x & 63, row = lane & 15, kq = lane >> 4;
     // x tile fastest, then y, z, for UP the parity in y and z
@@ -336,6 +335,7 @@ __device__ inline void put8(bf16* tile, int ld, int x, uint4 v) {
 }
 template <int C, int N, int D>
 __global__ __launch_bounds__(192) void k_wgrad3(WgArgs a) {
+    static_assert(WG_POS % D == 0 && D % (WG_POS / D) == 0, "a stage is whole lines of one plane");
     constexpr int R = WG_POS / D, LI = (R + 2) * 3, LD = D + 4, LG = WG_POS + 4, TC = 27 * C;
     constexpr int CH = C < 16 ? C : 16, H8 = CH / 8;  // staged input channels, in groups of 8
     constexpr int CT = C < 16 ? 1 : C / 16, NT = N / 16;
@@ -407,6 +407,7 @@ __global__ __launch_bounds__(192) void k_wgrad3(WgArgs a) {
 // one H^3 with CQ: DOWN has in fine and g coarse, UP in coarse and g fine.
 template <int CF, int CQ, int H, bool IS_UP>
 __global__ __launch_bounds__(256) void k_wgrad2(WgArgs a) {
+    static_assert(WG_POS % H == 0 && H % (WG_POS / H) == 0, "a stage is whole lines of one plane");
     constexpr int R = WG_POS / H, LD = H + 4, LG = WG_POS + 4, D = 2 * H;
     constexpr int C = IS_UP ? CQ : CF, N = IS_UP ? CF : CQ, TC = 8 * C;
     constexpr int FT = CF / 16, QT = CQ / 16;
@@ -679,7 +680,8 @@ static std::string g_net_err;
 // two leave half the chip's wavefront slots empty.
 template <int C, int N, int D, int YB>
 static int conv3(pgf_net* net, const ConvArgs& a) {
-    const int rows = D / YB * D;
+    constexpr int rows = D / YB * D;
+    static_assert(rows * N <= BIAS_PART, "the layer's bias partials fit their place");
     const dim3 grid(rows * (N / 16));
     if (!a.act) hipLaunchKernelGGL((k_conv3<false, C, N, D, YB>), grid, dim3(256), 0, net->stream, a);
     // (the network's input has no gradient)
@@ -690,7 +692,8 @@ static int conv3(pgf_net* net, const ConvArgs& a) {
 template <int MODE, int C, int N, int DIN, int NT>
 static int conv2(pgf_net* net, const ConvArgs& a) {
     constexpr int S = MODE == DOWN ? DIN / 2 : DIN;
-    const int rows = S * S * S / 64 * (MODE == UP ? 4 : 1);
+    constexpr int rows = S * S * S / 64 * (MODE == UP ? 4 : 1);
+    static_assert(rows * N <= BIAS_PART, "the layer's bias partials fit their place");
     const dim3 grid(rows * (N / (16 * NT)));
     if (a.act) hipLaunchKernelGGL((k_conv2<true, MODE, C, N, DIN, NT>), grid, dim3(256), 0, net->stream, a);
     else hipLaunchKernelGGL((k_conv2<false, MODE, C, N, DIN, NT>), grid, dim3(256), 0, net->stream, a);
