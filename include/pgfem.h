@@ -203,6 +203,15 @@ PGF_API int pgf_set_isv(pgf_ctx* ctx, const double* delta_max_conv);
 PGF_API int pgf_spmv(pgf_ctx* ctx, const double* x, double* y);   /* y = K_ff x, host vectors [n_free] */
 PGF_API int pgf_pcg(pgf_ctx* ctx, const double* b, double* x, const double* x0, double rtol, int32_t maxit,
                     int32_t precision, pgf_solve_info* info);
+/* Where the device allows it, a solve (pgf_pcg, the solves of pgf_newton_step,
+ * pgf_batch_pcg with the layout left to the library) runs in one launch whose
+ * blocks stay resident and iterate together; a system too large for that, short
+ * memory and a refused cooperative launch (another process holds the device's
+ * queue for them) make it separate launches, with the same results up to the
+ * order of sums.  allow: 0 always separate launches, 1 resident where possible
+ * (the default), -1 as it is; n_resident (may be NULL): solves of this context
+ * that ran resident so far. */
+PGF_API int pgf_resident_solves(pgf_ctx* ctx, int32_t allow, int64_t* n_resident);
 /* optional initial guess for the next Newton solves, [n_free] (learned predictor) */
 PGF_API int pgf_set_guess(pgf_ctx* ctx, const double* dx);
 
@@ -212,10 +221,12 @@ PGF_API int pgf_set_guess(pgf_ctx* ctx, const double* dx);
  * (MatMatSolve, src/SensitivityDirect.cpp:96-136).  K_ff of the context must be
  * block diagonal over the free-row ranges sys_ptr[0..n_sys] (a context built on
  * a concatenation of independent meshes; checked).  Every (system, rhs) pair
- * runs its own Jacobi-PCG from a zero start to ||r|| <= rtol ||b||, all pairs
- * in one captured-graph iteration sweep.  b, x: host [nrhs][n_free], nrhs 1..4;
- * iters, relres: [n_sys][nrhs]; tune[0..1] in: threads per row (4/8/16) and rows
- * per tile, 0 = the library's choice; out: the choice, 0 where the systems were
+ * runs its own Jacobi-PCG from a zero start to ||r|| <= rtol ||b||: on resident
+ * teams of blocks, each solving one system after the other, or with an explicit
+ * layout, and where that is not possible, by captured-graph replays of one
+ * iteration sweep over all pairs.  b, x: host [nrhs][n_free], nrhs 1..4; iters,
+ * relres: [n_sys][nrhs]; tune[0..1] in: threads per row (4/8/16) and rows per
+ * tile, 0 = the library's choice; out: the choice, 0 where the systems were
  * solved on resident teams of blocks, which have neither. */
 PGF_API int pgf_batch_pcg(pgf_ctx* ctx, int32_t n_sys, const int64_t* sys_ptr, int32_t nrhs, const double* b,
                           double* x, double rtol, int32_t maxit, int32_t* iters, double* relres, double* ms,
@@ -224,8 +235,8 @@ PGF_API int pgf_batch_pcg(pgf_ctx* ctx, int32_t n_sys, const int64_t* sys_ptr, i
  * every pair runs inside a single kernel, grid-wide barriers between the
  * phases (p update, SpMM, alpha, vector update, beta and convergence), no
  * host round trip and no graph replay until all pairs have converged or hit
- * maxit.  Same arithmetic in the same order: results equal pgf_batch_pcg's
- * bit for bit.  Same arguments.  Holds at most 256 row tiles, one block per
+ * maxit.  Same arithmetic in the same order as the graph replays: results equal
+ * pgf_batch_pcg's with the same explicit layout bit for bit.  Same arguments.  Holds at most 256 row tiles, one block per
  * CU (PGF_EUNSUPPORTED beyond): the size it has been run and checked at. */
 PGF_API int pgf_batch_pcg_persistent(pgf_ctx* ctx, int32_t n_sys, const int64_t* sys_ptr, int32_t nrhs,
                                      const double* b, double* x, double rtol, int32_t maxit, int32_t* iters,

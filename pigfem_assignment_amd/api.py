@@ -325,6 +325,13 @@ class DeviceContext:
                                    rtol, maxit, precision, C.byref(info)))
         return x, info
 
+    def resident_solves(self, allow=-1):
+        """number of this context's solves that ran in one resident launch; allow:
+        0 separate launches from now on, 1 resident where possible (pgf_resident_solves)"""
+        n = C.c_int64()
+        self._chk(self.lib.pgf_resident_solves(self.h, int(allow), C.byref(n)))
+        return n.value
+
     def newton_step(self, frac, rel_tol=1e-8, abs_tol=0.0, max_iter=40, precision=64, lin_rtol=1e-10,
                     lin_maxit=50000, dt=1.0, use_guess=False, adaptive_lin=False, fp32_maxit=0):
         o = L.NewtonOpts(rel_tol, abs_tol, max_iter, precision, lin_rtol, lin_maxit, int(use_guess), dt,

@@ -731,9 +731,10 @@ int run_batch(pgfd::Ctx& c, const std::vector<int64_t>& sys_ptr, const double* b
               bool persistent) {
     const int n_sys = (int)sys_ptr.size() - 1;
     const int64_t nf = c.n_free;
-    if (!persistent && !(G_req > 0 && rows_req > 0)) {
+    if (!persistent && c.allow_resident && !(G_req > 0 && rows_req > 0)) {
         int rc = 0;
         if (run_teams<NR>(c, sys_ptr, b, x, rtol, maxit, iters, relres, ms_out, &rc)) {
+            ++c.n_resident;
             if (tuned) tuned[0] = tuned[1] = 0;
             return rc;
         }

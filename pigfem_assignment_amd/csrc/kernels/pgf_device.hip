@@ -644,6 +644,7 @@ static void make_team(Ctx& c) {
 
 template <typename TA>
 static bool pcg_team(Ctx& c, const TA* A, const double* b, bool x0, bool resume, double rtol, int maxit) {
+    if (!c.allow_resident) return false;
     if (!c.team_tried) make_team(c);
     if (!c.team.fits) return false;
     const pgft::TeamShape shape =
@@ -704,6 +705,7 @@ static void run_pcg(Ctx& c, const TA* A, const double* b, bool x0, double rtol, 
     HIPCHK(hipEventRecord(e0, c.stream));
     if (x0) enqueue_spmv<TA, double>(c, A, c.x, c.q);
     const bool on_team = pcg_team<TA>(c, A, b, x0, false, rtol, maxit);
+    c.n_resident += on_team;
     if (!on_team) pcg_launches<TA>(c, A, b, x0, false, rtol, maxit);
     auto rr = [&] { return c.h_scal[pgft::T_RR]; };
     const double rr0 = c.h_scal[pgft::T_RR0];
@@ -1417,6 +1419,13 @@ PGF_API int pgf_pcg(pgf_ctx* c, const double* b, double* x, const double* x0, do
         HIPCHK(c->copy.down(x, c->x, sizeof(double) * n, c->stream));
         return 0;
     });
+}
+
+PGF_API int pgf_resident_solves(pgf_ctx* c, int32_t allow, int64_t* n_resident) {
+    if (!c || allow < -1 || allow > 1) return PGF_EARG;
+    if (allow >= 0) c->allow_resident = allow != 0;
+    if (n_resident) *n_resident = c->n_resident;
+    return 0;
 }
 
 PGF_API int pgf_set_guess(pgf_ctx* c, const double* dx) {

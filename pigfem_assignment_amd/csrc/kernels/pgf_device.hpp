@@ -101,6 +101,8 @@ struct Ctx {
     std::vector<int64_t> unfit_sys;
     unsigned unfit_nrhs = 0;
     int n_cu = 0;
+    bool allow_resident = true;    // solves on teams where possible
+    int64_t n_resident = 0;        // solves that ran on teams
     double* partial = nullptr;     // block partial sums
     double* scal = nullptr;        // device scalars: PCG state (pgft::T_N), residual norm
     unsigned* counter = nullptr;   // last-block counters

@@ -15,8 +15,10 @@ from pigfem_assignment_amd.api import DeviceContext
 pytestmark = pytest.mark.gpu
 
 
-def test_fallback_follows_the_callers_tolerance():
+@pytest.mark.parametrize("resident", [1, 0])
+def test_fallback_follows_the_callers_tolerance(resident):
     ctx = DeviceContext(configs.c0_problem(n=60))
+    ctx.resident_solves(resident)
     ctx.apply_load_fraction(1.0)
     ctx.assemble(L.PGF_ASM_FUNC)
     b = -ctx.internal_force()[: ctx.csr.n_free]
@@ -42,4 +44,4 @@ def test_fallback_follows_the_callers_tolerance():
             print("tolerance %.3e met first at %d, 0.9 of it at %d; %d iterations (%s)" % (tol, first, last, k, kind), flush=True)
             assert not falls_back(tol, k)
             assert falls_back(tol, first - 1)
-    assert seen == {"at", "risen"}
+    assert seen == {"at", "risen"} and (ctx.resident_solves() > 0) == (resident == 1)
