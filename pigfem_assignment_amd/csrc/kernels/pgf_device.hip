@@ -675,7 +675,7 @@ static bool pcg_team(Ctx& c, const TA* A, const double* b, bool x0, bool resume,
                            c.team.slots, n_slots, pgft::EMPTY);
         const hipError_t e = hipLaunchCooperativeKernel(shape.kernel, dim3((unsigned)c.team.plan.blocks), dim3(pgft::TT), args,
                                                         shape.lds, c.stream);
-        if (first && !resume && (e == hipErrorIllegalState || e == hipErrorCooperativeLaunchTooLarge)) {
+        if (first && (e == hipErrorIllegalState || e == hipErrorCooperativeLaunchTooLarge)) {
             (void)hipGetLastError();
             return false;
         }
@@ -714,7 +714,7 @@ static void run_pcg(Ctx& c, const TA* A, const double* b, bool x0, double rtol, 
     if (spare && info->converged && !met(aim) && c.h_scal[pgft::T_IT] < maxit) {
         const double rr1 = rr();
         hipLaunchKernelGGL(k_copy, dim3(grid_for(c.n_free)), dim3(256), 0, c.stream, c.n_free, (const double*)c.x, spare);
-        if (on_team) (void)pcg_team<TA>(c, A, b, x0, true, aim, maxit);
+        if (on_team) (void)pcg_team<TA>(c, A, b, x0, true, aim, maxit);  // (refused: x is what it was)
         else pcg_launches<TA>(c, A, b, x0, true, aim, maxit);
         if (!met(rtol)) {
             hipLaunchKernelGGL(k_copy, dim3(grid_for(c.n_free)), dim3(256), 0, c.stream, c.n_free, (const double*)spare, c.x);
