@@ -225,9 +225,10 @@ PGF_API int pgf_set_guess(pgf_ctx* ctx, const double* dx);
  * teams of blocks, each solving one system after the other, or with an explicit
  * layout, and where that is not possible, by captured-graph replays of one
  * iteration sweep over all pairs.  b, x: host [nrhs][n_free], nrhs 1..4; iters,
- * relres: [n_sys][nrhs]; tune[0..1] in: threads per row (4/8/16) and rows per
- * tile, 0 = the library's choice; out: the choice, 0 where the systems were
- * solved on resident teams of blocks, which have neither. */
+ * relres: [n_sys][nrhs]; ms: the iterations, with the layout of the teams on the
+ * call that makes it; tune[0..1] in: threads per row (4/8/16) and rows per tile,
+ * 0 = the library's choice; out: the choice, 0 where the systems were solved on
+ * resident teams of blocks, which have neither. */
 PGF_API int pgf_batch_pcg(pgf_ctx* ctx, int32_t n_sys, const int64_t* sys_ptr, int32_t nrhs, const double* b,
                           double* x, double rtol, int32_t maxit, int32_t* iters, double* relres, double* ms,
                           int32_t* tune);

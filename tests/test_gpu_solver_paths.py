@@ -9,6 +9,7 @@ largest entry, the bar ten times that; for batches the explicit layout (8
 threads per row, 512 rows per tile), which iterates by the same launches.
 """
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -165,3 +166,22 @@ def test_two_contexts_solve_from_two_threads():
         t.join()
     assert not wrong
     assert all(ctx.resident_solves() == 11 for ctx, _, _ in work)
+
+
+def test_reported_time_of_a_batch_contains_its_layout():
+    """The first call with some systems takes longer by their layout, and says so."""
+    small, B = _batch([24, 32]), _batch(range(100, 160, 3))
+    ctx = DeviceContext(small)
+    ctx.assemble(L.PGF_ASM_JAC)
+    ctx.batch_pcg(small.sys_ptr, np.ones((3, small.n_free)), maxit=5)  # loads the kernels
+    ctx = DeviceContext(B)
+    ctx.assemble(L.PGF_ASM_JAC)
+    F = np.random.RandomState(0).standard_normal((3, B.n_free))
+    wall, told = [], []
+    for _ in range(2):
+        t = time.perf_counter()
+        told.append(ctx.batch_pcg(B.sys_ptr, F, rtol=1e-30, maxit=20)[3])
+        wall.append(1e3 * (time.perf_counter() - t))
+    print("wall %s ms, reported %s ms" % (wall, told), flush=True)
+    # (the rest: vectors that the context keeps)
+    assert wall[0] - wall[1] > 5 and told[0] - told[1] >= 0.3 * (wall[0] - wall[1]) and told[0] <= wall[0]
