@@ -98,7 +98,7 @@ EXPORTS = [
     "pgf_create", "pgf_destroy", "pgf_last_error", "pgf_device_info", "pgf_csr_info_get", "pgf_get_csr",
     "pgf_get_colors", "pgf_set_solution", "pgf_get_solution", "pgf_set_load", "pgf_apply_load_fraction",
     "pgf_assemble", "pgf_get_matrix", "pgf_get_matrix32", "pgf_get_internal_force", "pgf_n_cohesive_points",
-    "pgf_isv_commit", "pgf_isv_rollback", "pgf_get_isv", "pgf_set_isv", "pgf_spmv", "pgf_pcg", "pgf_set_guess",
+    "pgf_isv_commit", "pgf_isv_rollback", "pgf_get_isv", "pgf_set_isv", "pgf_spmv", "pgf_pcg", "pgf_set_guess", "pgf_resident_solves",
     "pgf_newton_step", "pgf_time_assemble", "pgf_time_assemble_split", "pgf_time_spmv",
     "pgf_set_gather_layout", "pgf_get_gather_layout",
     "pgfh_problem_create", "pgfh_problem_destroy", "pgfh_last_error", "pgfh_problem_info", "pgfh_mesh_desc",
