@@ -376,7 +376,9 @@ class DeviceContext:
     def batch_pcg(self, sys_ptr, B, rtol=1e-10, maxit=100000, tune=(0, 0), persistent=False):
         """Solve K_ff X = B per system (free-row ranges sys_ptr) for the rows of
         B [nrhs][n_free]; returns X, iterations [n_sys][nrhs], relres, ms, tune.
-        persistent: the whole solve in one cooperative launch
+        tune: (threads per row, rows per tile) of separate launches, (0, 0) for
+        the library's choice, which returns (0, 0) for resident teams.
+        persistent: the separate launches' iterations in one cooperative launch
         (pgf_batch_pcg_persistent) instead of graph replays."""
         sp = np.ascontiguousarray(sys_ptr, np.int64)
         B = np.ascontiguousarray(B, np.float64)

@@ -1,7 +1,8 @@
 // Batched solves of many independent systems sharing one device context.  With
 // the layout left to the library the systems are solved on resident teams
-// (pgf_team.hpp, run_teams below); an explicit layout, systems that fit no team
-// and a refused cooperative launch take the launches described next.  The
+// (pgf_team.hpp, run_teams below); an explicit layout, systems that fit no team,
+// short memory and a refused cooperative launch take the launches described next.
+// The
 // free-free block K_ff of a context whose mesh is a concatenation of
 // independent meshes (RVEs) is block diagonal, one block per RVE, and each
 // block is solved for NR right-hand sides (load cases / sensitivity

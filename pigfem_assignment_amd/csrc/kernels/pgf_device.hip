@@ -31,6 +31,7 @@ static std::string g_last_error;
 // for the current device, never the array's name.
 constexpr size_t NOALLOC_DOUBLES =
     8 + (PGF_NOALLOC_MAX_SEG + 1) + (size_t)PGF_NOALLOC_MAX_SEG * 13 + (size_t)PGF_NOALLOC_MAX_SEG * 64 * 13;
+static_assert(PGF_NOALLOC_MAX_SEG * 64 >= PGF_NOALLOC_MAX_SEG + 4096, "partials of volume_average_blocks");
 static __device__ __align__(256) double scratch[NOALLOC_DOUBLES];
 static std::mutex g_scratch_mutex;
 static double* g_scratch_ptr[64] = {nullptr};
