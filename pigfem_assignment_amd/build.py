@@ -28,8 +28,8 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
 CXXFLAGS = ["-O3", "-fPIC", "-std=c++17", "-fvisibility=hidden", "-I" + os.path.join(ROOT, "include")]
 # functions and loops of the host code on boundaries of their own: setting up
-# 1000 x 1000 quads with 400 inclusions took 860 or 1,020 ms (350 or 470 on the
-# machine with the GPU) by where the linker happened to put a loop
+# 1000 x 1000 quads with 400 inclusions took 860 or 1,020 ms (350 or 470 on a
+# faster CPU) by where the linker happened to put a loop
 HOSTFLAGS = CXXFLAGS + ["-falign-functions=64", "-falign-loops=32"]
 # packed FP32 instructions are disabled for every device code object
 HIPFLAGS = CXXFLAGS + ["--offload-arch=" + ARCH, "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
