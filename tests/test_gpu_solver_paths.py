@@ -183,5 +183,5 @@ def test_reported_time_of_a_batch_contains_its_layout():
         told.append(ctx.batch_pcg(B.sys_ptr, F, rtol=1e-30, maxit=20)[3])
         wall.append(1e3 * (time.perf_counter() - t))
     print("wall %s ms, reported %s ms" % (wall, told), flush=True)
-    # (the rest: vectors that the context keeps)
-    assert wall[0] - wall[1] > 5 and told[0] - told[1] >= 0.3 * (wall[0] - wall[1]) and told[0] <= wall[0]
+    # (the layout takes about 10 ms of the first call, 20 iterations 1.4 ms)
+    assert told[0] - told[1] > 2 and told[0] <= wall[0]
